@@ -118,6 +118,7 @@ int device_cu_count();
 // group, so the launch and the workspace query both use this count.
 int max_pool_groups();
 hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
+int mean_pool_row_len(int D);
 hipError_t launch_mean_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
 // Any block size / head dim (pooling_generic.hip); LDS need, checked by the caller against
 // kGenericPoolMaxLds.

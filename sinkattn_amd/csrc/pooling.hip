@@ -516,58 +516,177 @@ __global__ __launch_bounds__(256, 4) void max_pool_persistent_kernel(PoolArgs a,
 }
 
 // ------------------------------------------------------------------------------------
-// Mean-pooled scores.  Pass 1: per-block means of Q and K (replicate-padded tail).
+// Mean-pooled scores.  Pass 1: per-block means of Q and K (replicate-padded tail), fp32,
+// into workspace rows of mean_pool_row_len(D) floats (zero past D).  Bound by the read of Q
+// and K: a 256-thread group takes one block, RL threads per 16-byte chunk of the head dim
+// (16 at D = 128, 16-bit), each summing every RL-th row with eight loads in flight; the RL
+// partial sums meet in LDS.  Q and K go in one launch.  At [2,12,32760,128] bf16, blocks of
+// 128: 77 us for 403 MB, 5.2 TB/s, the rate of a large device copy (a thread per channel with
+// one 2-byte load in flight took 2 x 128 us).
 // ------------------------------------------------------------------------------------
 template <int IT>
-__global__ __launch_bounds__(128) void mean_pool_rows_kernel(PoolArgs a, int which) {
-  // blockIdx.x = block index, blockIdx.y = bh; thread = d.
-  const int blk = blockIdx.x, bh = blockIdx.y, d = threadIdx.x;
-  const int b = bh / a.H, h = bh - b * a.H;
-  const int N = which == 0 ? a.Nq : a.Nk;
-  const int nb = which == 0 ? a.nqb : a.nkb;
-  const int64_t* st = which == 0 ? a.qs : a.ks;
-  const void* base = which == 0 ? a.q : a.k;
-  const int D = blockDim.x;
-  const int bs = a.bs;
-  float acc = 0.f;
-  for (int i = 0; i < bs; ++i) {
-    const int n = min(blk * bs + i, N - 1);
-    const int64_t off = (int64_t)b * st[0] + (int64_t)h * st[1] + (int64_t)n * st[2] + d;
-    float x;
-    if (IT == kF32) x = reinterpret_cast<const float*>(base)[off];
-    else if (IT == kBF16) x = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(base)[off]);
-    else x = f16_bits_to_f32(reinterpret_cast<const uint16_t*>(base)[off]);
-    acc += x;
-  }
-  float* dst = a.ws + (which == 0 ? 0 : (int64_t)a.B * a.H * a.nqb * D);
-  dst[((int64_t)bh * nb + blk) * D + d] = acc / (float)bs;
+__device__ __forceinline__ float pool_elem(const char* p) {
+  if constexpr (IT == kF32) return *reinterpret_cast<const float*>(p);
+  else if constexpr (IT == kBF16) return bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(p));
+  else return f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(p));
 }
 
-// Pass 2: one wave per (bh, qb) row: dot products against every pooled key, softmax.
-__global__ __launch_bounds__(64) void mean_pool_scores_kernel(PoolArgs a, int D) {
-  const int qb = blockIdx.x, bh = blockIdx.y, lane = threadIdx.x;
-  const float* qp = a.ws + ((int64_t)bh * a.nqb + qb) * D;
-  const float* kp = a.ws + (int64_t)a.B * a.H * a.nqb * D + (int64_t)bh * a.nkb * D;
-  float* out = reinterpret_cast<float*>(a.out) + ((int64_t)bh * a.nqb + qb) * a.nkb;
-  float mx = neg_inf();
-  for (int kb = lane; kb < a.nkb; kb += 64) {
-    float acc = 0.f;
-    for (int d = 0; d < D; ++d) acc = __builtin_fmaf(qp[d], kp[(int64_t)kb * D + d], acc);
-    const float sc = acc * a.scale;
-    out[kb] = sc;
-    mx = fmaxf(mx, sc);
-  }
+template <int IT>
+__global__ __launch_bounds__(256) void mean_pool_rows_kernel(PoolArgs a, int D, int Dp) {
+  constexpr int ES = ElemSize<IT>::value;
+  constexpr int EPC = 16 / ES;
+  __shared__ float part[256 * EPC];
+  const int tid = threadIdx.x;
+  const bool is_q = (int)blockIdx.x < a.nqb;
+  const int blk = is_q ? blockIdx.x : blockIdx.x - a.nqb;
+  const int bh = blockIdx.y;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int N = is_q ? a.Nq : a.Nk;
+  const int64_t* st = is_q ? a.qs : a.ks;
+  const char* base = (const char*)(is_q ? a.q : a.k) + ((int64_t)b * st[0] + (int64_t)h * st[1]) * ES;
+  const int64_t rstride = st[2] * ES;
+  const int chunks = (D + EPC - 1) / EPC;  // <= 256 (D <= 1024)
+  const int RL = 256 / chunks;
+  const int c = tid % chunks, rl = tid / chunks;
+  float acc[EPC];
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  float sum = 0.f;
-  for (int kb = lane; kb < a.nkb; kb += 64) {
-    const float e = expf(out[kb] - mx);
-    out[kb] = e;
-    sum += e;
-  }
+  for (int e = 0; e < EPC; ++e) acc[e] = 0.f;
+  if (rl < RL) {
+    const char* src = base + c * 16;
+    const int row0 = blk * a.bs, last = N - 1;
+    if ((c + 1) * EPC <= D) {
+      for (int i0 = rl; i0 < a.bs; i0 += 8 * RL) {
+        u32x4 w[8];
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  for (int kb = lane; kb < a.nkb; kb += 64) out[kb] = out[kb] / sum;
+        for (int u = 0; u < 8; ++u) {
+          const int i = i0 + u * RL;
+          w[u] = u32x4{0, 0, 0, 0};
+          if (i < a.bs) w[u] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(row0 + i, last) * rstride);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if constexpr (IT == kF32) {
+              acc[j] += __uint_as_float(w[u][j]);
+            } else {
+              const uint32_t lo = w[u][j] & 0xffffu, hi = w[u][j] >> 16;
+              acc[2 * j] += IT == kBF16 ? bf16_bits_to_f32(lo) : f16_bits_to_f32(lo);
+              acc[2 * j + 1] += IT == kBF16 ? bf16_bits_to_f32(hi) : f16_bits_to_f32(hi);
+            }
+          }
+      }
+    } else {  // the head dim ends inside this chunk: element by element
+      for (int i = rl; i < a.bs; i += RL) {
+        const char* p = src + (int64_t)min(row0 + i, last) * rstride;
+#pragma unroll
+        for (int e = 0; e < EPC; ++e)
+          if (c * EPC + e < D) acc[e] += pool_elem<IT>(p + e * ES);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) part[(rl * chunks + c) * EPC + e] = acc[e];
+  }
+  __syncthreads();
+  float* dst = a.ws + ((is_q ? 0 : (int64_t)a.B * a.H * a.nqb) + (int64_t)bh * (is_q ? a.nqb : a.nkb) + blk) * Dp;
+  const int w = chunks * EPC;
+  for (int d = tid; d < Dp; d += 256) {
+    float s = 0.f;
+    if (d < D)
+      for (int r = 0; r < RL; ++r) s += part[r * w + d];
+    dst[d] = s / (float)a.bs;
+  }
+}
+
+// Pass 2: a group of 16 waves takes 16 query blocks of one head against every key block, on
+// the fp32 matrix cores (v_mfma_f32_16x16x4_f32; fp32 products and sums).  Lane l of a wave
+// holds query block l % 16 (A) and key block l % 16 (B) of its tile, and of every 16 channels
+// the four from 4 (l / 16), one 16-byte read, so that a read covers 64 consecutive bytes of 16
+// rows; D holds key block l % 16 and query blocks 4 (l / 16) .. +3, so a store writes 16
+// consecutive map entries.  Wave w takes key tiles w, w + 16, ...; then each wave softmaxes one
+// row, from registers up to 512 key blocks.  Bound by latency: 24 heads of
+// 256 x 256 blocks take 21 us (one wave per query row with a thread per key block, whose reads
+// of a pooled row never coalesce, took 785 us; four waves per group 25 us).
+constexpr int kMeanRows = 16;
+constexpr int kMeanWaves = 16;
+
+__global__ __launch_bounds__(64 * kMeanWaves) void mean_pool_scores_kernel(PoolArgs a, int Dp) {
+  const int bh = blockIdx.y, qb0 = blockIdx.x * kMeanRows;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, sl = lane & 15;
+  const float* qp = a.ws + ((int64_t)bh * a.nqb + min(qb0 + sl, a.nqb - 1)) * Dp + 4 * g;
+  const float* kp = a.ws + ((int64_t)a.B * a.H * a.nqb + (int64_t)bh * a.nkb) * Dp + 4 * g;
+  float* out = reinterpret_cast<float*>(a.out) + ((int64_t)bh * a.nqb + qb0) * a.nkb;
+  for (int k0 = wave * 16; k0 < a.nkb; k0 += 16 * kMeanWaves) {
+    const float* kr = kp + (int64_t)min(k0 + sl, a.nkb - 1) * Dp;
+    f32x4 s = f32x4{};
+    int d = 0;
+    for (; d + 128 <= Dp; d += 128) {  // 16 loads in flight
+      f32x4 qv[8], kv[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        qv[j] = *reinterpret_cast<const f32x4*>(qp + d + 16 * j);
+        kv[j] = *reinterpret_cast<const f32x4*>(kr + d + 16 * j);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[j][e], kv[j][e], s, 0, 0, 0);
+    }
+    for (; d < Dp; d += 16) {
+      const f32x4 qv = *reinterpret_cast<const f32x4*>(qp + d);
+      const f32x4 kv = *reinterpret_cast<const f32x4*>(kr + d);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[e], kv[e], s, 0, 0, 0);
+    }
+    const int kb = k0 + sl;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (qb0 + 4 * g + i < a.nqb && kb < a.nkb) out[(int64_t)(4 * g + i) * a.nkb + kb] = s[i] * a.scale;
+  }
+  __syncthreads();  // the group's scores are in memory
+  for (int r = wave; r < kMeanRows; r += kMeanWaves) {
+    if (qb0 + r >= a.nqb) break;
+    float* row = out + (int64_t)r * a.nkb;
+    constexpr int C = 8;
+    if (a.nkb <= 64 * C) {
+      float x[C];
+      float mx = neg_inf();
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        x[i] = lane + 64 * i < a.nkb ? row[lane + 64 * i] : neg_inf();
+        mx = fmaxf(mx, x[i]);
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (lane + 64 * i < a.nkb) {
+          x[i] = expf(x[i] - mx);
+          sum += x[i];
+        }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (lane + 64 * i < a.nkb) row[lane + 64 * i] = x[i] / sum;
+    } else {
+      float mx = neg_inf();
+      for (int kb = lane; kb < a.nkb; kb += 64) mx = fmaxf(mx, row[kb]);
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      float sum = 0.f;
+      for (int kb = lane; kb < a.nkb; kb += 64) {
+        const float e = expf(row[kb] - mx);
+        row[kb] = e;
+        sum += e;
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+      for (int kb = lane; kb < a.nkb; kb += 64) row[kb] = row[kb] / sum;
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------
@@ -635,17 +754,22 @@ hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stre
   return hipGetLastError();
 }
 
-hipError_t launch_mean_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream) {
-  if (a.B * a.H == 0) return hipSuccess;
-  for (int which = 0; which < 2; ++which) {
-    const dim3 grid(which == 0 ? a.nqb : a.nkb, a.B * a.H);
-    if (dtype == kF32) mean_pool_rows_kernel<kF32><<<grid, D, 0, stream>>>(a, which);
-    else if (dtype == kBF16) mean_pool_rows_kernel<kBF16><<<grid, D, 0, stream>>>(a, which);
-    else mean_pool_rows_kernel<kF16><<<grid, D, 0, stream>>>(a, which);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  mean_pool_scores_kernel<<<dim3(a.nqb, a.B * a.H), 64, 0, stream>>>(a, D);
+// Floats of a pooled row in the workspace: whole steps of 16 channels for the scores kernel.
+int mean_pool_row_len(int D) { return (D + 15) & ~15; }
+
+hipError_t launch_mean_pool(const PoolArgs& args, int dtype, int D, hipStream_t stream) {
+  if (args.B * args.H == 0) return hipSuccess;
+  PoolArgs a = args;  // the pooled rows start at the workspace's first 16-byte boundary
+  a.ws = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(args.ws) + 15) & ~(uintptr_t)15);
+  const int Dp = mean_pool_row_len(D);
+  const dim3 grid(a.nqb + a.nkb, a.B * a.H);
+  if (dtype == kF32) mean_pool_rows_kernel<kF32><<<grid, 256, 0, stream>>>(a, D, Dp);
+  else if (dtype == kBF16) mean_pool_rows_kernel<kBF16><<<grid, 256, 0, stream>>>(a, D, Dp);
+  else mean_pool_rows_kernel<kF16><<<grid, 256, 0, stream>>>(a, D, Dp);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  mean_pool_scores_kernel<<<dim3((a.nqb + kMeanRows - 1) / kMeanRows, a.B * a.H), 64 * kMeanWaves, 0,
+                            stream>>>(a, Dp);
   return hipGetLastError();
 }
 

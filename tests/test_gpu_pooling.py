@@ -288,3 +288,20 @@ def test_pooling_mode_dispatch():
         sa._compute_block_scores(qc, kc, kc, sa.SinkSparseConfig(pooling_mode="bogus"))
     t = sa._compute_block_scores(qc, kc, kc, sa.SinkSparseConfig(pooling_mode="triton"))
     assert t.dtype == torch.float32 and t.shape == (1, 2, 2, 2)
+
+
+@pytest.mark.parametrize("B,H,Nq,Nk,bs,D", [(1, 1, 1, 1, 128, 128), (1, 2, 17 * 16 + 1, 33, 16, 128),
+                                            (2, 1, 40, 600, 1, 64), (1, 1, 300, 1030, 2, 256),
+                                            (1, 2, 5000, 2600, 1024, 48), (1, 1, 65, 64, 4, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_mean_mode_tile_edges(B, H, Nq, Nk, bs, D, dtype):
+    """Remainders of the 16-row score tiles, rows past the 512 key blocks kept in registers, head
+    dims that end inside a 16-byte chunk or a quarter, strided operands.  Bound: fp32 sums of
+    at most 1024 rows and 256 products, each within 1024 * 2^-24 relative of its terms."""
+    g = torch.Generator().manual_seed(bs + D)
+    q = torch.randn(B, Nq, H, D, generator=g).to(dtype).permute(0, 2, 1, 3)
+    k = torch.randn(B, Nk, H, D, generator=g).to(dtype).permute(0, 2, 1, 3)
+    ours = ops.mean_pool_scores(q.cuda(), k.cuda(), block_size=bs).cpu()
+    ref = torch_ref.mean_pool_scores(q, k, block_size=bs)
+    assert ours.shape == ref.shape
+    assert torch.allclose(ours, ref, rtol=2e-5, atol=1e-7)
