@@ -495,8 +495,7 @@ size_t sinkattn_mean_pool_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int6
                                           int64_t block_size) {
   if (block_size <= 0) return 0;
   return (size_t)(B * H * (cdiv(Nq, block_size) + cdiv(Nk, block_size)) * sa::mean_pool_row_len((int)D)) *
-             sizeof(float) +
-         16;  // the kernels align the rows to 16 bytes themselves
+         sizeof(float);
 }
 
 int sinkattn_mean_pool_scores(const void* q, const void* k, int dtype, int64_t B, int64_t H,

@@ -608,6 +608,7 @@ __global__ __launch_bounds__(256) void mean_pool_rows_kernel(PoolArgs a, int D, 
 // 256 x 256 blocks take 21 us (one wave per query row with a thread per key block, whose reads
 // of a pooled row never coalesce, took 785 us; four waves per group 25 us).
 constexpr int kMeanRows = 16;
+typedef f32x4 f32x4_dword __attribute__((aligned(4)));  // the caller's workspace may start at any float
 constexpr int kMeanWaves = 16;
 
 __global__ __launch_bounds__(64 * kMeanWaves) void mean_pool_scores_kernel(PoolArgs a, int Dp) {
@@ -625,8 +626,8 @@ __global__ __launch_bounds__(64 * kMeanWaves) void mean_pool_scores_kernel(PoolA
       f32x4 qv[8], kv[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        qv[j] = *reinterpret_cast<const f32x4*>(qp + d + 16 * j);
-        kv[j] = *reinterpret_cast<const f32x4*>(kr + d + 16 * j);
+        qv[j] = *reinterpret_cast<const f32x4_dword*>(qp + d + 16 * j);
+        kv[j] = *reinterpret_cast<const f32x4_dword*>(kr + d + 16 * j);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -634,8 +635,8 @@ __global__ __launch_bounds__(64 * kMeanWaves) void mean_pool_scores_kernel(PoolA
         for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[j][e], kv[j][e], s, 0, 0, 0);
     }
     for (; d < Dp; d += 16) {
-      const f32x4 qv = *reinterpret_cast<const f32x4*>(qp + d);
-      const f32x4 kv = *reinterpret_cast<const f32x4*>(kr + d);
+      const f32x4 qv = *reinterpret_cast<const f32x4_dword*>(qp + d);
+      const f32x4 kv = *reinterpret_cast<const f32x4_dword*>(kr + d);
 #pragma unroll
       for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[e], kv[e], s, 0, 0, 0);
     }
@@ -757,10 +758,8 @@ hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stre
 // Floats of a pooled row in the workspace: whole steps of 16 channels for the scores kernel.
 int mean_pool_row_len(int D) { return (D + 15) & ~15; }
 
-hipError_t launch_mean_pool(const PoolArgs& args, int dtype, int D, hipStream_t stream) {
-  if (args.B * args.H == 0) return hipSuccess;
-  PoolArgs a = args;  // the pooled rows start at the workspace's first 16-byte boundary
-  a.ws = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(args.ws) + 15) & ~(uintptr_t)15);
+hipError_t launch_mean_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream) {
+  if (a.B * a.H == 0) return hipSuccess;
   const int Dp = mean_pool_row_len(D);
   const dim3 grid(a.nqb + a.nkb, a.B * a.H);
   if (dtype == kF32) mean_pool_rows_kernel<kF32><<<grid, 256, 0, stream>>>(a, D, Dp);
