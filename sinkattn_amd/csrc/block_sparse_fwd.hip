@@ -13,13 +13,13 @@
 //     O^T += V^T P^T       (A = V^T rows from LDS, B = P^T straight from the S^T VGPRs)
 // Computing the transposed products makes the S^T accumulator layout (one query column
 // per lane, keys down the registers) line up with the B-operand layout of the second
-// MFMA, so P never leaves registers.  block_sparse_fwd_kernel (D = 32 and 64, all input
-// types; v_mfma_f32_32x32x16, K rows permuted so that the key order in the P^T registers is
-// natural) stages K and V^T through registers, V transposed while staging;
-// block_sparse_fwd_d128_kernel (D = 128, 16-bit; v_mfma_f32_16x16x32) copies K and V
-// row-major by buffer DMA and reads V^T with transpose loads; block_sparse_fwd_f32_kernel
-// splits fp32 operands into bf16 pairs.  The plan kernels at the end of the file turn the
-// bool mask into per-row lists and the launch order.
+// MFMA, so P never leaves registers.  block_sparse_fwd_d128_kernel and
+// block_sparse_fwd_small_kernel (16-bit, D = 128; 64 and 32; v_mfma_f32_16x16x32) copy K and V
+// row-major by buffer DMA and read V^T with transpose loads; block_sparse_fwd_kernel (16-bit
+// D = 32 and 64 whose K or V rows overlap; v_mfma_f32_32x32x16, K rows permuted so that the
+// key order in the P^T registers is natural) stages K and V^T through registers, V transposed
+// while staging; block_sparse_fwd_f32_kernel splits fp32 operands into bf16 pairs.  The plan
+// kernels at the end of the file turn the bool mask into per-row lists and the launch order.
 
 #include "common.h"
 #include "kernels.h"
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
 }
 
 // ------------------------------------------------------------------------------------
-// D = 128, bf16/f16: K and V tiles go global -> LDS by buffer DMA (no staging
+// bf16/f16 (figures for D = 128): K and V tiles go global -> LDS by buffer DMA (no staging
 // registers; rows >= Nk read as zero through the buffer bounds), and V^T is read from
 // the row-major V tile with the gfx950 transpose read ds_read_b64_tr_b16.  Both products
 // run on v_mfma_f32_16x16x32, which with random 16-bit operands draws less power per flop
@@ -175,85 +175,113 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
 // Lane l holds query 16 qt + l % 16 in both products; its S^T registers (kt, qt) hold keys
 // 16 kt + 4 (l / 16) + i, i < 4.  A PV k-step kc of 32 keys takes its eight B values from
 // S^T tiles (2 kc, qt) and (2 kc + 1, qt), and the transpose reads pick the same keys for
-// the A operand, so P never leaves the registers.  The row sums come from the matrix cores as
-// well: one more MFMA per k-step and q tile with an all-ones A operand sums the 16-bit P values
+// the A operand, so P never leaves the registers.  At D = 128 the row sums come from the matrix
+// cores as well: one more MFMA per k-step and q tile with an all-ones A operand sums the 16-bit P values
 // the PV product uses (O / l is then a weighted mean with weights that sum to one; l is within
 // 2^-8 relative of the fp32 sum for bf16, 2^-11 for f16), which keeps 64 adds per tile off
 // the VALU.  K and V are staged against each other:
 // V(i)'s copies are spread over S(i) and K(i+1)'s over softmax(i), one per step, so that
 // the copies of the four waves never queue up at the CU's vector-memory pipe in one burst;
 // three work-group barriers per tile (K free, V landed, V free and K(i+1) landed).  LDS
-// layout: 128 rows x 16 chunks of 16 bytes per tile, physical chunk = logical ^ (row & 15)
-// for K (a 16-lane K read touches 16 distinct chunks) and logical ^ 2 (row & 7) for V (a
-// half-wave transpose read touches 8 distinct 32-byte column pairs).
+// layout: 128 rows x D / 8 chunks of 16 bytes per tile, the chunks of a row swizzled as in
+// TileGeom (at D = 128 logical ^ (row & 15) for K, logical ^ 2 (row & 7) for V).
 // ------------------------------------------------------------------------------------
 constexpr float kLazyRescaleLog2 = 8.0f;
 
-// Per-lane LDS addresses of the d128 tile loop (bytes).
-struct D128Lanes {
-  uint32_t k_off, v_off;  // global byte offset of this lane's first 16-byte DMA chunk
-  uint32_t ka[4];         // K A operand of k-step ks: row l % 16 (+ 16 kt), chunk 4 ks + l / 16
-  uint32_t va[8];         // V^T transpose reads of d-tile dt (+ 32 kc rows, + 16 h rows)
+// Geometry of a staged 128-row tile of D 16-bit columns (D = 32, 64 or 128).
+template <int D>
+struct TileGeom {
+  static constexpr int kRow = 2 * D;            // bytes of a row
+  static constexpr int kChunks = D / 8;         // 16-byte chunks of a row
+  static constexpr int kRows256 = 128 / D;      // rows per 256 bytes of LDS (one pass over the banks)
+  static constexpr int kCopyRows = 64 / kChunks;  // rows one wave's copy instruction fills
+  static constexpr int kCopies = D / 16;        // copies of a wave per tile
+  // Chunk swizzles: a 16-lane K read (one chunk of 16 rows) and a half-wave transpose read of V
+  // (32 bytes of 8 rows) both spread over 256 distinct bytes of LDS.
+  static __device__ __forceinline__ int kswz(int row) { return (row / kRows256) & (kChunks - 1); }
+  static __device__ __forceinline__ int vswz(int row) { return 2 * ((row / kRows256) & (kChunks / 2 - 1)); }
 };
 
-__device__ __forceinline__ D128Lanes d128_lanes(int wave, int lane, uint32_t kstride, uint32_t vstride) {
-  D128Lanes L;
+// Per-lane LDS addresses of the tile loop (bytes).
+template <int D>
+struct TileLanes {
+  uint32_t k_off, v_off;  // global byte offset of this lane's first 16-byte DMA chunk
+  uint32_t ka[D / 32];    // K A operand of k-step ks: row l % 16 (+ 16 kt), chunk 4 ks + l / 16
+  uint32_t va[D / 16];    // V^T transpose reads of d-tile dt (+ 32 kc rows, + 16 h rows)
+};
+
+template <int D>
+__device__ __forceinline__ TileLanes<D> tile_lanes(int wave, int lane, uint32_t kstride, uint32_t vstride) {
+  using G = TileGeom<D>;
+  TileLanes<D> L;
   const int g = lane >> 4, sl = lane & 15;
-  // DMA: instruction j of wave w fills tile rows 16j + 4w + lane/16 (LDS bytes
-  // [(256j + 64w) * 16, +1024)); the swizzle of those rows does not depend on j.
-  const int drow = 4 * wave + g;
-  L.k_off = (uint32_t)drow * kstride + (uint32_t)((sl ^ (drow & 15)) * 16);
-  L.v_off = (uint32_t)drow * vstride + (uint32_t)((sl ^ (2 * (drow & 7))) * 16);
+  // DMA: instruction j of wave w fills tile rows (4j + w) kCopyRows + lane / kChunks (LDS
+  // bytes [(256j + 64w) * 16, +1024)); the swizzles of those rows do not depend on j.
+  const int drow = G::kCopyRows * wave + lane / G::kChunks, dch = lane % G::kChunks;
+  L.k_off = (uint32_t)drow * kstride + (uint32_t)((dch ^ G::kswz(drow)) * 16);
+  L.v_off = (uint32_t)drow * vstride + (uint32_t)((dch ^ G::vswz(drow)) * 16);
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) L.ka[ks] = (uint32_t)(sl * 256 + (((4 * ks + g) ^ sl) * 16));
+  for (int ks = 0; ks < D / 32; ++ks) L.ka[ks] = (uint32_t)(sl * G::kRow + (((4 * ks + g) ^ G::kswz(sl)) * 16));
   // Transpose read h of d-tile dt at k-step kc: lane s of 16-lane group g points at key row
   // 32 kc + 16 h + 4 g + s / 4, columns 16 dt + 4 (s % 4) .. +3.  Lane l of the group then
   // receives element l % 4 of the rows of lanes 4 j + (l % 16) / 4, j < 4: d = 16 dt + l % 16
   // at keys 32 kc + 16 h + 4 g + j, the keys of B slots 4 h + j.
-  const int row = 4 * g + (sl >> 2);  // + 32 kc + 16 h, which leave row & 7 unchanged
+  const int row = 4 * g + (sl >> 2);  // + 32 kc + 16 h, which leave the swizzle unchanged
   const int a4 = sl & 3;
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt) {
+  for (int dt = 0; dt < D / 16; ++dt) {
     const int chunk = 2 * dt + (a4 >> 1);
-    L.va[dt] = (uint32_t)(row * 256 + ((chunk ^ (2 * (row & 7))) * 16) + (a4 & 1) * 8);
+    L.va[dt] = (uint32_t)(row * G::kRow + ((chunk ^ G::vswz(row)) * 16) + (a4 & 1) * 8);
   }
   return L;
 }
 
-// Copy j (of 8) of this wave's share of a 128-row tile: rows 16j + 4w + lane/16, from the
-// buffer `rs` (rows past its size read as zero) into the LDS tile at `dst`.
-__device__ __forceinline__ void d128_copy_one(SA_LDS char* dst, const __amdgpu_buffer_rsrc_t& rs, uint32_t stride,
+// Copy j of this wave's share of a 128-row tile, from the buffer `rs` (rows past its size read
+// as zero) into the LDS tile at `dst`.
+template <int D>
+__device__ __forceinline__ void tile_copy_one(SA_LDS char* dst, const __amdgpu_buffer_rsrc_t& rs, uint32_t stride,
                                               uint32_t lane_off, int wave, int j) {
-  dma16(rs, (SA_LDS void*)(dst + (256 * j + 64 * wave) * 16), lane_off + (uint32_t)j * 16u * stride);
+  dma16(rs, (SA_LDS void*)(dst + (256 * j + 64 * wave) * 16),
+        lane_off + (uint32_t)j * (uint32_t)(4 * TileGeom<D>::kCopyRows) * stride);
 }
 
 // 128 rows of K (or V) from `base` (row stride `stride` bytes, `rows_valid` rows readable:
 // rows past it read as zero through the buffer bounds) into the LDS tile at `dst`.
-__device__ __forceinline__ void d128_copy_tile(SA_LDS char* dst, const char* base, uint32_t stride,
-                                               int rows_valid, uint32_t lane_off, int wave) {
+template <int D>
+__device__ __forceinline__ void tile_copy(SA_LDS char* dst, const char* base, uint32_t stride, int rows_valid,
+                                          uint32_t lane_off, int wave) {
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (uint32_t)rows_valid * stride);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) d128_copy_one(dst, rs, stride, lane_off, wave, j);
+  for (int j = 0; j < TileGeom<D>::kCopies; ++j) tile_copy_one<D>(dst, rs, stride, lane_off, wave, j);
 }
 
-// One 128-key tile of the d128 loop for this wave's 32 query rows:
+// One 128-key tile of the loop for this wave's 32 query rows:
 //   S^T = K Q^T from the K tile, with vcopy(j) (this tile's V copy j into the V buffer, free
 //   since the previous tile's B2) after every fourth (k-step, key tile) pair; barrier B1
 //   (every wave is done with K); the online softmax with kcopy(j) (the next tile's K copy j
-//   into the K buffer) after step j; barrier BV (every wave's V copies have landed: vmcnt(8)
-//   leaves only the eight K copies issued after them in flight); O^T += V^T P^T from the V
+//   into the K buffer) after step j; barrier BV (every wave's V copies have landed: the wait
+//   leaves only the K copies issued after them in flight); O^T += V^T P^T from the V
 //   tile; barrier B2 (the next K has landed, every wave is done with V).  kcopy must issue a
 //   copy for every j, also after the last tile (then from a 0-byte buffer), so that the
 //   count of BV holds.
+// Row sums: kMfmaSums (D = 128) takes them from the matrix cores over the 16-bit P, l_acc
+// holding each query's whole sum in every lane; otherwise they are fp32 adds of the
+// unrounded exponentials, l_acc[qt][0] holding this lane's share.
 // Keys at or past klim are masked; bias is added to the log2-domain logits (compensation
 // tiles); c = softmax scale * log2(e).  g = lane / 16.
-template <int CT, typename FV, typename FK>
-__device__ __forceinline__ void d128_tile(SA_LDS char* lk, SA_LDS char* lv, const D128Lanes& L,
-                                          const u32x4 (&qf)[2][4], int key0, int klim, float bias,
-                                          float c, int g, f32x4 (&o)[8][2], float (&m_run)[2],
+template <int D>
+constexpr bool kMfmaSums = D == 128;
+
+template <int CT, int D, typename FV, typename FK>
+__device__ __forceinline__ void attn_tile(SA_LDS char* lk, SA_LDS char* lv, const TileLanes<D>& L,
+                                          const u32x4 (&qf)[2][D / 32], int key0, int klim, float bias,
+                                          float c, int g, f32x4 (&o)[D / 16][2], float (&m_run)[2],
                                           f32x4 (&l_acc)[2], FV&& vcopy, FK&& kcopy) {
-  constexpr int KR = 4;  // K reads issued ahead of their MFMAs
-  constexpr int VR = 3;  // transpose-read pairs issued ahead of their MFMAs
+  constexpr int DT = D / 16;    // d tiles of O^T
+  constexpr int NP = 8 * D / 32;  // (k-step, key tile) pairs of S^T
+  constexpr int KR = 4;         // K reads issued ahead of their MFMAs
+  constexpr int VR = 3;         // transpose-read pairs issued ahead of their MFMAs
+  constexpr int NC = TileGeom<D>::kCopies;
   f32x4 s[8][2];
 #pragma unroll
   for (int kt = 0; kt < 8; ++kt) {
@@ -262,17 +290,17 @@ __device__ __forceinline__ void d128_tile(SA_LDS char* lk, SA_LDS char* lv, cons
   }
   {
     // pair p = 8 ks + kt: one K read (rows 16 kt .., d slice ks), the MFMAs of both q tiles
-    u32x4 kr[32];
-    auto kread = [&](int p) { return *(SA_LDS const u32x4*)(lk + L.ka[p >> 3] + (p & 7) * 4096); };
+    u32x4 kr[NP];
+    auto kread = [&](int p) { return *(SA_LDS const u32x4*)(lk + L.ka[p >> 3] + (p & 7) * (32 * D)); };
 #pragma unroll
     for (int p = 0; p < KR; ++p) kr[p] = kread(p);
     __builtin_amdgcn_sched_group_barrier(0x100, KR, 0);
 #pragma unroll
-    for (int p = 0; p < 32; ++p) {
+    for (int p = 0; p < NP; ++p) {
       const int ks = p >> 3, kt = p & 7;
       s[kt][0] = mfma16x16x32<CT>(kr[p], qf[0][ks], s[kt][0]);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (p + KR < 32) {
+      if (p + KR < NP) {
         kr[p + KR] = kread(p + KR);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
@@ -311,7 +339,7 @@ __device__ __forceinline__ void d128_tile(SA_LDS char* lk, SA_LDS char* lv, cons
       const float alpha = fast_exp2(m_run[qt] - m_tile);
       l_acc[qt] *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) o[dt][qt] *= alpha;
+      for (int dt = 0; dt < DT; ++dt) o[dt][qt] *= alpha;
       m_run[qt] = m_tile;
     }
   }
@@ -324,13 +352,14 @@ __device__ __forceinline__ void d128_tile(SA_LDS char* lk, SA_LDS char* lv, cons
       for (int e = 0; e < 2; ++e) {
         const float v0 = fast_exp2(__builtin_fmaf(s[2 * kc + h][qt][2 * e], c, nb));
         const float v1 = fast_exp2(__builtin_fmaf(s[2 * kc + h][qt][2 * e + 1], c, nb));
+        if constexpr (!kMfmaSums<D>) l_acc[qt][0] += v0 + v1;
         p[kc][qt][2 * h + e] = pack2<CT>(v0, v1);
       }
   };
-  auto vread = [&](int r) -> u32x4 {  // r = 8 kc + dt
-    SA_LDS char* base = lv + L.va[r & 7] + (r >> 3) * 8192;
+  auto vread = [&](int r) -> u32x4 {  // r = DT kc + dt
+    SA_LDS char* base = lv + L.va[r % DT] + (r / DT) * (64 * D);
     const v4i16 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)base);
-    const v4i16 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)(base + 4096));
+    const v4i16 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)(base + 32 * D));
     const u32x2 y0 = __builtin_bit_cast(u32x2, x0), y1 = __builtin_bit_cast(u32x2, x1);
     return u32x4{y0[0], y0[1], y1[0], y1[1]};
   };
@@ -338,40 +367,42 @@ __device__ __forceinline__ void d128_tile(SA_LDS char* lk, SA_LDS char* lv, cons
 #pragma unroll
   for (int step = 0; step < 8; ++step) {
     make_p(step >> 1, step & 1);
-    kcopy(step);
+    if (step < NC) kcopy(step);
     __builtin_amdgcn_sched_barrier(0);
   }
   // BV: this tile's V has landed for every wave (the own V copies are done once at most the
-  // eight K copies issued after them are in flight)
-  __builtin_amdgcn_s_waitcnt(8 | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(8)
+  // K copies issued after them are in flight)
+  __builtin_amdgcn_s_waitcnt(NC | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(NC)
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_s_setprio(1);
   {
-    // pair r = 8 kc + dt: two transpose reads (d tile dt, keys of k-step kc), both q tiles
-    u32x4 vr[32];
+    // pair r = DT kc + dt: two transpose reads (d tile dt, keys of k-step kc), both q tiles
+    u32x4 vr[4 * DT];
 #pragma unroll
     for (int r = 0; r < VR; ++r) vr[r] = vread(r);
     __builtin_amdgcn_sched_group_barrier(0x100, 2 * VR, 0);
 #pragma unroll
-    for (int r = 0; r < 32; ++r) {
-      const int kc = r >> 3, dt = r & 7;
+    for (int r = 0; r < 4 * DT; ++r) {
+      const int kc = r / DT, dt = r % DT;
       o[dt][0] = mfma16x16x32<CT>(vr[r], p[kc][0], o[dt][0]);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (r + VR < 32) {
+      if (r + VR < 4 * DT) {
         vr[r + VR] = vread(r + VR);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
       }
       o[dt][1] = mfma16x16x32<CT>(vr[r], p[kc][1], o[dt][1]);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (dt == 7) {
-        // row sums of the 16-bit P of this k-step: A = all ones, so every row of the product
-        // is the column sum, and every lane holds its query's running sum
-        const uint32_t one = CT == kBF16 ? 0x3F803F80u : 0x3C003C00u;
-        const u32x4 ones = {one, one, one, one};
-        l_acc[0] = mfma16x16x32<CT>(ones, p[kc][0], l_acc[0]);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        l_acc[1] = mfma16x16x32<CT>(ones, p[kc][1], l_acc[1]);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if constexpr (kMfmaSums<D>) {
+        if (dt == DT - 1) {
+          // row sums of the 16-bit P of this k-step: A = all ones, so every row of the product
+          // is the column sum, and every lane holds its query's running sum
+          const uint32_t one = CT == kBF16 ? 0x3F803F80u : 0x3C003C00u;
+          const u32x4 ones = {one, one, one, one};
+          l_acc[0] = mfma16x16x32<CT>(ones, p[kc][0], l_acc[0]);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          l_acc[1] = mfma16x16x32<CT>(ones, p[kc][1], l_acc[1]);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
       }
     }
   }
@@ -379,16 +410,16 @@ __device__ __forceinline__ void d128_tile(SA_LDS char* lk, SA_LDS char* lv, cons
   drain_then_barrier();  // B2: next K landed, every wave done with V
 }
 
-// Everything the d128 kernels need to know about one (b, h, q-block) work item.  All values
+// Everything these kernels need to know about one (b, h, q-block) work item.  All values
 // are wave-uniform (scalar registers).
-struct D128Item {
+struct AttnItem {
   int item, qb, cnt, ntot;
   const char *qbase, *kbase, *vbase, *kdbase, *vdbase;
   const SA_CONST int32_t* list;
 };
 
-__device__ __forceinline__ D128Item d128_item(const FwdArgs& a, int item) {
-  D128Item it;
+__device__ __forceinline__ AttnItem attn_item(const FwdArgs& a, int item) {
+  AttnItem it;
   it.item = item;
   const int bh = item / a.nqb;
   it.qb = item - bh * a.nqb;
@@ -412,46 +443,38 @@ __device__ __forceinline__ D128Item d128_item(const FwdArgs& a, int item) {
 // Tile `t` of an item's walk (listed tiles, then compensation tiles): its first key.  The
 // list entry is read unconditionally at an index clamped into the row's own list, so that the
 // load can be issued a whole tile before it is needed without ever leaving the plan.
-__device__ __forceinline__ int d128_key0(const D128Item& it, int t) {
+__device__ __forceinline__ int attn_key0(const AttnItem& it, int t) {
   const int e = it.list[t < it.cnt ? t : (it.cnt > 0 ? it.cnt - 1 : 0)];
   return t < it.cnt ? e * 128 : (t - it.cnt) * 128;
 }
 
-// K rows [key0, key0 + 128) of the listed keys (comp = false) or of the pooled keys
-// (comp = true); rows at or past klim read as zero.
-template <int CT>
-__device__ __forceinline__ void d128_issue_k(const D128Item& it, int key0, int klim, bool comp, SA_LDS char* lk,
-                                             const D128Lanes& L, uint32_t kstride, int wave) {
-  const char* base = (comp ? it.kdbase : it.kbase) + (int64_t)key0 * kstride;
-  d128_copy_tile(lk, base, kstride, klim - key0, L.k_off, wave);
-}
-
-// O of this wave's 32 rows through its 8 KB of an idle LDS tile buffer: lane l holds d values
-// 16 dt + 4 (l / 16) .. +3 of row 16 qt + l % 16, written as 8-byte pieces; after the
-// transpose every store instruction writes 4 whole 256-byte rows.  The caller guarantees that
+// O of this wave's 32 rows through its share (64 D bytes) of an idle LDS tile buffer: lane l
+// holds d values 16 dt + 4 (l / 16) .. +3 of row 16 qt + l % 16, written as 8-byte pieces; after
+// the transpose every store instruction writes whole rows.  The caller guarantees that
 // no wave reads the buffer and no copy into it is in flight; each wave touches only its own
 // slice.
-template <int CT>
-__device__ __forceinline__ void d128_store_o_staged(const FwdArgs& a, const D128Item& it, const f32x4 (&o)[8][2],
-                                                    const float (&m_run)[2], const f32x4 (&l_acc)[2],
-                                                    SA_LDS char* buf, int wave, int lane) {
+template <int CT, int D>
+__device__ __forceinline__ void store_o_staged(const FwdArgs& a, const AttnItem& it, const f32x4 (&o)[D / 16][2],
+                                               const float (&m_run)[2], const f32x4 (&l_acc)[2],
+                                               SA_LDS char* buf, int wave, int lane) {
+  using G = TileGeom<D>;
   const int g = lane >> 4, sl = lane & 15;
   float l[2], inv[2];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
-    l[qt] = l_acc[qt][0];
+    l[qt] = kMfmaSums<D> ? l_acc[qt][0] : sum_col16(l_acc[qt][0]);
     inv[qt] = l[qt] > 0.f ? 1.f / l[qt] : 0.f;
   }
-  SA_LDS char* ob = buf + wave * 8192;
+  SA_LDS char* ob = buf + wave * (64 * D);
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const int chunk = (2 * dt + (g >> 1)) ^ sl;  // row 16 qt + sl: row & 15 == sl
+    for (int dt = 0; dt < D / 16; ++dt) {
+      const int chunk = (2 * dt + (g >> 1)) ^ G::kswz(sl);  // row 16 qt + sl swizzles like row sl
       u32x2 w;
       w[0] = pack2<CT>(o[dt][qt][0] * inv[qt], o[dt][qt][1] * inv[qt]);
       w[1] = pack2<CT>(o[dt][qt][2] * inv[qt], o[dt][qt][3] * inv[qt]);
-      *(SA_LDS u32x2*)(ob + (16 * qt + sl) * 256 + chunk * 16 + (g & 1) * 8) = w;
+      *(SA_LDS u32x2*)(ob + (16 * qt + sl) * G::kRow + chunk * 16 + (g & 1) * 8) = w;
     }
   __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0) only
   const int bh = it.item / a.nqb;
@@ -459,9 +482,9 @@ __device__ __forceinline__ void d128_store_o_staged(const FwdArgs& a, const D128
   const int q0 = it.qb * 128 + wave * 32;
   char* obase = (char*)a.out + ((int64_t)b * a.os[0] + (int64_t)h * a.os[1]) * 2;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int rr = 4 * i + (lane >> 4), cc = lane & 15;
-    const u32x4 val = *(SA_LDS const u32x4*)(ob + rr * 256 + ((cc ^ (rr & 15)) * 16));
+  for (int i = 0; i < 32 / G::kCopyRows; ++i) {
+    const int rr = G::kCopyRows * i + lane / G::kChunks, cc = lane % G::kChunks;
+    const u32x4 val = *(SA_LDS const u32x4*)(ob + rr * G::kRow + ((cc ^ G::kswz(rr)) * 16));
     if (q0 + rr < a.Nq)
       *reinterpret_cast<u32x4*>(obase + ((int64_t)(q0 + rr) * a.os[2]) * 2 + cc * 16) = val;
   }
@@ -476,37 +499,32 @@ __device__ __forceinline__ void d128_store_o_staged(const FwdArgs& a, const D128
 }
 
 // ------------------------------------------------------------------------------------
-// The per-q-block form: one work-group per order slot (or per row without an order).
+// One work-group per order slot (or per row without an order).
 // ------------------------------------------------------------------------------------
-template <int CT>
-__global__ __launch_bounds__(256, 2) void block_sparse_fwd_d128_kernel(FwdArgs a) {
-  __shared__ u32x4 lds_k[2048];
-  __shared__ u32x4 lds_v[2048];
-
+template <int CT, int D>
+__device__ __forceinline__ void fwd_qblock(const FwdArgs& a, SA_LDS char* lk, SA_LDS char* lv) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, sl = lane & 15;
   const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[blockIdx.x] : (int)blockIdx.x);
   if (item < 0) return;
-  const D128Item it = d128_item(a, item);
+  const AttnItem it = attn_item(a, item);
   const uint32_t kstride = (uint32_t)a.ks[2] * 2, vstride = (uint32_t)a.vs[2] * 2;
-  const D128Lanes L = d128_lanes(wave, lane, kstride, vstride);
-  SA_LDS char* lk = (SA_LDS char*)lds_k;
-  SA_LDS char* lv = (SA_LDS char*)lds_v;
+  const TileLanes<D> L = tile_lanes<D>(wave, lane, kstride, vstride);
 
   // Q^T B operands: query 16 qt + l % 16 of the wave's rows, d slice 32 ks + 8 (l / 16)
-  u32x4 qf[2][4];
+  u32x4 qf[2][D / 32];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     const int qrow = it.qb * 128 + wave * 32 + 16 * qt + sl;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < D / 32; ++ks)
       qf[qt][ks] = qrow < a.Nq ? *(const u32x4*)(it.qbase + ((int64_t)qrow * a.qs[2] + 32 * ks + 8 * g) * 2)
                                : u32x4{0, 0, 0, 0};
   }
-  f32x4 o[8][2];
+  f32x4 o[D / 16][2];
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt) {
+  for (int dt = 0; dt < D / 16; ++dt) {
     o[dt][0] = f32x4{};
     o[dt][1] = f32x4{};
   }
@@ -517,17 +535,18 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_d128_kernel(FwdArgs a
   // kernel arguments the tile loop needs, read once
   const int Nk = a.Nk, Nd = a.Nd;
   const float comp_bias = a.comp_bias;
-  int key0 = d128_key0(it, 0);
+  int key0 = attn_key0(it, 0);
   int klim = it.cnt > 0 ? Nk : Nd;
   if (it.ntot > 0) {
-    d128_issue_k<CT>(it, key0, klim, it.cnt == 0, lk, L, kstride, wave);
+    tile_copy<D>(lk, (it.cnt == 0 ? it.kdbase : it.kbase) + (int64_t)key0 * kstride, kstride, klim - key0, L.k_off,
+                 wave);
     drain_then_barrier();
   }
   for (int t = 0; t < it.ntot; ++t) {
     const bool next = t + 1 < it.ntot;
     const bool comp = t >= it.cnt;
     const bool comp_next = t + 1 >= it.cnt;
-    const int key0_next = d128_key0(it, t + 1);
+    const int key0_next = attn_key0(it, t + 1);
     const int klim_next = comp_next ? Nd : Nk;
     const __amdgpu_buffer_rsrc_t vrs =
         make_rsrc((comp ? it.vdbase : it.vbase) + (int64_t)key0 * vstride, (uint32_t)(klim - key0) * vstride);
@@ -535,16 +554,34 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_d128_kernel(FwdArgs a
     // access), so that every tile issues the same copies and waits
     const __amdgpu_buffer_rsrc_t krs = make_rsrc((comp_next ? it.kdbase : it.kbase) + (int64_t)key0_next * kstride,
                                                  next ? (uint32_t)(klim_next - key0_next) * kstride : 0u);
-    d128_tile<CT>(lk, lv, L, qf, key0, klim, t < it.cnt ? 0.f : comp_bias, c, g, o, m_run, l_acc,
-                  [&](int j) { d128_copy_one(lv, vrs, vstride, L.v_off, wave, j); },
-                  [&](int j) { d128_copy_one(lk, krs, kstride, L.k_off, wave, j); });
+    attn_tile<CT, D>(lk, lv, L, qf, key0, klim, t < it.cnt ? 0.f : comp_bias, c, g, o, m_run, l_acc,
+                     [&](int j) { tile_copy_one<D>(lv, vrs, vstride, L.v_off, wave, j); },
+                     [&](int j) { tile_copy_one<D>(lk, krs, kstride, L.k_off, wave, j); });
     key0 = key0_next;
     klim = klim_next;
   }
 
-  // O through this wave's 8 KB of the K buffer: every wave has passed the last barrier, so
+  // O through this wave's share of the K buffer: every wave has passed the last barrier, so
   // no wave still reads K and no copy into it is in flight.
-  d128_store_o_staged<CT>(a, it, o, m_run, l_acc, lk, wave, lane);
+  store_o_staged<CT, D>(a, it, o, m_run, l_acc, lk, wave, lane);
+}
+
+template <int CT>
+__global__ __launch_bounds__(256, 2) void block_sparse_fwd_d128_kernel(FwdArgs a) {
+  __shared__ u32x4 lds_k[2048];
+  __shared__ u32x4 lds_v[2048];
+  fwd_qblock<CT, 128>(a, (SA_LDS char*)lds_k, (SA_LDS char*)lds_v);
+}
+
+// Head dims 64 and 32: the same tile loop on 16 KB and 8 KB tiles.  Bound by the exponentials
+// (as many per key as at head dim 128, for half or a quarter of the matrix work).  f16
+// [2,16,8100,64], a quarter of the blocks kept: 176 us, 0.84 PFLOP/s (295 us with K and V^T
+// staged through registers on 32x32x16; three groups per CU spill 17 registers: 189 us).
+template <int CT, int D>
+__global__ __launch_bounds__(256, 2) void block_sparse_fwd_small_kernel(FwdArgs a) {
+  __shared__ u32x4 lds_k[16 * D];
+  __shared__ u32x4 lds_v[16 * D];
+  fwd_qblock<CT, D>(a, (SA_LDS char*)lds_k, (SA_LDS char*)lds_v);
 }
 
 // fp32 operands: every value is split as x = hi + lo with hi = bf16(x) and
@@ -1277,11 +1314,23 @@ static int fwd_grid(const FwdArgs& a) {
   return a.order ? plan_launch_slots(rows, a.nqb) : rows;
 }
 
+// Whether the buffer copies can address K and V: the rows of a head do not overlap (a buffer
+// that ends after the last key then reads every later row as zero) and a head spans less than
+// 2 GiB.  The C ABI requires this at head dim 128; at 64 and 32 other strides (a broadcast key
+// dim, for one) take block_sparse_fwd_kernel, which addresses every row by itself.
+static bool buffer_rows(const FwdArgs& a, int D) {
+  const int64_t lim = (int64_t)1 << 31;
+  return a.Nk > 0 && a.ks[2] >= D && a.vs[2] >= D && a.Nk * a.ks[2] * 2 < lim && a.Nk * a.vs[2] * 2 < lim;
+}
+
 template <int IT, int CT>
 static hipError_t launch_fwd_dt(const FwdArgs& a, int D, hipStream_t stream) {
   const int grid = fwd_grid(a);
   if (D == 128)
     block_sparse_fwd_d128_kernel<CT><<<grid, 256, 0, stream>>>(a);
+  else if (buffer_rows(a, D))
+    if (D == 64) block_sparse_fwd_small_kernel<CT, 64><<<grid, 256, 0, stream>>>(a);
+    else block_sparse_fwd_small_kernel<CT, 32><<<grid, 256, 0, stream>>>(a);
   else if (D == 64)
     block_sparse_fwd_kernel<IT, CT, 64><<<grid, 256, 0, stream>>>(a);
   else

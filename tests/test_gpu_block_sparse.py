@@ -217,6 +217,28 @@ def test_head_dim_64_and_cross_lengths():
     _check(out, lse[..., 0], q, k, v, mask)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("Nq,Nk,layout", [(1, 1, "bhsd"), (31, 129, "bshd"), (130, 1, "bhsd"), (257, 1000, "bshd"),
+                                          (900, 640, "bhsd")])
+def test_small_head_dims_edges_and_key_strides(dtype, D, Nq, Nk, layout):
+    """Remainders of the 128-row tiles at head dims 32 and 64, both layouts; and keys whose rows
+    overlap (a broadcast key dim), which the buffer copies cannot address.  The row sums are
+    fp32 sums of unrounded exponentials: the lse is held to 1e-4 + 1e-5 |lse|."""
+    q, k, v = _inputs(2, 3, Nq, Nk, D, dtype, seed=Nq + Nk, layout=layout)
+    mask = _random_mask(2, 3, -(-Nq // 128), -(-Nk // 128), 0.5, seed=3, empty_rows=1 if Nq > 128 else 0)
+    plan = ops.block_sparse_plan(mask)
+    out, lse = ops.block_sparse_attention(q, k, v, plan)
+    _check(out, lse, q, k, v, mask)
+    ref_l = torch_ref.dense_masked_attention(q, k, v, mask)[1]
+    fin = torch.isfinite(ref_l)
+    assert ((lse.cpu() - ref_l)[fin].abs() <= 1e-4 + 1e-5 * ref_l[fin].abs()).all()
+    ke, ve = k[:, :, :1].expand(-1, -1, Nk, -1), v[:, :, :1].expand(-1, -1, Nk, -1)
+    assert ke.stride(2) == 0 or Nk == 1
+    oe, le = ops.block_sparse_attention(q, ke, ve, plan)
+    _check(oe, le, q, ke, ve, mask)
+
+
 def _chunk_layout(nbh, nqb):
     """Chunking of the launch order: heads [0, nbh_w) in Cw chunks (qb mod Cw), the heads
     of the partial last round of 8 in Cs = Cw * F finer chunks."""
