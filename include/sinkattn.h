@@ -212,8 +212,8 @@ int sinkattn_lse_mix(const void* sink_out, const int64_t sink_strides[4],
  * block_size 16, 32, 64 or 128 with D 128: bf16/f16 inputs use the bf16/f16 matrix cores
  * (products are exact, sums fp32) and a device workspace of
  * sinkattn_block_mass_pool_workspace_bytes() bytes (per-row block sums of the resident
- * work-groups, queried for the current device); f32 inputs at block_size 128, D 128 use
- * the fp32 matrix cores (nkb <= 256) and need no workspace.  Every other shape
+ * work-groups, queried for the current device); f32 inputs at these block sizes, D 128 use
+ * the fp32 matrix cores (up to about 490 key blocks) and need no workspace.  Every other shape
  * (block_size 1..1024, D 1..256, f32 otherwise) runs a generic kernel (fp32 dot products,
  * two passes over the keys, no workspace; the query may still return a size for a
  * matrix-core block size, which the call then leaves unused), limited by LDS to about
@@ -245,8 +245,9 @@ int sinkattn_block_mass_pool(const void* q, const void* k, int dtype,
  * D 128 (nd <= 1024 at block_size 128) run the persistent MFMA kernel: `workspace` is a
  * device buffer of at least sinkattn_max_pool_workspace_bytes(...) bytes (per-(row,
  * key-block) maxima of the rows in flight); calls that share one workspace must be
- * ordered on one stream.  Other shapes run the generic kernel (no workspace; same LDS
- * bound as the generic block-mass kernel).
+ * ordered on one stream.  f32 with D 128 (up to about 490 key blocks) runs on the fp32 matrix
+ * cores, other shapes on the generic kernel (no workspace; same LDS bound as the generic
+ * block-mass kernel).
  * ---------------------------------------------------------------------------------- */
 size_t sinkattn_max_pool_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t block_size,
                                          int dtype);

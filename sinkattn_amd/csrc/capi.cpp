@@ -438,7 +438,6 @@ int sinkattn_block_mass_pool(const void* q, const void* k, int dtype, int64_t B,
   a.scale = scale;
   a.out = out;
   a.ws = reinterpret_cast<float*>(workspace);
-  const bool at128 = block_size == 128 && D == 128;
   if (mass_mfma_block(block_size) && D == 128 && dtype != SINKATTN_F32) {  // persistent MFMA kernel, workspace slots
     if (workspace == nullptr) return fail("block_mass_pool: null workspace");
     if (k_strides[2] < D) return fail("block_mass_pool: k row stride below the head dim");
@@ -446,7 +445,7 @@ int sinkattn_block_mass_pool(const void* q, const void* k, int dtype, int64_t B,
       return fail("block_mass_pool: one head of k spans more than 2 GiB");
     return hip_status(sa::launch_block_mass_pool(a, dtype, (int)D, (hipStream_t)stream), "pool launch");
   }
-  if (at128 && a.nkb <= 256)  // fp32 MFMA kernel
+  if (dtype == SINKATTN_F32 && sa::pool_f32_mfma(a))  // fp32 MFMA kernel
     return hip_status(sa::launch_block_mass_pool(a, dtype, (int)D, (hipStream_t)stream), "pool launch");
   if ((rc = check_generic_pool("block_mass_pool", a, dtype)) != 0) return rc;
   return hip_status(sa::launch_block_mass_generic(a, dtype, (hipStream_t)stream), "pool launch");
@@ -487,6 +486,8 @@ int sinkattn_max_pool(const void* q, const void* k, int dtype, int64_t B, int64_
       return fail("max_pool: k row stride below the head dim or one head of k over 2 GiB");
     return hip_status(sa::launch_max_pool(a, dtype, (int)D, (hipStream_t)stream), "max_pool launch");
   }
+  if (dtype == SINKATTN_F32 && sa::pool_f32_mfma(a))  // fp32 MFMA kernel
+    return hip_status(sa::launch_max_pool(a, dtype, (int)D, (hipStream_t)stream), "max_pool launch");
   if ((rc = check_generic_pool("max_pool", a, dtype)) != 0) return rc;
   return hip_status(sa::launch_max_pool_generic(a, dtype, (hipStream_t)stream), "max_pool launch");
 }

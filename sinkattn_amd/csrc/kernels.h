@@ -112,6 +112,7 @@ int64_t plan_order_cache_ints(int rows, int nqb, int entries);
 hipError_t launch_block_sparse_plan(const PlanArgs& a, hipStream_t stream);
 hipError_t launch_block_sparse_fwd(const FwdArgs& a, int dtype, int D, hipStream_t stream);
 hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
+bool pool_f32_mfma(const PoolArgs& a);
 int block_mass_groups();
 int device_cu_count();
 // Resident work-groups of the persistent max-pool kernel: its workspace holds one slot per
@@ -121,7 +122,7 @@ hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stre
 int mean_pool_row_len(int D);
 hipError_t launch_mean_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
 // Any block size / head dim (pooling_generic.hip); LDS need, checked by the caller against
-// kGenericPoolMaxLds.
+// kGenericPoolMaxLds (the LDS of a CU).
 constexpr size_t kGenericPoolMaxLds = 160 * 1024;
 size_t generic_pool_lds_need(int D, int nkb, int dtype);
 hipError_t launch_block_mass_generic(const PoolArgs& a, int dtype, hipStream_t stream);

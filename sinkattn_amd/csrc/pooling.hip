@@ -9,9 +9,8 @@
 //     sums go to the group's slot ws[kb][row] of a global workspace.  The reference maximum
 //     is the row maximum of the first tile and moves only when a tile's sum exceeds 2^64
 //     (kSumLimit); then the row's earlier sums are rescaled.
-//   * fp32 (block_mass_f32_kernel): one group per q-block; the sums stay in LDS, and the
-//     reference maximum moves when a tile's maximum exceeds it by more than
-//     kRescaleMargin (log2 units), rescaling the earlier sums.
+//   * fp32 (block_mass_f32_kernel): one group per 64 query rows; the sums stay in LDS, the
+//     reference maximum as above.
 //   At the end every row is normalised by its own total and the rows are averaged per key
 //   block.
 //
@@ -27,8 +26,6 @@
 #include "tile.h"
 
 namespace sa {
-
-constexpr float kRescaleMargin = 8.f;  // block_mass_f32_kernel only
 
 // ------------------------------------------------------------------------------------
 // Exact block mass, 16-bit inputs, head dim 128, block size KB in {16, 32, 64, 128};
@@ -205,104 +202,360 @@ __global__ __launch_bounds__(256, 3) void block_mass_persistent_kernel(PoolArgs 
 }
 
 // ------------------------------------------------------------------------------------
-// Exact block mass, f32 inputs: fp32 matrix cores (v_mfma_f32_32x32x2_f32).
-// Work-group = 4 waves = 128 rows.  Each 128-key block is staged as four 32-key fp32
-// sub-tiles (rows padded to 132 floats).  The contraction index of MFMA step s is
-// d = s for lanes 0-31 and d = s + 64 for lanes 32-63, so four consecutive steps read
-// one 16-byte LDS vector.
+// Exact block mass, f32 inputs, head dim 128, block size KB in {16, 32, 64, 128}: fp32 matrix
+// cores (v_mfma_f32_16x16x4_f32, fp32 products and sums).  Bound by the matrix cores, 256 flops
+// per clock and CU in fp32.  An item is 64 query rows of one head, 16 per wave, so that a short
+// sequence still gives every CU an equal share ([1,12,4096,128]: 768 items, three per CU, where
+// items of 128 rows would load half the CUs twice).  K streams in tiles of 32 keys through two
+// LDS buffers by DMA, the next tile's copies issued a whole tile ahead, one barrier per tile.
+//     S^T[16 kt .. +16] = K Q^T   (A = 16 K rows from LDS, B = Q^T in VGPRs)
+// Lane l holds query l % 16 and, of every 16 channels, the four from 4 (l / 16): one 16-byte
+// read feeds four matrix instructions; its S^T registers hold keys 16 kt + 4 (l / 16) + i.  The
+// 16-byte chunks of a K row are swizzled by row & 15, so a 16-lane read touches 256 distinct
+// bytes.  A row's per-block sums of exp2(scale*log2e*s - m_ref) stay in LDS; m_ref is the row
+// maximum of the first tile and moves (rescaling the earlier sums) only when a tile's sum passes
+// 2^64.  [1,12,4096,128]: 0.45 ms,
+// 115 TFLOP/s of the 153 a large fp32 matrix product reaches here (0.70 ms with 32-key tiles
+// staged through registers behind two barriers); blocks of 64 at [2,10,6545,128] 2.0 ms (30.5 ms
+// on the generic kernel's VALU dot products).
+// XCD x (work-group i runs on XCD i % 8) takes the items [x, x + 1) * items_per_xcd, so that its
+// L2 holds few heads' K at a time.  Blocks of 128 rows span two items, whose halves meet in an
+// atomic add to the zeroed map (two addends: the sum does not depend on their order).
 // ------------------------------------------------------------------------------------
-template <int NKBMAX>
-__global__ __launch_bounds__(256) void block_mass_f32_kernel(PoolArgs a) {
-  constexpr int KP = 132;  // padded row length (floats)
-  __shared__ float lds_k[32 * KP];
-  __shared__ float sums[128 * NKBMAX];
-  __shared__ float row_tot[128];
+constexpr int kF32Rows = 64;  // query rows of an item
+constexpr int kF32Keys = 32;  // keys of a tile
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int hl = lane >> 5, l32 = lane & 31;
-  const int qb = blockIdx.x;
-  const int bh = blockIdx.y;
-  const int b = bh / a.H, h = bh - b * a.H;
-  const int nkb = a.nkb;
+__host__ __device__ inline int f32_sum_pitch(int nkb) { return nkb | 1; }  // floats: rows on distinct banks
+constexpr size_t kF32StaticLds = 2 * kF32Keys * 512 + kF32Rows * 4;
 
-  const float* qbase = (const float*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1]);
-  const float* kbase = (const float*)a.k + ((int64_t)b * a.ks[0] + (int64_t)h * a.ks[1]);
+// One item's view of the K stream: the copies of a tile and its scores.
+struct F32Tiles {
+  const char* kbase;
+  uint32_t kstride, doff[2], ka;
+  int Nk, wave;
+  f32x4 qv[8];  // Q^T B operands: this lane's channels 16 j + 4 (l / 16) ..
 
-  const int r = wave * 32 + l32;
-  const int qrow = qb * 128 + r;
-  float qf[64];
+  __device__ __forceinline__ F32Tiles(const PoolArgs& a, int b, int h, int hk, int qrow, int lane, int wave_)
+      : Nk(a.Nk), wave(wave_) {
+    const int g = lane >> 4, sl = lane & 15;
+    kbase = (const char*)a.k + ((int64_t)b * a.ks[0] + (int64_t)hk * a.ks[1]) * 4;
+    kstride = (uint32_t)a.ks[2] * 4;
+    // Copy j (of 4) of wave w fills tile rows 8j + 2w + lane / 32; the swizzle of those rows
+    // alternates with j.
+    const int drow = 2 * wave + (lane >> 5);
+    doff[0] = (uint32_t)drow * kstride + (uint32_t)(((lane & 31) ^ drow) * 16);
+    doff[1] = (uint32_t)drow * kstride + (uint32_t)(((lane & 31) ^ (drow + 8)) * 16);
+    ka = (uint32_t)(sl * 512 + ((g ^ sl) * 16));  // chunk 4 j + g: XOR 64 j
+    const float* q = (const float*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1] + (int64_t)qrow * a.qs[2]);
 #pragma unroll
-  for (int s4 = 0; s4 < 16; ++s4) {
-    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (qrow < a.Nq)
-      v = *reinterpret_cast<const f32x4*>(qbase + (int64_t)qrow * a.qs[2] + hl * 64 + s4 * 4);
-    qf[4 * s4] = v[0]; qf[4 * s4 + 1] = v[1]; qf[4 * s4 + 2] = v[2]; qf[4 * s4 + 3] = v[3];
+    for (int j = 0; j < 8; ++j)
+      qv[j] = qrow < a.Nq ? *reinterpret_cast<const f32x4*>(q + 16 * j + 4 * g) : f32x4{};
   }
 
-  const float c = a.scale * kLog2e;
-  float m_ref = neg_inf();
-  float* my = sums + r * NKBMAX;
+  __device__ __forceinline__ void copy(SA_LDS char* dst, int t) const {
+    const int key0 = t * kF32Keys;
+    const int valid = min(kF32Keys, Nk - key0);
+    // ends with the last valid row (rows may lie closer than 128 floats); keys past it are masked
+    const __amdgpu_buffer_rsrc_t rs =
+        make_rsrc(kbase + (int64_t)key0 * kstride, (uint32_t)(valid - 1) * kstride + 512u);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      dma16(rs, (SA_LDS void*)(dst + (4 * j + wave) * 1024), doff[j & 1] + (uint32_t)(8 * j) * kstride);
+  }
 
-  for (int kb = 0; kb < nkb; ++kb) {
-    float ps = 0.f;
-    for (int t = 0; t < 4; ++t) {
-      const int key0 = kb * 128 + t * 32;
-      __syncthreads();
+  __device__ __forceinline__ void scores(SA_LDS const char* cur, f32x4 (&s)[2]) const {
+    // four chains: the odd and even 16-channel steps apart (independent instructions, and half the
+    // additions in a row)
+    f32x4 acc[2][2] = {{f32x4{}, f32x4{}}, {f32x4{}, f32x4{}}};
 #pragma unroll
-      for (int i = 0; i < 32 * 32 / 256; ++i) {
-        const int id = i * 256 + tid;
-        const int row = id >> 5, c4 = id & 31;
-        const int key = key0 + row;
-        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (key < a.Nk) v = *reinterpret_cast<const f32x4*>(kbase + (int64_t)key * a.ks[2] + c4 * 4);
-        *reinterpret_cast<f32x4*>(lds_k + row * KP + c4 * 4) = v;
-      }
-      __syncthreads();
-      f32x16 s = f32x16{};
+    for (int j = 0; j < 8; ++j) {
+      f32x4 kv[2];
 #pragma unroll
-      for (int s4 = 0; s4 < 16; ++s4) {
-        const f32x4 av = *reinterpret_cast<const f32x4*>(lds_k + l32 * KP + hl * 64 + s4 * 4);
+      for (int kt = 0; kt < 2; ++kt) kv[kt] = *(SA_LDS const f32x4*)(cur + (ka ^ (64u * j)) + kt * 8192);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          s = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], qf[4 * s4 + e], s, 0, 0, 0);
-      }
-      if (key0 + 32 > a.Nk) {
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
-          if (key0 + 8 * (j >> 2) + 4 * hl + (j & 3) >= a.Nk) s[j] = neg_inf();
-      }
+        for (int kt = 0; kt < 2; ++kt)
+          acc[j & 1][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[kt][e], qv[j][e], acc[j & 1][kt], 0, 0, 0);
+    }
+    s[0] = acc[0][0] + acc[1][0];
+    s[1] = acc[0][1] + acc[1][1];
+  }
+};
+
+template <int KB>
+__global__ __launch_bounds__(256, 3) void block_mass_f32_kernel(PoolArgs a, int items, int items_per_xcd) {
+  constexpr int TPB = KB > kF32Keys ? KB / kF32Keys : 1;  // tiles per key block
+  constexpr int NS = KB < kF32Keys ? kF32Keys / KB : 1;   // key blocks per tile
+  extern __shared__ float sums[];  // [64][f32_sum_pitch(nkb)]
+  // each buffer its own variable: through one the compiler makes a tile's reads wait for the
+  // next tile's copies
+  __shared__ u32x4 lds_k0[kF32Keys * 32];
+  __shared__ u32x4 lds_k1[kF32Keys * 32];
+  __shared__ float row_inv[kF32Rows];
+  const int item = (int)(blockIdx.x % kXcds) * items_per_xcd + (int)(blockIdx.x / kXcds);
+  if (item >= items) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, sl = lane & 15;
+  const int nkb = a.nkb, pitch = f32_sum_pitch(nkb);
+  const int ntiles = (a.Nk + kF32Keys - 1) / kF32Keys;
+  const int nqi = (a.Nq + kF32Rows - 1) / kF32Rows;
+  const int bh = item / nqi, qi = item - bh * nqi;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int r = wave * 16 + sl;  // this lane's row of the item
+  const int qrow = qi * kF32Rows + r;
+  const F32Tiles tl(a, b, h, h, qrow, lane, wave);
+  tl.copy((SA_LDS char*)lds_k0, 0);
+  const float c = a.scale * kLog2e;
+  float m_ref = 0.f, l_tot = 0.f, run = 0.f;
+  float* my = sums + r * pitch;
+
+  auto tile = [&](int t, SA_LDS char* cur, SA_LDS char* next) __attribute__((always_inline)) {
+    drain_then_barrier();  // tile t has landed; every wave is done with the other buffer
+    if (t + 1 < ntiles) tl.copy(next, t + 1);
+    f32x4 s[2];
+    tl.scores(cur, s);
+    const int left = a.Nk - t * kF32Keys - 4 * g;  // key 16 kt + i of this lane exists when below it
+    const bool cut = (t + 1) * kF32Keys > a.Nk;
+    auto row_max = [&]() __attribute__((always_inline)) {
       float mx = neg_inf();
 #pragma unroll
-      for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[j]);
-      mx = max_xor32(mx) * c;
-      if (mx > m_ref + kRescaleMargin) {
-        const float f = fast_exp2(m_ref - mx);
-        for (int j = hl; j < kb; j += 2) my[j] *= f;
-        ps *= f;
-        m_ref = mx;
-      }
+      for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) ps += fast_exp2(__builtin_fmaf(s[j], c, -m_ref));
+        for (int i = 0; i < 4; ++i)
+          if (!cut || 16 * kt + i < left) mx = fmaxf(mx, s[kt][i] * c);
+      return max_col16(mx);
+    };
+    if (t == 0) m_ref = row_max();  // key 0 always exists
+    float ps[2];
+    auto tile_sums = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        ps[kt] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = fast_exp2(__builtin_fmaf(s[kt][i], c, -m_ref));
+          ps[kt] += !cut || 16 * kt + i < left ? e : 0.f;
+        }
+        ps[kt] = sum_col16(ps[kt]);
+      }
+    };
+    tile_sums();
+    if (!(ps[0] + ps[1] <= kSumLimit)) {
+      // Rare: scores far above m_ref.  Move m_ref to this tile's maximum and rescale the row's
+      // earlier sums (the row's four lanes split them).
+      const float mx = row_max();
+      const float f = fast_exp2(m_ref - mx);
+      for (int j = g; j < t * NS / TPB; j += 4) my[j] *= f;
+      l_tot *= f;
+      run *= f;
+      m_ref = mx;
+      tile_sums();
     }
-    ps = sum_xor32(ps);
-    if (hl == 0) my[kb] = ps;
+    l_tot += ps[0] + ps[1];
+    if constexpr (NS == 2) {
+      if (g < 2 && 2 * t + g < nkb) my[2 * t + g] = g == 0 ? ps[0] : ps[1];
+    } else {
+      run += ps[0] + ps[1];
+      if ((t + 1) % TPB == 0 || t + 1 == ntiles) {
+        if (g == 0) my[t / TPB] = run;
+        run = 0.f;
+      }
+    }
+  };
+  for (int t = 0; t < ntiles; t += 2) {
+    tile(t, (SA_LDS char*)lds_k0, (SA_LDS char*)lds_k1);
+    if (t + 1 < ntiles) tile(t + 1, (SA_LDS char*)lds_k1, (SA_LDS char*)lds_k0);
   }
+
+  if (g == 0) row_inv[r] = qrow < a.Nq ? 1.f / fmaxf(l_tot, 1e-6f) : 0.f;
   __syncthreads();
-  {
-    float tot = 0.f;
-    for (int j = hl; j < nkb; j += 2) tot += my[j];
-    tot = sum_xor32(tot);
-    if (hl == 0) row_tot[r] = tot;
+  // Map entries: the mean over a q-block's rows of sum / total.
+  constexpr int RB = KB < kF32Rows ? KB : kF32Rows;  // rows of this item in one q-block
+  float* out = reinterpret_cast<float*>(a.out);
+  for (int qs = 0; qs < kF32Rows / RB; ++qs) {
+    const int qb = (qi * kF32Rows + qs * RB) / KB;
+    const int rows = min(KB, a.Nq - qb * KB);  // rows of the whole q-block
+    if (qb >= a.nqb) break;
+    for (int kb = tid; kb < nkb; kb += 256) {
+      float acc = 0.f;
+#pragma unroll 8
+      for (int rr = 0; rr < RB; ++rr) acc += sums[(qs * RB + rr) * pitch + kb] * row_inv[qs * RB + rr];
+      float* dst = out + ((int64_t)bh * a.nqb + qb) * nkb + kb;
+      if constexpr (KB > kF32Rows) atomicAdd(dst, acc / (float)rows);
+      else *dst = acc / (float)rows;
+    }
   }
+}
+
+__global__ __launch_bounds__(256) void fill_zero_kernel(float* p, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.f;
+}
+
+// Whether the fp32 matrix-core kernels take a call: head dim 128, a block size they have, the
+// values of an item's rows within the CU's LDS beside the K tiles (about 490 key blocks), a tile
+// of K rows within a buffer's 32-bit offsets, and an item count within the grid.  Any other
+// call runs the generic kernels (6-7 TFLOP/s against 100-125).
+bool pool_f32_mfma(const PoolArgs& a) {
+  return a.D == 128 && (a.bs == 16 || a.bs == 32 || a.bs == 64 || a.bs == 128) &&
+         kF32StaticLds + (size_t)kF32Rows * f32_sum_pitch(a.nkb) * 4 <= kGenericPoolMaxLds &&
+         a.ks[2] * 4 * kF32Keys < ((int64_t)1 << 31) &&
+         (int64_t)a.B * a.H * (a.Nq / kF32Rows + 1) < ((int64_t)1 << 30);
+}
+
+// The kernel's dynamic LDS and, where two items share a map entry, the zeroed map.
+static hipError_t f32_pool_setup(const void* kern, const PoolArgs& a, bool zero, size_t lds, hipStream_t stream) {
+  const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess || !zero) return e;
+  const int64_t n = (int64_t)a.B * a.H * a.nqb * a.nkb;
+  fill_zero_kernel<<<(int)min((int64_t)1024, (n + 255) / 256), 256, 0, stream>>>((float*)a.out, n);
+  return hipGetLastError();
+}
+
+template <int KB>
+static hipError_t launch_mass_f32(const PoolArgs& a, hipStream_t stream) {
+  const int items = a.B * a.H * ((a.Nq + kF32Rows - 1) / kF32Rows);
+  const int per = (items + kXcds - 1) / kXcds;
+  const size_t lds = (size_t)kF32Rows * f32_sum_pitch(a.nkb) * 4;
+  const hipError_t e =
+      f32_pool_setup(reinterpret_cast<const void*>(block_mass_f32_kernel<KB>), a, KB > kF32Rows, lds, stream);
+  if (e != hipSuccess) return e;
+  block_mass_f32_kernel<KB><<<per * kXcds, 256, lds, stream>>>(a, items, per);
+  return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------
+// Max-pool map, f32 inputs, head dim 128: the tiles and items of block_mass_f32_kernel with each
+// row's block maxima R[r,kb] = max_j s * (sm_scale * log2e) in LDS (fp32, so the reference's
+// rounding of R to q.dtype is the identity) and m_r the maximum over the row.  Po[qb,kb] =
+// max over the block's rows of exp2(R - m_r); rows past the end take m = +inf, which gives 0.
+// The maximum is taken over the bits (values >= 0, a NaN above them all), atomically into the
+// zeroed map where a block of 128 rows spans two items; max_pool_f32_norm_kernel then divides
+// each map row by its sum.  Causal: key blocks after the query block are not seen and raw scores
+// above the diagonal of the diagonal block get -1e6.  [1,10,6545,128]: 1.07 ms at
+// blocks of 128 and 1.1 at 64 (19.1 ms on the generic kernel).
+// ------------------------------------------------------------------------------------
+template <int KB>
+__global__ __launch_bounds__(256, 3) void max_pool_f32_kernel(PoolArgs a, int items, int items_per_xcd) {
+  constexpr int TPB = KB > kF32Keys ? KB / kF32Keys : 1;
+  constexpr int NS = KB < kF32Keys ? kF32Keys / KB : 1;
+  extern __shared__ float maxima[];  // [64][f32_sum_pitch(nkb)]
+  __shared__ u32x4 lds_k0[kF32Keys * 32];
+  __shared__ u32x4 lds_k1[kF32Keys * 32];
+  __shared__ float row_m[kF32Rows];
+  const int item = (int)(blockIdx.x % kXcds) * items_per_xcd + (int)(blockIdx.x / kXcds);
+  if (item >= items) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, sl = lane & 15;
+  const int nkb = a.nkb, pitch = f32_sum_pitch(nkb);
+  const int nqi = (a.Nq + kF32Rows - 1) / kF32Rows;
+  const int bh = item / nqi, qi = item - bh * nqi;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int r = wave * 16 + sl;
+  const int qrow = qi * kF32Rows + r;
+  const int qbr = qrow / KB;  // this row's q-block
+  // keys any row of the item sees
+  const int key_end = a.causal ? min(a.Nk, ((qi * kF32Rows + kF32Rows - 1) / KB + 1) * KB) : a.Nk;
+  const int ntiles = (key_end + kF32Keys - 1) / kF32Keys;
+  const F32Tiles tl(a, b, h, h / (a.H / a.Hk), qrow, lane, wave);
+  tl.copy((SA_LDS char*)lds_k0, 0);
+  // The reference forms qk_scale = fp32(sm_scale) * fp32(1.44269504).
+  const float c = a.scale * 1.44269504f;
+  float m = neg_inf(), run = neg_inf();
+  float* my = maxima + r * pitch;
+
+  auto tile = [&](int t, SA_LDS char* cur, SA_LDS char* next) __attribute__((always_inline)) {
+    drain_then_barrier();  // tile t has landed; every wave is done with the other buffer
+    if (t + 1 < ntiles) tl.copy(next, t + 1);
+    f32x4 s[2];
+    tl.scores(cur, s);
+    const int key0 = t * kF32Keys;
+    if ((t + 1) * kF32Keys > a.Nk || (a.causal && key0 + kF32Keys > qi * kF32Rows / KB * KB)) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = key0 + 16 * kt + 4 * g + i;
+          if (a.causal) {
+            if (key / KB == qbr && qrow < key) s[kt][i] += -1.0e6f;
+            if (key / KB > qbr) s[kt][i] = neg_inf();
+          }
+          if (key >= a.Nk) s[kt][i] = neg_inf();
+        }
+    }
+    float mx[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      mx[kt] = neg_inf();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        mx[kt] = fmaxf(mx[kt], s[kt][i]);
+        if (s[kt][i] != neg_inf()) m = fmaxf(m, s[kt][i] * c);
+      }
+      mx[kt] = max_col16(mx[kt]);
+    }
+    if constexpr (NS == 2) {
+      if (g < 2 && 2 * t + g < nkb) my[2 * t + g] = (g == 0 ? mx[0] : mx[1]) * c;
+    } else {
+      run = fmaxf(run, fmaxf(mx[0], mx[1]));
+      if ((t + 1) % TPB == 0 || t + 1 == ntiles) {
+        if (g == 0) my[t / TPB] = run * c;
+        run = neg_inf();
+      }
+    }
+  };
+  for (int t = 0; t < ntiles; t += 2) {
+    tile(t, (SA_LDS char*)lds_k0, (SA_LDS char*)lds_k1);
+    if (t + 1 < ntiles) tile(t + 1, (SA_LDS char*)lds_k1, (SA_LDS char*)lds_k0);
+  }
+
+  m = max_col16(m);
+  if (g == 0) row_m[r] = qrow < a.Nq ? m : pos_inf();
   __syncthreads();
-  const int nrows = min(128, a.Nq - qb * 128);
-  float* out = reinterpret_cast<float*>(a.out) + ((int64_t)bh * a.nqb + qb) * nkb;
-  for (int kb = tid; kb < nkb; kb += 256) {
-    float acc = 0.f;
-    for (int rr = 0; rr < nrows; ++rr) acc += sums[rr * NKBMAX + kb] / fmaxf(row_tot[rr], 1e-6f);
-    out[kb] = acc / (float)nrows;
+  constexpr int RB = KB < kF32Rows ? KB : kF32Rows;  // rows of this item in one q-block
+  unsigned* out = reinterpret_cast<unsigned*>(a.out);
+  for (int qs = 0; qs < kF32Rows / RB; ++qs) {
+    const int qb = (qi * kF32Rows + qs * RB) / KB;
+    if (qb >= a.nqb) break;
+    const int kb_end = a.causal ? min(nkb, qb + 1) : nkb;
+    for (int kb = tid; kb < kb_end; kb += 256) {
+      unsigned v = 0u;
+#pragma unroll 8
+      for (int rr = 0; rr < RB; ++rr)
+        v = max(v, __float_as_uint(fast_exp2(maxima[(qs * RB + rr) * pitch + kb] - row_m[qs * RB + rr])));
+      unsigned* dst = out + ((int64_t)bh * a.nqb + qb) * nkb + kb;
+      if constexpr (KB > kF32Rows) atomicMax(dst, v);
+      else *dst = v;
+    }
   }
+}
+
+// Map rows divided by their sums (one wave per row); entries past a causal row's end are 0.
+__global__ __launch_bounds__(256) void max_pool_f32_norm_kernel(PoolArgs a) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= a.B * a.H * a.nqb) return;
+  const int kb_end = a.causal ? min(a.nkb, row % a.nqb + 1) : a.nkb;
+  float* p = reinterpret_cast<float*>(a.out) + (int64_t)row * a.nkb;
+  float sum = 0.f;
+  for (int kb = lane; kb < kb_end; kb += 64) sum += p[kb];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  for (int kb = lane; kb < a.nkb; kb += 64) p[kb] = kb < kb_end ? p[kb] / sum : 0.f;
+}
+
+template <int KB>
+static hipError_t launch_max_f32(const PoolArgs& a, hipStream_t stream) {
+  const int items = a.B * a.H * ((a.Nq + kF32Rows - 1) / kF32Rows);
+  const int per = (items + kXcds - 1) / kXcds;
+  const size_t lds = (size_t)kF32Rows * f32_sum_pitch(a.nkb) * 4;
+  hipError_t e = f32_pool_setup(reinterpret_cast<const void*>(max_pool_f32_kernel<KB>), a, KB > kF32Rows, lds, stream);
+  if (e != hipSuccess) return e;
+  max_pool_f32_kernel<KB><<<per * kXcds, 256, lds, stream>>>(a, items, per);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  max_pool_f32_norm_kernel<<<(a.B * a.H * a.nqb + 3) / 4, 256, 0, stream>>>(a);
+  return hipGetLastError();
 }
 
 // Rounding of an fp32 value to the 16-bit type CT (returned as fp32).
@@ -708,11 +961,13 @@ int max_pool_groups() { return 4 * device_cu_count(); }
 hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream) {
   (void)D;
   if (a.B * a.H * a.nqb == 0) return hipSuccess;
-  const dim3 grid(a.nqb, a.B * a.H);
   if (dtype == kF32) {
-    if (a.nkb <= 64) block_mass_f32_kernel<64><<<grid, 256, 0, stream>>>(a);
-    else block_mass_f32_kernel<256><<<grid, 256, 0, stream>>>(a);
-    return hipGetLastError();
+    switch (a.bs) {
+      case 16: return launch_mass_f32<16>(a, stream);
+      case 32: return launch_mass_f32<32>(a, stream);
+      case 64: return launch_mass_f32<64>(a, stream);
+      default: return launch_mass_f32<128>(a, stream);
+    }
   }
   const int items = a.B * a.H * ((a.Nq + 127) / 128);
   const int groups = min(items, block_mass_groups());
@@ -736,6 +991,14 @@ hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream
 hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream) {
   (void)D;
   if (a.B * a.H * a.nqb == 0) return hipSuccess;
+  if (dtype == kF32) {
+    switch (a.bs) {
+      case 16: return launch_max_f32<16>(a, stream);
+      case 32: return launch_max_f32<32>(a, stream);
+      case 64: return launch_max_f32<64>(a, stream);
+      default: return launch_max_f32<128>(a, stream);
+    }
+  }
   const int items = a.B * a.H * ((a.Nq + 127) / 128);
   const int groups = min(items, max_pool_groups());
 #define SA_MAXP(KB)                                                                  \

@@ -1,5 +1,5 @@
 // Block-score kernels for any block size and head dim (the MFMA kernels in pooling.hip
-// cover block 128 / head dim 128, the shapes the calibration runs at).
+// cover blocks 16, 32, 64 and 128 at head dim 128, the shapes the calibration runs at).
 //
 // block_mass_generic: `_compute_exact_block_mass_scores` (sinkattention/sparse_attention.py
 //   :145-227) for block sizes 1..1024, head dims 1..256, bf16/f16/f32.

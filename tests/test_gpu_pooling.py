@@ -290,6 +290,46 @@ def test_pooling_mode_dispatch():
     assert t.dtype == torch.float32 and t.shape == (1, 2, 2, 2)
 
 
+# The fp32 matrix-core kernels (head dim 128, blocks 16-128): items of 64 rows (two to a
+# 128-row block), tiles of 32 keys (two blocks of 16 each), the last key counts before the row
+# values no longer fit LDS, keys whose rows overlap, and the 2^64 rescale.  Bar: the pooling
+# bar of 1e-5 relative (fp32 products and sums on both sides).
+@pytest.mark.parametrize("bs,Nq,Nk", [(128, 1, 1), (128, 193, 127), (128, 64, 500), (64, 65, 33), (64, 130, 2000),
+                                      (32, 63, 31), (32, 300, 257), (16, 79, 49), (16, 90, 7830)])
+def test_exact_mass_f32_tile_edges(bs, Nq, Nk):
+    g = torch.Generator().manual_seed(bs + Nq)
+    q = torch.randn(2, Nq, 3, 128, generator=g).transpose(1, 2)
+    k = torch.randn(2, Nk, 3, 128, generator=g).transpose(1, 2)
+    k[:, :, : Nk // 3] -= 4.0 * (Nq % 2)
+    _close(ops.block_mass_scores(q.cuda(), k.cuda(), block_size=bs), torch_ref.exact_block_mass(q, k, block_size=bs))
+    ke = k[:, :, :1].expand(-1, -1, Nk, -1)
+    _close(ops.block_mass_scores(q.cuda(), k.cuda()[:, :, :1].expand(-1, -1, Nk, -1), block_size=bs),
+           torch_ref.exact_block_mass(q, ke.contiguous(), block_size=bs))
+
+
+@pytest.mark.parametrize("bs", [16, 32, 64, 128])
+def test_exact_mass_f32_rescale(bs):
+    g = torch.Generator().manual_seed(bs)
+    q = 0.5 + 0.1 * torch.randn(1, 2, 200, 128, generator=g)
+    k = torch.randn(1, 2, 500, 128, generator=g)
+    k[:, :, :128] = -10.0  # ~80 log2 units below the keys after them
+    ours = ops.block_mass_scores(q.cuda(), k.cuda(), block_size=bs)
+    _close(ours, torch_ref.exact_block_mass(q, k, block_size=bs))
+    assert float(ours[..., : 128 // bs].sum(-1).max()) < 1e-20
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bs,H,Hk,N", [(128, 2, 2, 1), (128, 4, 2, 321), (64, 2, 1, 190), (32, 2, 2, 333),
+                                       (16, 4, 4, 259), (16, 1, 1, 7800)])
+def test_max_pool_f32_tile_edges(bs, H, Hk, N, causal):
+    """exp2 of fp32 scores of 128 products each: the fp32 bar below, as on the generic kernel."""
+    q, k = _qkd(1, H, Hk, N, N, 128, torch.float32, seed=bs + N)
+    sm = 1.0 / 128 ** 0.5
+    ours = ops.max_pool_scores(q.cuda(), k.cuda(), sm, block_size=bs, causal=causal).cpu()
+    ref = torch_ref.max_pool_map(q, k, sm, block_size=bs, causal=causal)
+    assert torch.allclose(ours, ref, rtol=2e-5, atol=1e-8)
+
+
 @pytest.mark.parametrize("B,H,Nq,Nk,bs,D", [(1, 1, 1, 1, 128, 128), (1, 2, 17 * 16 + 1, 33, 16, 128),
                                             (2, 1, 40, 600, 1, 64), (1, 1, 300, 1030, 2, 256),
                                             (1, 2, 5000, 2600, 1024, 48), (1, 1, 65, 64, 4, 8)])
