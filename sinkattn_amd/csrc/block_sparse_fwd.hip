@@ -586,17 +586,22 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_small_kernel(FwdArgs 
 
 // fp32 operands: every value is split as x = hi + lo with hi = bf16(x) and
 // lo = bf16(x - hi); each product is formed as hi*hi + hi*lo + lo*hi on the bf16 matrix
-// cores (about 16 mantissa bits), for QK^T and for PV (P split the same way).  Same
-// tiling as block_sparse_fwd_kernel; the hi and lo tiles of K and V^T double the LDS.
+// cores (about 16 mantissa bits), for QK^T and for PV (P split the same way).  Bound by those
+// three products (12 D flops per score).  The layouts, transpose reads and softmax of the
+// 16-bit tile loop on steps of 64 keys, whose four tiles (K and V, hi and lo) take 64 KB at
+// D = 128, so that two groups share a CU.  The tiles pass through registers, where they are
+// split, in two halves to stay within 256 VGPRs: a step's V is loaded before S and before the
+// softmax and written after them, the next step's K loaded before and halfway through PV, so the
+// loads fly under matrix instructions and a step has two barriers.  Row sums are fp32 sums of
+// unrounded exponentials.  [2,12,5001,128] at 35% density and one dense head: 0.45 ms, 0.30
+// PFLOP/s of fp32 work (0.93 ms with tiles of 128 keys, one group per CU and V transposed while
+// staging); [1,12,4096,128] at 74%: 0.28 ms (0.49).
 __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& hi, uint32_t& lo) {
-  const float h0 = (float)(__bf16)x0, h1 = (float)(__bf16)x1;
-  hi = pack2<kBF16>(h0, h1);
-  lo = pack2<kBF16>(x0 - h0, x1 - h1);
+  hi = pack2<kBF16>(x0, x1);
+  lo = pack2<kBF16>(x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xffff0000u));
 }
 
-__device__ __forceinline__ void split8(const float* p, u32x4& hi, u32x4& lo) {
-  const f32x4 a = reinterpret_cast<const f32x4*>(p)[0];
-  const f32x4 b = reinterpret_cast<const f32x4*>(p)[1];
+__device__ __forceinline__ void split8(f32x4 a, f32x4 b, u32x4& hi, u32x4& lo) {
   uint32_t h[4], l[4];
   split_pair(a[0], a[1], h[0], l[0]);
   split_pair(a[2], a[3], h[1], l[1]);
@@ -606,163 +611,226 @@ __device__ __forceinline__ void split8(const float* p, u32x4& hi, u32x4& lo) {
   lo = u32x4{l[0], l[1], l[2], l[3]};
 }
 
+// Part P (of 2) of a 64-row tile: D / 32 pieces of 8 floats per thread in the whole tile.  `src` is
+// this thread's first piece, (tid / (D / 8)) rows in; rows at or past `rows` are zero.
 template <int D>
-__global__ __launch_bounds__(256) void block_sparse_fwd_f32_kernel(FwdArgs a) {
-  constexpr int KC = D / 8, DS = D / 16, DT = D / 32;
-  __shared__ u32x4 kh[128 * KC], kl[128 * KC];
-  __shared__ u32x4 vh[D * 16], vl[D * 16];
+struct F32Part {
+  static constexpr int kPieces = D / 32, kFirst = (kPieces + 1) / 2;
+  static constexpr int kRowStep = 256 / (D / 8);  // rows between a thread's pieces
+  f32x4 x[kFirst][2];
 
+  template <int P>
+  __device__ __forceinline__ void load(const float* src, int64_t stride, int rows, int tid) {
+    auto piece = [&](int i) __attribute__((always_inline)) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(src + (int64_t)(i * kRowStep) * stride);
+      x[i - P * kFirst][0] = p[0];
+      x[i - P * kFirst][1] = p[1];
+    };
+    if (rows >= 64) {  // the whole tile (wave-uniform)
+#pragma unroll
+      for (int i = P * kFirst; i < (P ? kPieces : kFirst); ++i) piece(i);
+    } else {
+#pragma unroll
+      for (int i = P * kFirst; i < (P ? kPieces : kFirst); ++i) {
+        x[i - P * kFirst][0] = x[i - P * kFirst][1] = f32x4{};
+        if (i * kRowStep + tid / (D / 8) < rows) piece(i);
+      }
+    }
+  }
+
+  // The part split into the hi and lo tiles, chunks swizzled as the 16-bit K or V tile.
+  template <int P, bool V>
+  __device__ __forceinline__ void write(SA_LDS char* hi, SA_LDS char* lo, int tid) const {
+    using G = TileGeom<D>;
+#pragma unroll
+    for (int i = P * kFirst; i < (P ? kPieces : kFirst); ++i) {
+      const int row = i * kRowStep + tid / G::kChunks, ch = tid % G::kChunks;
+      const int at = row * G::kRow + ((ch ^ (V ? G::vswz(row) : G::kswz(row))) * 16);
+      u32x4 h, l;
+      split8(x[i - P * kFirst][0], x[i - P * kFirst][1], h, l);
+      *(SA_LDS u32x4*)(hi + at) = h;
+      *(SA_LDS u32x4*)(lo + at) = l;
+    }
+  }
+};
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void block_sparse_fwd_f32_kernel(FwdArgs a) {
+  constexpr int KS = D / 32, DT = D / 16;
+  __shared__ u32x4 lds_kh[8 * D], lds_kl[8 * D], lds_vh[8 * D], lds_vl[8 * D];
+  SA_LDS char* kh = (SA_LDS char*)lds_kh;
+  SA_LDS char* kl = (SA_LDS char*)lds_kl;
+  SA_LDS char* vh = (SA_LDS char*)lds_vh;
+  SA_LDS char* vl = (SA_LDS char*)lds_vl;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int hl = lane >> 5, l32 = lane & 31;
-  const int item = a.order ? a.order[blockIdx.x] : (int)blockIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, sl = lane & 15;
+  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[blockIdx.x] : (int)blockIdx.x);
   if (item < 0) return;
   const int bh = item / a.nqb;
   const int qb = item - bh * a.nqb;
   const int b = bh / a.H, h = bh - b * a.H;
-  const int cnt = a.counts[item];
-  const int32_t* list = a.idx + (int64_t)item * a.nkb;
+  // the plan through the constant address space: scalar loads
+  const int cnt = __builtin_amdgcn_readfirstlane(((const SA_CONST int32_t*)a.counts)[item]);
+  const SA_CONST int32_t* list = (const SA_CONST int32_t*)(a.idx + (int64_t)item * a.nkb);
   const float* qbase = (const float*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1]);
   const float* kbase = (const float*)a.k + ((int64_t)b * a.ks[0] + (int64_t)h * a.ks[1]);
   const float* vbase = (const float*)a.v + ((int64_t)b * a.vs[0] + (int64_t)h * a.vs[1]);
-
-  const int qrow = qb * 128 + wave * 32 + l32;
-  u32x4 qh[DS], ql[DS];
-#pragma unroll
-  for (int s = 0; s < DS; ++s) {
-    qh[s] = u32x4{0, 0, 0, 0};
-    ql[s] = u32x4{0, 0, 0, 0};
-    if (qrow < a.Nq) split8(qbase + (int64_t)qrow * a.qs[2] + s * 16 + hl * 8, qh[s], ql[s]);
-  }
-  f32x16 o[DT];
-#pragma unroll
-  for (int i = 0; i < DT; ++i) o[i] = f32x16{};
-  float m_run = neg_inf(), l_run = 0.f;
+  const TileLanes<D> L = tile_lanes<D>(wave, lane, 0, 0);
   const float c = a.scale * kLog2e;
-  const int prow = k_row_perm(l32);
-  const int fk = k_swz_kc<KC>(prow);
 
-  for (int it = 0; it < cnt; ++it) {
-    const int key0 = list[it] * 128;
-    __syncthreads();
+  // Q^T B operands, split: query 16 qt + l % 16 of the wave's rows, d slice 32 ks + 8 (l / 16)
+  u32x4 qh[2][KS], ql[2][KS];
 #pragma unroll
-    for (int c8 = 0; c8 < D / 16; ++c8) {
-      const int id = c8 * 256 + tid;
-      const int row = id / KC, ch = id % KC;
-      const int key = key0 + row;
-      u32x4 hi = u32x4{0, 0, 0, 0}, lo = u32x4{0, 0, 0, 0};
-      if (key < a.Nk) split8(kbase + (int64_t)key * a.ks[2] + ch * 8, hi, lo);
-      kh[row * KC + (ch ^ k_swz_kc<KC>(row))] = hi;
-      kl[row * KC + (ch ^ k_swz_kc<KC>(row))] = lo;
-    }
+  for (int qt = 0; qt < 2; ++qt) {
+    const int qrow = qb * 128 + wave * 32 + 16 * qt + sl;
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) {
-      const int id = i * 256 + tid;
-      const int dp = id % (D / 2), kg = id / (D / 2);
-      uint32_t wh[8], wl[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = key0 + kg * 8 + e;
-        f32x2 x = f32x2{0.f, 0.f};
-        if (key < a.Nk) x = *reinterpret_cast<const f32x2*>(vbase + (int64_t)key * a.vs[2] + 2 * dp);
-        split_pair(x[0], x[1], wh[e], wl[e]);
+    for (int ks = 0; ks < KS; ++ks) {
+      f32x4 x0 = f32x4{}, x1 = f32x4{};
+      if (qrow < a.Nq) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(qbase + (int64_t)qrow * a.qs[2] + 32 * ks + 8 * g);
+        x0 = p[0];
+        x1 = p[1];
       }
-      u32x4 eh, oh, el, ol;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        eh[j] = (wh[2 * j] & 0xffffu) | (wh[2 * j + 1] << 16);
-        oh[j] = (wh[2 * j] >> 16) | (wh[2 * j + 1] & 0xffff0000u);
-        el[j] = (wl[2 * j] & 0xffffu) | (wl[2 * j + 1] << 16);
-        ol[j] = (wl[2 * j] >> 16) | (wl[2 * j + 1] & 0xffff0000u);
-      }
-      const int d0 = 2 * dp;
-      vh[d0 * 16 + (kg ^ v_swz(d0))] = eh;
-      vh[(d0 + 1) * 16 + (kg ^ v_swz(d0 + 1))] = oh;
-      vl[d0 * 16 + (kg ^ v_swz(d0))] = el;
-      vl[(d0 + 1) * 16 + (kg ^ v_swz(d0 + 1))] = ol;
-    }
-    __syncthreads();
-
-    f32x16 s[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) s[t] = f32x16{};
-#pragma unroll
-    for (int ds = 0; ds < DS; ++ds)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int idx = (t * 32 + prow) * KC + ((2 * ds + hl) ^ fk);
-        const u32x4 ah = kh[idx], al = kl[idx];
-        s[t] = mfma32x32x16<kBF16>(ah, qh[ds], s[t]);
-        s[t] = mfma32x32x16<kBF16>(ah, ql[ds], s[t]);
-        s[t] = mfma32x32x16<kBF16>(al, qh[ds], s[t]);
-      }
-    if (key0 + 128 > a.Nk) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-          if (key0 + t * 32 + tile_key(hl, j) >= a.Nk) s[t][j] = neg_inf();
-    }
-    float mx = neg_inf();
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[t][j]);
-    mx = max_xor32(mx);
-    const float m_new = fmaxf(m_run, mx * c);
-    const float alpha = fast_exp2(m_run - m_new);
-    l_run *= alpha;
-#pragma unroll
-    for (int i = 0; i < DT; ++i) o[i] *= alpha;
-    u32x4 ph[4][2], pl[4][2];
-    float lsum = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float v0 = fast_exp2(__builtin_fmaf(s[t][8 * u + 2 * e], c, -m_new));
-          const float v1 = fast_exp2(__builtin_fmaf(s[t][8 * u + 2 * e + 1], c, -m_new));
-          lsum += v0 + v1;
-          uint32_t hv, lv;
-          split_pair(v0, v1, hv, lv);
-          ph[t][u][e] = hv;
-          pl[t][u][e] = lv;
-        }
-    l_run += lsum;
-    m_run = m_new;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const int R = dt * 32 + l32;
-      const int fv = v_swz(R);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int idx = R * 16 + ((4 * t + 2 * u + hl) ^ fv);
-          const u32x4 ah = vh[idx], al = vl[idx];
-          o[dt] = mfma32x32x16<kBF16>(ah, ph[t][u], o[dt]);
-          o[dt] = mfma32x32x16<kBF16>(ah, pl[t][u], o[dt]);
-          o[dt] = mfma32x32x16<kBF16>(al, ph[t][u], o[dt]);
-        }
+      split8(x0, x1, qh[qt][ks], ql[qt][ks]);
     }
   }
+  f32x4 o[DT][2];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt][0] = o[dt][1] = f32x4{};
+  float m_run[2] = {neg_inf(), neg_inf()}, l_run[2] = {0.f, 0.f};
 
-  const float l = sum_xor32(l_run);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (qrow < a.Nq) {
+  // two steps per listed block; a last block of at most 64 keys is one
+  int steps = 2 * cnt;
+  if (cnt > 0 && list[cnt - 1] * 128 + 64 >= a.Nk) --steps;
+  auto key_of = [&](int t) { return list[t >> 1] * 128 + (t & 1) * 64; };
+  int key0 = steps > 0 ? key_of(0) : 0;
+  int key0_next = steps > 1 ? key_of(1) : 0;
+  const float* ksrc = kbase + (int64_t)(tid / (D / 8)) * a.ks[2] + tid % (D / 8) * 8;
+  const float* vsrc = vbase + (int64_t)(tid / (D / 8)) * a.vs[2] + tid % (D / 8) * 8;
+  if (steps > 0) {
+    F32Part<D> x0, x1;
+    x0.template load<0>(ksrc + (int64_t)key0 * a.ks[2], a.ks[2], a.Nk - key0, tid);
+    x1.template load<1>(ksrc + (int64_t)key0 * a.ks[2], a.ks[2], a.Nk - key0, tid);
+    x0.template write<0, false>(kh, kl, tid);
+    x1.template write<1, false>(kh, kl, tid);
+  }
+  __syncthreads();
+  for (int t = 0; t < steps; ++t) {
+    const bool next = t + 1 < steps;
+    const int key0_after = t + 2 < steps ? key_of(t + 2) : 0;  // read a step before it is needed
+    F32Part<D> x;
+    x.template load<0>(vsrc + (int64_t)key0 * a.vs[2], a.vs[2], a.Nk - key0, tid);
+
+    f32x4 s[4][2];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) s[kt][0] = s[kt][1] = f32x4{};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const u32x4 ah = *(SA_LDS const u32x4*)(kh + L.ka[ks] + kt * (32 * D));
+        const u32x4 al = *(SA_LDS const u32x4*)(kl + L.ka[ks] + kt * (32 * D));
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) s[kt][qt] = mfma16x16x32<kBF16>(ah, qh[qt][ks], s[kt][qt]);
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) s[kt][qt] = mfma16x16x32<kBF16>(ah, ql[qt][ks], s[kt][qt]);
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) s[kt][qt] = mfma16x16x32<kBF16>(al, qh[qt][ks], s[kt][qt]);
+      }
+    x.template write<0, true>(vh, vl, tid);
+    x.template load<1>(vsrc + (int64_t)key0 * a.vs[2], a.vs[2], a.Nk - key0, tid);
+    if (key0 + 64 > a.Nk) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (key0 + 16 * kt + 4 * g + i >= a.Nk) s[kt][0][i] = s[kt][1][i] = neg_inf();
+    }
+    u32x4 ph[2][2], pl[2][2];  // [k-step of 32 keys][query tile]
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      float mx = neg_inf();
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][qt][i]);
+      const float m_tile = max_col16(mx) * c;
+      // The reference point follows the maximum at once: the largest P is then 1, which splits
+      // without error (a reference 8 log2 units behind, as in 16 bits, raised the output's error
+      // by 1.7%).
+      if (m_tile > m_run[qt]) {
+        const float alpha = fast_exp2(m_run[qt] - m_tile);
+        l_run[qt] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt][qt] *= alpha;
+        m_run[qt] = m_tile;
+      }
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const float v0 = fast_exp2(__builtin_fmaf(s[2 * kc + u][qt][2 * e], c, -m_run[qt]));
+            const float v1 = fast_exp2(__builtin_fmaf(s[2 * kc + u][qt][2 * e + 1], c, -m_run[qt]));
+            l_run[qt] += v0 + v1;
+            uint32_t hv, lv;
+            split_pair(v0, v1, hv, lv);
+            ph[kc][qt][2 * u + e] = hv;
+            pl[kc][qt][2 * u + e] = lv;
+          }
+    }
+    x.template write<1, true>(vh, vl, tid);
+    __syncthreads();  // V has landed, every wave is done with K
+
+    const float* knext = ksrc + (int64_t)key0_next * a.ks[2];
+    const int krows = next ? a.Nk - key0_next : 0;
+    x.template load<0>(knext, a.ks[2], krows, tid);
+    if (D == 128) __builtin_amdgcn_s_setprio(1);  // 2% faster at D = 128, 2% slower at 64
+    auto vread = [&](SA_LDS char* v, int kc, int dt) -> u32x4 {
+      SA_LDS char* at = v + L.va[dt] + kc * (64 * D);
+      const u32x2 y0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)at));
+      const u32x2 y1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)(at + 32 * D)));
+      return u32x4{y0[0], y0[1], y1[0], y1[1]};
+    };
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      if (kc == 1) {
+        x.template write<0, false>(kh, kl, tid);
+        x.template load<1>(knext, a.ks[2], krows, tid);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const u32x4 ah = vread(vh, kc, dt), al = vread(vl, kc, dt);
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) o[dt][qt] = mfma16x16x32<kBF16>(ah, ph[kc][qt], o[dt][qt]);
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) o[dt][qt] = mfma16x16x32<kBF16>(ah, pl[kc][qt], o[dt][qt]);
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) o[dt][qt] = mfma16x16x32<kBF16>(al, ph[kc][qt], o[dt][qt]);
+      }
+    }
+    if (D == 128) __builtin_amdgcn_s_setprio(0);
+    x.template write<1, false>(kh, kl, tid);
+    __syncthreads();  // the next K has landed, every wave is done with V
+    key0 = key0_next;
+    key0_next = key0_after;
+  }
+
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    const float l = sum_col16(l_run[qt]);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int qrow = qb * 128 + wave * 32 + 16 * qt + sl;
+    if (qrow >= a.Nq) continue;
     float* obase = (float*)a.out + ((int64_t)b * a.os[0] + (int64_t)h * a.os[1] + (int64_t)qrow * a.os[2]);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = dt * 32 + 8 * g + 4 * hl;
-        store4<kF32>(obase + d, o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv,
-                     o[dt][4 * g + 3] * inv);
-      }
-    if (a.lse != nullptr && hl == 0)
-      a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] = cnt > 0 ? (m_run + __log2f(l)) * kLn2 : pos_inf();
+      store4<kF32>(obase + 16 * dt + 4 * g, o[dt][qt][0] * inv, o[dt][qt][1] * inv, o[dt][qt][2] * inv,
+                   o[dt][qt][3] * inv);
+    if (a.lse != nullptr && g == 0)
+      a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] = cnt > 0 ? (m_run[qt] + __log2f(l)) * kLn2 : pos_inf();
   }
 }
 

@@ -239,6 +239,26 @@ def test_small_head_dims_edges_and_key_strides(dtype, D, Nq, Nk, layout):
     _check(oe, le, q, ke, ve, mask)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Nq,Nk,layout", [(1, 1, "bhsd"), (31, 65, "bshd"), (130, 64, "bhsd"), (257, 1000, "bshd"),
+                                          (900, 577, "bhsd")])
+def test_f32_steps_edges(D, Nq, Nk, layout):
+    """fp32 operands in steps of 64 keys: last blocks of one and of two steps, ragged rows, a broadcast
+    key dim.  Operands split into bf16 pairs keep 16 mantissa bits (2^-17 relative), so a logit
+    is within 3 * 2^-17 * |q||k| / sqrt(D) <= 3 * 2^-17 * 2 sqrt(D) of its exact value and the
+    output, an average of |v| <= 5, within 2.6e-3; 2e-4 is what random rounding leaves of it."""
+    q, k, v = _inputs(1, 3, Nq, Nk, D, torch.float32, seed=Nq + Nk, layout=layout)
+    mask = _random_mask(1, 3, -(-Nq // 128), -(-Nk // 128), 0.5, seed=5, empty_rows=1 if Nq > 128 else 0)
+    plan = ops.block_sparse_plan(mask)
+    for kk, vv in ((k, v), (k[:, :, :1].expand(-1, -1, Nk, -1), v[:, :, :1].expand(-1, -1, Nk, -1))):
+        out, lse = ops.block_sparse_attention(q, kk, vv, plan)
+        _check(out, lse, q, kk, vv, mask)
+        ref_o, ref_l = torch_ref.dense_masked_attention(q, kk, vv, mask)
+        fin = torch.isfinite(ref_l)
+        assert (out.cpu() - ref_o).abs().max() <= 2e-4
+        assert (lse.cpu() - ref_l)[fin].abs().max() <= 1e-4
+
+
 def _chunk_layout(nbh, nqb):
     """Chunking of the launch order: heads [0, nbh_w) in Cw chunks (qb mod Cw), the heads
     of the partial last round of 8 in Cs = Cw * F finer chunks."""
