@@ -146,6 +146,36 @@ int sinkattn_block_sparse_fwd_comp(const void* q, const void* k, const void* v, 
                                    float softmax_scale, void* stream);
 
 /* ------------------------------------------------------------------------------------
+ * Dense attention forward.
+ *
+ * Replaces the dense `scaled_dot_product_attention` of the calibration processor and of the
+ * forced-dense steps (wanx/runtime/sink_sparse_wan.py:389-429;
+ * zimg/runtime/sink_sparse_zimage.py:420-614): sinkattn_block_sparse_fwd with every key block
+ * listed, without a plan.  bf16/f16, D = 128, Nk >= 1; lse (fp32 [B,H,Nq], or NULL) as there.
+ * ---------------------------------------------------------------------------------- */
+int sinkattn_dense_fwd(const void* q, const void* k, const void* v, int dtype,
+                       int64_t B, int64_t H, int64_t Nq, int64_t Nk, int64_t D,
+                       const int64_t q_strides[4], const int64_t k_strides[4],
+                       const int64_t v_strides[4], void* out, const int64_t out_strides[4],
+                       float* lse, float softmax_scale, void* stream);
+
+/* ------------------------------------------------------------------------------------
+ * Dense attention and its exact block-mass map in one pass.
+ *
+ * Replaces, for a calibration call, `_compute_exact_block_mass_scores` at block size 128 and
+ * the dense attention that follows it (sinkattention/sparse_attention.py:145-227;
+ * wanx/runtime/sink_sparse_wan.py:389-429): out as sinkattn_dense_fwd, mass fp32
+ * [B,H,nqb,nkb] as sinkattn_block_mass_pool.  workspace: the query's bytes (at most 2 GiB, or
+ * one head's sums if those are more; 512 bytes per pair of blocks).
+ * ---------------------------------------------------------------------------------- */
+size_t sinkattn_dense_mass_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk);
+int sinkattn_dense_mass(const void* q, const void* k, const void* v, int dtype,
+                        int64_t B, int64_t H, int64_t Nq, int64_t Nk, int64_t D,
+                        const int64_t q_strides[4], const int64_t k_strides[4],
+                        const int64_t v_strides[4], void* out, const int64_t out_strides[4],
+                        float* mass, void* workspace, float softmax_scale, void* stream);
+
+/* ------------------------------------------------------------------------------------
  * Token mean pooling of the compensation branch.
  *
  * Replaces `_mean_pool_sequence_preserve_prefix` / `_mean_pool_sequence` /

@@ -49,6 +49,17 @@ SIGNATURES = {
          _c_i64_4, _c_i64_4, _c_i64_4, _c_p, _c_p, _c_i64_4, _c_i64_4, _c_i64, _c_i64, ctypes.c_float,
          _c_p, _c_i64_4, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, ctypes.c_float, _c_p],
     ),
+    "sinkattn_dense_fwd": (
+        ctypes.c_int,
+        [_c_p, _c_p, _c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+         _c_i64_4, _c_i64_4, _c_i64_4, _c_p, _c_i64_4, _c_p, ctypes.c_float, _c_p],
+    ),
+    "sinkattn_dense_mass_workspace_bytes": (ctypes.c_size_t, [_c_i64, _c_i64, _c_i64, _c_i64]),
+    "sinkattn_dense_mass": (
+        ctypes.c_int,
+        [_c_p, _c_p, _c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+         _c_i64_4, _c_i64_4, _c_i64_4, _c_p, _c_i64_4, _c_p, _c_p, ctypes.c_float, _c_p],
+    ),
     "sinkattn_mean_pool_tokens_rows": (ctypes.c_int64, [_c_i64, _c_i64, _c_i64]),
     "sinkattn_mean_pool_tokens": (
         ctypes.c_int,

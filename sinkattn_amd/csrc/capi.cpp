@@ -246,6 +246,80 @@ int sinkattn_block_sparse_fwd_comp(const void* q, const void* k, const void* v, 
                                out_strides, lse, counts, idx, order, nqb, nkb, softmax_scale, comp, stream);
 }
 
+static int fill_dense_args(sa::FwdArgs& a, const char* who, const void* q, const void* k, const void* v,
+                           int dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int64_t D,
+                           const int64_t* qs, const int64_t* ks, const int64_t* vs, void* out, const int64_t* os) {
+  if (dtype != SINKATTN_BF16 && dtype != SINKATTN_F16) return fail("%s: unsupported dtype %d (bf16 or f16)", who, dtype);
+  if (D != 128) return fail("%s: head dim %lld not supported (128)", who, (long long)D);
+  if (B < 0 || H < 0 || Nq < 0 || Nk < 1) return fail("%s: bad size", who);
+  const int64_t nqb = cdiv(Nq, 128), nkb = cdiv(Nk, 128);
+  if (B * H * nqb > kMaxInt - 8 || Nq > kMaxInt || Nk > kMaxInt) return fail("%s: sizes exceed int32", who);
+  if (B * H * nqb > 0) {
+    int rc;
+    if ((rc = check_operand("q", q, qs)) != 0) return rc;
+    if ((rc = check_operand("k", k, ks)) != 0) return rc;
+    if ((rc = check_operand("v", v, vs)) != 0) return rc;
+    if ((rc = check_operand("out", out, os)) != 0) return rc;
+    if (ks[2] < D || vs[2] < D) return fail("%s: k/v row stride below the head dim", who);
+    if (Nk * ks[2] * 2 >= (int64_t)1 << 31 || Nk * vs[2] * 2 >= (int64_t)1 << 31)
+      return fail("%s: one head of k or v spans more than 2 GiB", who);
+    for (int i = 0; i < 4; ++i) {
+      a.qs[i] = qs[i];
+      a.ks[i] = ks[i];
+      a.vs[i] = vs[i];
+      a.os[i] = os[i];
+    }
+  }
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.out = out;
+  a.B = (int)B;
+  a.H = (int)H;
+  a.Nq = (int)Nq;
+  a.Nk = (int)Nk;
+  a.nqb = (int)nqb;
+  a.nkb = (int)nkb;
+  return 0;
+}
+
+int sinkattn_dense_fwd(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t H,
+                       int64_t Nq, int64_t Nk, int64_t D, const int64_t q_strides[4],
+                       const int64_t k_strides[4], const int64_t v_strides[4], void* out,
+                       const int64_t out_strides[4], float* lse, float softmax_scale, void* stream) {
+  sa::FwdArgs a{};
+  const int rc = fill_dense_args(a, "dense_fwd", q, k, v, dtype, B, H, Nq, Nk, D, q_strides, k_strides, v_strides,
+                                 out, out_strides);
+  if (rc != 0) return rc;
+  a.lse = lse;
+  a.scale = softmax_scale;
+  return hip_status(sa::launch_dense_fwd(a, dtype, (hipStream_t)stream), "dense_fwd launch");
+}
+
+size_t sinkattn_dense_mass_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk) {
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0) return 0;
+  const int64_t nqb = cdiv(Nq, 128), nkb = cdiv(Nk, 128);
+  return (size_t)(sa::dense_mass_heads(B * H, nqb, nkb) * nqb * nkb * 512);
+}
+
+int sinkattn_dense_mass(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t H,
+                        int64_t Nq, int64_t Nk, int64_t D, const int64_t q_strides[4],
+                        const int64_t k_strides[4], const int64_t v_strides[4], void* out,
+                        const int64_t out_strides[4], float* mass, void* workspace, float softmax_scale,
+                        void* stream) {
+  sa::FwdArgs a{};
+  const int rc = fill_dense_args(a, "dense_mass", q, k, v, dtype, B, H, Nq, Nk, D, q_strides, k_strides, v_strides,
+                                 out, out_strides);
+  if (rc != 0) return rc;
+  if (cdiv(Nk, 128) > (1 << 22)) return fail("dense_mass: too many key blocks");
+  if (B * H * Nq == 0) return 0;
+  if (mass == nullptr || workspace == nullptr) return fail("dense_mass: null map or workspace");
+  a.scale = softmax_scale;
+  a.mass = mass;
+  a.mass_ws = reinterpret_cast<float*>(workspace);
+  return hip_status(sa::launch_dense_mass(a, dtype, (hipStream_t)stream), "dense_mass launch");
+}
+
 int64_t sinkattn_mean_pool_tokens_rows(int64_t N, int64_t prefix, int64_t gap) {
   if (N < 0 || gap < 1) return -1;
   if (gap == 1) return N;

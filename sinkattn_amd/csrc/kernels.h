@@ -39,6 +39,11 @@ struct FwdArgs {
   int64_t kds[2], vds[2];
   int Nd, comp_qblocks;
   float comp_bias;
+  // Dense forms: heads [bh0, bh0 + nbh) of the launch; the block-mass map [B,H,nqb,nkb] and
+  // the workspace of its row sums, [heads of a launch][nqb][nkb][128].
+  int bh0, nbh;
+  float* mass;
+  float* mass_ws;
 };
 
 struct PoolArgs {
@@ -111,6 +116,9 @@ int plan_order_slots(int rows, int nqb);
 int64_t plan_order_cache_ints(int rows, int nqb, int entries);
 hipError_t launch_block_sparse_plan(const PlanArgs& a, hipStream_t stream);
 hipError_t launch_block_sparse_fwd(const FwdArgs& a, int dtype, int D, hipStream_t stream);
+hipError_t launch_dense_fwd(const FwdArgs& a, int dtype, hipStream_t stream);
+int64_t dense_mass_heads(int64_t nbh, int64_t nqb, int64_t nkb);
+hipError_t launch_dense_mass(const FwdArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
 bool pool_f32_mfma(const PoolArgs& a);
 int block_mass_groups();

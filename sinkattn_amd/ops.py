@@ -211,6 +211,69 @@ def block_sparse_attention(
     return out, lse
 
 
+def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: Optional[float] = None,
+                    return_lse: bool = False) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """softmax(Q K^T * scale) V over every key, bf16/f16 [B, H, N, 128] views on the GPU.  Returns
+    out as a [B, H, Nq, D] view of [B, Nq, H, D] memory and lse as fp32 [B, H, Nq] (or None)."""
+    _require_cuda("dense_attention", q, k, v)
+    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+        raise ValueError("q, k, v must be [B, H, N, D]")
+    B, H, Nq, D = (int(x) for x in q.shape)
+    Nk = int(k.shape[2])
+    if tuple(k.shape) != (B, H, Nk, D) or tuple(v.shape) != (B, H, Nk, D):
+        raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match q {tuple(q.shape)}")
+    if not (q.dtype == k.dtype == v.dtype):
+        raise TypeError("q, k, v must share a dtype")
+    if softmax_scale is None:
+        softmax_scale = 1.0 / math.sqrt(D)
+    qk, kk, vk = _kernel_operand(q), _kernel_operand(k), _kernel_operand(v)
+    out = torch.empty((B, Nq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    lse = torch.empty((B, H, Nq), dtype=torch.float32, device=q.device) if return_lse else None
+    L = _lib.lib()
+    with torch.cuda.device(q.device):
+        _lib.check(
+            L.sinkattn_dense_fwd(
+                qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), _lib.dtype_code(q.dtype), B, H, Nq, Nk, D,
+                _lib.strides4(qk), _lib.strides4(kk), _lib.strides4(vk), out.data_ptr(), _lib.strides4(out),
+                _lib.ptr(lse), float(softmax_scale), _lib.stream_ptr(q.device),
+            ),
+            "dense_fwd",
+        )
+    return out, lse
+
+
+def dense_attention_mass(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                         softmax_scale: Optional[float] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """dense_attention's output and block_mass_scores' fp32 map [B, H, nqb, nkb] (blocks of 128)
+    from one pass over the scores, for at least one key."""
+    _require_cuda("dense_attention_mass", q, k, v)
+    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+        raise ValueError("q, k, v must be [B, H, N, D]")
+    B, H, Nq, D = (int(x) for x in q.shape)
+    Nk = int(k.shape[2])
+    if tuple(k.shape) != (B, H, Nk, D) or tuple(v.shape) != (B, H, Nk, D):
+        raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match q {tuple(q.shape)}")
+    if not (q.dtype == k.dtype == v.dtype):
+        raise TypeError("q, k, v must share a dtype")
+    if softmax_scale is None:
+        softmax_scale = 1.0 / math.sqrt(D)
+    qk, kk, vk = _kernel_operand(q), _kernel_operand(k), _kernel_operand(v)
+    out = torch.empty((B, Nq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    mass = torch.empty((B, H, _cdiv(Nq, KERNEL_BLOCK), _cdiv(Nk, KERNEL_BLOCK)), dtype=torch.float32, device=q.device)
+    L = _lib.lib()
+    ws = torch.empty(int(L.sinkattn_dense_mass_workspace_bytes(B, H, Nq, Nk)) // 4, dtype=torch.float32, device=q.device)
+    with torch.cuda.device(q.device):
+        _lib.check(
+            L.sinkattn_dense_mass(
+                qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), _lib.dtype_code(q.dtype), B, H, Nq, Nk, D,
+                _lib.strides4(qk), _lib.strides4(kk), _lib.strides4(vk), out.data_ptr(), _lib.strides4(out),
+                mass.data_ptr(), _lib.ptr(ws), float(softmax_scale), _lib.stream_ptr(q.device),
+            ),
+            "dense_mass",
+        )
+    return out, mass
+
+
 def _empty_like_layout(t: torch.Tensor, rows: int) -> torch.Tensor:
     """Uninitialised [B, H, rows, D] tensor whose dims are laid out in memory in the same
     order as t's (so a [B, N, H, D]-memory view gets a [B, rows, H, D]-memory result and

@@ -39,6 +39,7 @@ from .sparse_attention import (
     _make_full_block_mask,
     _mean_pool_sequence_preserve_prefix,
     _mix_attention_outputs,
+    _record_and_attend,
     load_sink_mask_package,
 )
 
@@ -400,9 +401,8 @@ class WanSinkCalibrationProcessor2_0:
                  attention_mask: Optional[torch.Tensor] = None, rotary_emb=None) -> torch.Tensor:
         del attention_mask
         q, k, v, img_ctx = _prepare_attention_tensors(attn, hidden_states, encoder_hidden_states, rotary_emb)
-        self.calibrator.record(self.layer_idx, q, k, v)
+        out = _record_and_attend(self.calibrator, self.layer_idx, q, k, v)
         img = _compute_image_branch(attn, q, img_ctx)
-        out = F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False)
         out = out.transpose(1, 2).flatten(2, 3).type_as(q)
         if img is not None:
             out = out + img

@@ -19,7 +19,6 @@ from pathlib import Path
 from typing import Any, Dict, Optional
 
 import torch
-import torch.nn.functional as F
 
 from . import ops
 from .sparse_attention import (
@@ -32,6 +31,7 @@ from .sparse_attention import (
     _device_package_groups,
     _ceil_div,
     _compute_block_scores,
+    _dense_attention,
     _dense_short_attention_with_lse,
     _device_cache_key,
     _fused_compensation_supported,
@@ -198,10 +198,6 @@ def _force_text_dense_runtime_mask(runtime_mask: torch.Tensor, *, image_blocks: 
     out[..., :, int(image_blocks):] = True
     out[..., int(image_blocks):, :] = True
     return out
-
-
-def _dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-    return F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False)
 
 
 # -- the model's own ops in front of the hot path ------------------------------------------

@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from oracle import torch_ref
-from sinkattn_amd import ops
+from sinkattn_amd import _lib, ops
 from sinkattn_amd import sparse_attention as sa
 
 pytestmark = pytest.mark.gpu
@@ -257,6 +257,55 @@ def test_f32_steps_edges(D, Nq, Nk, layout):
         fin = torch.isfinite(ref_l)
         assert (out.cpu() - ref_o).abs().max() <= 2e-4
         assert (lse.cpu() - ref_l)[fin].abs().max() <= 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Nq,Nk,layout", [(1, 1, "bhsd"), (130, 129, "bshd"), (700, 1500, "bhsd"), (1029, 640, "bshd")])
+def test_dense_forms(dtype, Nq, Nk, layout):
+    """The plan-free dense kernel and the one that also returns the block-mass map: attention bars
+    against the oracle, fp32 row sums (lse to 1e-4 + 1e-5 |lse|), the map at the pooling bar."""
+    q, k, v = _inputs(2, 3, Nq, Nk, 128, dtype, seed=Nq + Nk, sink_keys=2, layout=layout)
+    full = torch.ones(2, 3, -(-Nq // 128), -(-Nk // 128), dtype=torch.bool)
+    out, lse = ops.dense_attention(q, k, v, return_lse=True)
+    _check(out, lse, q, k, v, full.cuda())
+    ref_l = torch_ref.dense_masked_attention(q, k, v, full)[1]
+    assert ((lse.cpu() - ref_l).abs() <= 1e-4 + 1e-5 * ref_l.abs()).all()
+    o2, mass = ops.dense_attention_mass(q, k, v)
+    _check(o2, lse, q, k, v, full.cuda())
+    ref = torch_ref.exact_block_mass(q, k)
+    assert mass.shape == ref.shape and ((mass.cpu() - ref).abs() <= 1e-8 + 1e-5 * ref.abs()).all()
+
+
+def test_dense_mass_reference_moves():
+    # rising maxima, and first keys ~80 log2 units below the later ones: the row sums' unit
+    # moves past its 2^64 limit and the earlier sums are rescaled
+    g = torch.Generator().manual_seed(4)
+    q = 0.5 + 0.1 * torch.randn(1, 2, 400, 128, generator=g)
+    k = torch.randn(1, 2, 1500, 128, generator=g)
+    k[:, :, :128] = -10.0
+    k[:, :, 1200:] *= 3.0
+    qq, kk = q.bfloat16().cuda(), k.bfloat16().cuda()
+    out, mass = ops.dense_attention_mass(qq, kk, kk)
+    ref = torch_ref.exact_block_mass(qq, kk)
+    assert ((mass.cpu() - ref).abs() <= 1e-8 + 1e-5 * ref.abs()).all()
+    _check(out, ops.dense_attention(qq, kk, kk, return_lse=True)[1], qq, kk, kk,
+           torch.ones(1, 2, 4, 12, dtype=torch.bool).cuda())
+
+
+def test_dense_mass_in_several_launches():
+    # more heads than one launch's workspace holds (2 GiB of row sums): the heads at the seam
+    # against the pooling kernel's own map
+    B, H, N = 1, 13, 75600
+    assert _lib.lib().sinkattn_dense_mass_workspace_bytes(B, H, N, N) < H * 591 * 591 * 512
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn(B, N, H, 128, device="cuda", dtype=torch.bfloat16, generator=g).transpose(1, 2)
+               for _ in range(3))
+    out, mass = ops.dense_attention_mass(q, k, v)
+    for h in (0, 10, 11, 12):
+        want = ops.block_mass_scores(q[:, h:h + 1], k[:, h:h + 1])
+        assert ((mass[:, h:h + 1] - want).abs() <= 1e-8 + 1e-5 * want.abs()).all()
+        assert torch.equal(out[:, h:h + 1, :256], ops.dense_attention_mass(q[:, h:h + 1, :256], k[:, h:h + 1],
+                                                                           v[:, h:h + 1])[0])
 
 
 def _chunk_layout(nbh, nqb):

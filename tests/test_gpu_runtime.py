@@ -289,3 +289,29 @@ def test_zimage_calibrator_vs_oracle():
     want_mask = torch_ref.coverage_mask(got, coverage=0.85, keep_diagonal=True, block_size=128, text_length=256,
                                         force_text=True)
     assert torch.equal(pkg["sink_masks"]["0"].cpu(), want_mask)
+
+
+@pytest.mark.parametrize("N,mode", [(1500, "exact"), (1500, "triton"), (600, "exact")])
+def test_wan_calibration_processor_dense_attention(N, mode):
+    """The calibration processor against the oracle's dense attention and its calibrator against
+    a plain `record` of the same Q/K/V, where the map and the attention share one kernel (exact
+    mode from 1024 keys) and where they do not; gradients keep the torch path."""
+    torch.manual_seed(5)
+    H, D = 2, 128
+    attn = _WanAttn(H * D, H).to(DEV, torch.bfloat16)
+    attn.to_out[0] = nn.Identity()
+    x = torch.randn(2, N, H * D, device=DEV, dtype=torch.bfloat16)
+    cfg = SinkSparseConfig(pooling_mode=mode)
+    cal, ref = wr.SinkMaskCalibrator(cfg), wr.SinkMaskCalibrator(cfg)
+    with torch.no_grad():
+        out = wr.WanSinkCalibrationProcessor2_0(cal, 0)(attn, x)
+        q, k, v, _ = wr._prepare_attention_tensors(attn, x)
+        ref.record(0, q, k, v)
+    full = torch.ones(2, H, -(-N // 128), -(-N // 128), dtype=torch.bool)
+    want = torch_ref.dense_masked_attention(q, k, v, full)[0]
+    _check(out, want.transpose(1, 2).flatten(2, 3), 2e-2, 1e-3, f"calibration attention {mode} {N}")
+    assert cal.current_step == 0 and cal.score_counts == ref.score_counts
+    assert torch.allclose(cal.score_sums[0], ref.score_sums[0], rtol=1e-5, atol=1e-8)
+    xg = x.clone().requires_grad_()
+    wr.WanSinkCalibrationProcessor2_0(cal, 0)(attn, xg).float().sum().backward()
+    assert xg.grad is not None and bool(xg.grad.abs().sum() > 0)
