@@ -191,6 +191,14 @@ int sinkattn_mean_pool_tokens(const void* x, int dtype, int64_t B, int64_t H, in
                               int64_t D, const int64_t x_strides[4], int64_t prefix,
                               int64_t gap, void* out, const int64_t out_strides[4],
                               void* stream);
+/* K and V of one call in one launch, and rows [pool_end, N) kept after the pooled ones (the
+ * text suffix of the joint sequence, zimg/runtime/sink_sparse_zimage.py:553-592): prefix +
+ * ceil((pool_end - prefix) / gap) + N - pool_end rows each. */
+int sinkattn_mean_pool_kv(const void* k, const void* v, int dtype, int64_t B, int64_t H, int64_t N,
+                          int64_t D, const int64_t k_strides[4], const int64_t v_strides[4],
+                          int64_t prefix, int64_t pool_end, int64_t gap, void* k_out, void* v_out,
+                          const int64_t k_out_strides[4], const int64_t v_out_strides[4],
+                          void* stream);
 
 /* ------------------------------------------------------------------------------------
  * QK-norm + rotary embedding of Q and K in one pass.

@@ -65,6 +65,11 @@ SIGNATURES = {
         ctypes.c_int,
         [_c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64_4, _c_i64, _c_i64, _c_p, _c_i64_4, _c_p],
     ),
+    "sinkattn_mean_pool_kv": (
+        ctypes.c_int,
+        [_c_p, _c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64_4, _c_i64_4, _c_i64, _c_i64, _c_i64,
+         _c_p, _c_p, _c_i64_4, _c_i64_4, _c_p],
+    ),
     "sinkattn_qk_norm_rotary": (
         ctypes.c_int,
         [_c_p, _c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, ctypes.c_float, ctypes.c_float,

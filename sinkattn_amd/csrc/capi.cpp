@@ -328,37 +328,69 @@ int64_t sinkattn_mean_pool_tokens_rows(int64_t N, int64_t prefix, int64_t gap) {
   return p + cdiv(N - p, gap);
 }
 
-int sinkattn_mean_pool_tokens(const void* x, int dtype, int64_t B, int64_t H, int64_t N, int64_t D,
-                              const int64_t x_strides[4], int64_t prefix, int64_t gap, void* out,
-                              const int64_t out_strides[4], void* stream) {
-  if (!valid_dtype(dtype)) return fail("mean_pool_tokens: unsupported dtype %d", dtype);
-  if (B < 0 || H < 0 || N < 0 || gap < 1) return fail("mean_pool_tokens: bad size or gap");
+static int mean_pool_impl(const char* who, sa::TokenPoolArgs& a, int dtype, int64_t B, int64_t H, int64_t N,
+                          int64_t D, int64_t prefix, int64_t pool_end, int64_t gap, void* stream) {
+  if (!valid_dtype(dtype)) return fail("%s: unsupported dtype %d", who, dtype);
+  if (B < 0 || H < 0 || N < 0 || gap < 1) return fail("%s: bad size or gap", who);
   const int64_t es = dtype == SINKATTN_F32 ? 4 : 2;
   const int64_t chunks = D * es / 16;
   if (D <= 0 || (D * es) % 16 != 0 || chunks > 256 || (chunks & (chunks - 1)) != 0)
-    return fail("mean_pool_tokens: head dim %lld unsupported (row of 16..4096 bytes, power of two)", (long long)D);
-  const int64_t nout = sinkattn_mean_pool_tokens_rows(N, prefix, gap);
-  if (B * H > 65535 || N > kMaxInt) return fail("mean_pool_tokens: sizes exceed the launch limits");
+    return fail("%s: head dim %lld unsupported (row of 16..4096 bytes, power of two)", who, (long long)D);
+  const int64_t end = pool_end < 0 ? 0 : (pool_end > N ? N : pool_end);
+  int64_t p = prefix < 0 ? 0 : (prefix > end ? end : prefix);
+  if (gap == 1) p = end;  // every row is kept
+  const int64_t nout = p + cdiv(end - p, gap) + (N - end);
+  if (B * H > 65535 || N > kMaxInt || gap > kMaxInt) return fail("%s: sizes exceed the launch limits", who);
   if (B * H * nout == 0) return 0;
-  int rc;
-  if ((rc = check_operand("x", x, x_strides)) != 0) return rc;
-  if ((rc = check_operand("out", out, out_strides)) != 0) return rc;
-  sa::TokenPoolArgs a{};
-  a.x = x;
-  a.out = out;
-  for (int i = 0; i < 4; ++i) {
-    a.xs[i] = x_strides[i];
-    a.os[i] = out_strides[i];
+  for (int z = 0; z < a.tensors; ++z) {
+    int rc;
+    if ((rc = check_operand("x", a.x[z], a.xs[z])) != 0) return rc;
+    if ((rc = check_operand("out", a.out[z], a.os[z])) != 0) return rc;
   }
   a.B = (int)B;
   a.H = (int)H;
   a.N = (int)N;
   a.D = (int)D;
   a.Nout = (int)nout;
-  a.gap = gap == 1 ? 1 : (int)gap;
-  const int64_t p = prefix < 0 ? 0 : (prefix > N ? N : prefix);
-  a.prefix = (gap == 1 || p >= N) ? (int)N : (int)p;  // identity cases copy every row
-  return hip_status(sa::launch_mean_pool_tokens(a, dtype, (hipStream_t)stream), "mean_pool_tokens launch");
+  a.gap = (int)gap;
+  a.prefix = (int)p;
+  a.pool_end = (int)end;
+  return hip_status(sa::launch_mean_pool_tokens(a, dtype, (hipStream_t)stream), who);
+}
+
+int sinkattn_mean_pool_tokens(const void* x, int dtype, int64_t B, int64_t H, int64_t N, int64_t D,
+                              const int64_t x_strides[4], int64_t prefix, int64_t gap, void* out,
+                              const int64_t out_strides[4], void* stream) {
+  sa::TokenPoolArgs a{};
+  a.tensors = 1;
+  a.x[0] = x;
+  a.out[0] = out;
+  for (int i = 0; i < 4; ++i) {
+    a.xs[0][i] = x_strides != nullptr ? x_strides[i] : 0;
+    a.os[0][i] = out_strides != nullptr ? out_strides[i] : 0;
+  }
+  return mean_pool_impl("mean_pool_tokens", a, dtype, B, H, N, D, prefix, N, gap, stream);
+}
+
+int sinkattn_mean_pool_kv(const void* k, const void* v, int dtype, int64_t B, int64_t H, int64_t N, int64_t D,
+                          const int64_t k_strides[4], const int64_t v_strides[4], int64_t prefix,
+                          int64_t pool_end, int64_t gap, void* k_out, void* v_out,
+                          const int64_t k_out_strides[4], const int64_t v_out_strides[4], void* stream) {
+  if (k_strides == nullptr || v_strides == nullptr || k_out_strides == nullptr || v_out_strides == nullptr)
+    return fail("mean_pool_kv: null strides");
+  sa::TokenPoolArgs a{};
+  a.tensors = 2;
+  a.x[0] = k;
+  a.x[1] = v;
+  a.out[0] = k_out;
+  a.out[1] = v_out;
+  for (int i = 0; i < 4; ++i) {
+    a.xs[0][i] = k_strides[i];
+    a.xs[1][i] = v_strides[i];
+    a.os[0][i] = k_out_strides[i];
+    a.os[1][i] = v_out_strides[i];
+  }
+  return mean_pool_impl("mean_pool_kv", a, dtype, B, H, N, D, prefix, pool_end, gap, stream);
 }
 
 int sinkattn_qk_norm_rotary(const void* q_in, const void* k_in, int dtype, int64_t rows, int64_t C,

@@ -72,14 +72,15 @@ struct MaskArgs {
   uint8_t* ws_flags;  // [H*nq] workspace (empty-row and top-tie flags), padded to 256 B
 };
 
-// Token mean pooling: rows [0, prefix) copied, then groups of `gap` rows averaged
-// (a short last group repeats row N-1).  x [B,H,N,D] -> out [B,H,Nout,D].
+// Token mean pooling of `tensors` (1 or 2) tensors x [B,H,N,D] -> out [B,H,Nout,D]: rows
+// [0, prefix) copied, rows [prefix, pool_end) averaged in groups of `gap` (a short last group
+// repeats row pool_end-1), rows [pool_end, N) copied.
 struct TokenPoolArgs {
-  const void* x;
-  int64_t xs[4];
-  void* out;
-  int64_t os[4];
-  int B, H, N, D, Nout, prefix, gap;
+  const void* x[2];
+  int64_t xs[2][4];
+  void* out[2];
+  int64_t os[2][4];
+  int B, H, N, D, Nout, prefix, pool_end, gap, tensors;
 };
 
 // out = a*sink + (1-a)*dyn with a = sigmoid(lse_s - lse_d - log_gap), per-op rounding.

@@ -314,6 +314,36 @@ def mean_pool_tokens(x: torch.Tensor, gap: int, prefix: int = 0,
     return out
 
 
+def mean_pool_kv(k: torch.Tensor, v: torch.Tensor, gap: int, prefix: int = 0,
+                 pool_end: Optional[int] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """mean_pool_tokens of K and V [B, H, N, D] in one launch, with rows from `pool_end` (default
+    N) on kept after the pooled ones.  Each result has its input's memory layout."""
+    _require_cuda("mean_pool_kv", k, v)
+    if k.dim() != 4 or k.shape != v.shape or k.dtype != v.dtype:
+        raise ValueError(f"mean_pool_kv: k and v must be [B, H, N, D] of one shape and dtype, got {tuple(k.shape)} "
+                         f"and {tuple(v.shape)}")
+    B, H, N, D = (int(s) for s in k.shape)
+    gap, end = int(gap), N if pool_end is None else min(max(int(pool_end), 0), N)
+    if gap < 1:
+        raise ValueError(f"mean_pool_kv: bad gap {gap}")
+    first = min(max(int(prefix), 0), end)
+    rows = first + _cdiv(end - first, gap) + N - end
+    kk, vk = _kernel_operand(k), _kernel_operand(v)
+    out = [_empty_like_layout(t, rows) for t in (k, v)]
+    out = [o if o.stride(3) == 1 and all(s % 8 == 0 for s in o.stride()[:3])
+           else torch.empty((B, H, rows, D), dtype=k.dtype, device=k.device) for o in out]
+    with torch.cuda.device(k.device):
+        _lib.check(
+            _lib.lib().sinkattn_mean_pool_kv(
+                kk.data_ptr(), vk.data_ptr(), _lib.dtype_code(k.dtype), B, H, N, D, _lib.strides4(kk),
+                _lib.strides4(vk), first, end, gap, out[0].data_ptr(), out[1].data_ptr(), _lib.strides4(out[0]),
+                _lib.strides4(out[1]), _lib.stream_ptr(k.device),
+            ),
+            "mean_pool_kv",
+        )
+    return out[0], out[1]
+
+
 def block_sparse_attention_comp(
     q: torch.Tensor,
     k: torch.Tensor,

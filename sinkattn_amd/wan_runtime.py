@@ -184,8 +184,7 @@ class WanSinkSparseInnerAttention(nn.Module):
                   and _fused_compensation_supported(q, k, v)):
                 with _section(rs, "comp_pool"):
                     prefix = max(int(self.config.text_length), 0)
-                    k_dyn = ops.mean_pool_tokens(k, gap, prefix, like=k)
-                    v_dyn = ops.mean_pool_tokens(v, gap, prefix, like=v)
+                    k_dyn, v_dyn = ops.mean_pool_kv(k, v, gap, prefix)
                     dyn_len = int(k_dyn.size(2))
                 with _section(rs, "sparse_main"):  # sparse + compensation + mix
                     out = _block_sparse_attn_with_compensation(q, k, v, mask, k_dyn, v_dyn, gap)

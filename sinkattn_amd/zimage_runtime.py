@@ -501,11 +501,8 @@ class ZImageStaticSinkProcessor:
                       and _fused_compensation_supported(q_i, k_i, v_i)):
                     il = self.image_token_count
                     with sec("comp_pool"):
-                        dyn_k = ops.mean_pool_tokens(k_i[:, :, :il], gap)
-                        dyn_v = ops.mean_pool_tokens(v_i[:, :, :il], gap)
-                        if text_tokens > 0:
-                            dyn_k = torch.cat([dyn_k, k_i[:, :, il:n]], dim=2)
-                            dyn_v = torch.cat([dyn_v, v_i[:, :, il:n]], dim=2)
+                        # the pooled image keys, then the text keys
+                        dyn_k, dyn_v = ops.mean_pool_kv(k_i, v_i, gap, pool_end=il)
                         dyn_len = int(dyn_k.size(2))
                     with sec("sparse_main"):  # sparse + compensation on the image rows + mix
                         out_i = _block_sparse_attn_with_compensation(q_i, k_i, v_i, mask, dyn_k, dyn_v, gap,

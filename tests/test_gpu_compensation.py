@@ -197,3 +197,22 @@ def test_fused_compensation_argument_checks():
     o0, _ = ops.block_sparse_attention_comp(q, k, v, plan, kd, vd, 30, comp_rows=0)
     o1, _ = ops.block_sparse_attention(q, k, v, plan, return_lse=False)
     assert torch.equal(o0, o1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("N,gap,prefix,end", [(1, 30, 0, 1), (333, 30, 0, 333), (333, 7, 40, 200), (100, 8, 0, 64),
+                                              (64, 1, 5, 40), (50, 64, 0, 50), (90, 9, 90, 90), (70, 8, 0, 0)])
+def test_mean_pool_kv_matches_single_calls(dtype, N, gap, prefix, end):
+    """K and V in one launch with a kept suffix: the rows of mean_pool_tokens over [0, end), then
+    rows [end, N), bit for bit (the same sums in the same order); group sizes around the eight
+    loads in flight, both layouts."""
+    g = torch.Generator(device="cuda").manual_seed(N + gap)
+    k = torch.randn(2, N, 3, 64, device="cuda", generator=g).to(dtype).transpose(1, 2)
+    v = torch.randn(2, 3, N, 64, device="cuda", generator=g).to(dtype)
+    kd, vd = ops.mean_pool_kv(k, v, gap, prefix, end)
+    for got, x in ((kd, k), (vd, v)):
+        want = torch.cat([ops.mean_pool_tokens(x[:, :, :end], gap, prefix), x[:, :, end:]], 2) if end else x
+        assert torch.equal(got, want)
+        ref = torch_ref.mean_pool_tokens(x[:, :, :end], gap, prefix) if end else x[:, :, :0].cpu()
+        rnd = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -22}[dtype]
+        assert torch.allclose(got[:, :, :ref.shape[2]].float().cpu(), ref.float(), rtol=rnd, atol=1e-6)
