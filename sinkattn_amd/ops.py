@@ -165,6 +165,16 @@ class _PlanCache:
 PLAN_CACHE = _PlanCache()
 
 
+def _output(out: Optional[torch.Tensor], q: torch.Tensor) -> torch.Tensor:
+    """The caller's output tensor, checked, or a new one as a [B, H, N, D] view of [B, N, H, D] memory."""
+    if out is None:
+        B, H, N, D = q.shape
+        return torch.empty((B, N, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    if out.shape != q.shape or out.dtype != q.dtype or out.device != q.device:
+        raise ValueError(f"out must be {tuple(q.shape)} {q.dtype} on {q.device}, got {tuple(out.shape)} {out.dtype}")
+    return out
+
+
 def block_sparse_attention(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -172,11 +182,12 @@ def block_sparse_attention(
     plan: BlockSparsePlan,
     softmax_scale: Optional[float] = None,
     return_lse: bool = True,
+    out: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """Block-sparse attention forward on [B, H, N, D] views.
 
     Returns out as a [B, H, Nq, D] view of [B, Nq, H, D] memory (the layout the
-    reference's varlen call returns) and lse as fp32 [B, H, Nq] (or None).
+    reference's varlen call returns), or writes `out`, and lse as fp32 [B, H, Nq] (or None).
     """
     _require_cuda("block_sparse_attention", q, k, v)
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
@@ -194,7 +205,7 @@ def block_sparse_attention(
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
     qk, kk, vk = _kernel_operand(q), _kernel_operand(k), _kernel_operand(v)
-    out = torch.empty((B, Nq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    out = _output(out, q)
     lse = torch.empty((B, H, Nq), dtype=torch.float32, device=q.device) if return_lse else None
     L = _lib.lib()
     with torch.cuda.device(q.device):
@@ -355,6 +366,7 @@ def block_sparse_attention_comp(
     comp_rows: Optional[int] = None,
     softmax_scale: Optional[float] = None,
     return_lse: bool = False,
+    out: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """Block-sparse attention fused with the compensation branch: query rows below
     `comp_rows` (default all; must be a multiple of 128 or Nq) also attend every key of
@@ -381,7 +393,7 @@ def block_sparse_attention_comp(
     kdk, vdk = _kernel_operand(kd), _kernel_operand(vd)
     if kdk.stride(2) != kk.stride(2) or vdk.stride(2) != vk.stride(2):
         raise ValueError("kd/vd row strides must equal k/v row strides")
-    out = torch.empty((B, Nq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    out = _output(out, q)
     lse = torch.empty((B, H, Nq), dtype=torch.float32, device=q.device) if return_lse else None
     L = _lib.lib()
     with torch.cuda.device(q.device):

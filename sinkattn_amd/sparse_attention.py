@@ -653,6 +653,14 @@ def _block_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block_
     return out, lse.unsqueeze(-1).to(device=q.device, dtype=q.dtype)
 
 
+def _block_sparse_attn_into(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block_mask: torch.Tensor,
+                            out: torch.Tensor) -> torch.Tensor:
+    """`_block_sparse_attn(..., return_lse=False)` written into `out` [B,H,Nq,D]."""
+    _ensure_block_sparse_available()
+    plan = ops.PLAN_CACHE.get(block_mask if block_mask.is_cuda else block_mask.to(q.device))
+    return ops.block_sparse_attention(q, k, v, plan, softmax_scale=None, return_lse=False, out=out)[0]
+
+
 def _fused_compensation_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """The fused sparse + compensation kernel covers bf16/f16 GPU tensors with d = 128."""
     return (q.is_cuda and q.dim() == 4 and q.dtype in (torch.bfloat16, torch.float16)
@@ -662,7 +670,8 @@ def _fused_compensation_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
 def _block_sparse_attn_with_compensation(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                          block_mask: torch.Tensor, k_dynamic: torch.Tensor,
                                          v_dynamic: torch.Tensor, sample_gap: int,
-                                         compensated_rows: Optional[int] = None) -> torch.Tensor:
+                                         compensated_rows: Optional[int] = None,
+                                         out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Sparse attention and the pooled-K/V compensation with adaptive mixing in one kernel.
 
     The reference runs `_block_sparse_attn(..., return_lse=True)`, an attention over
@@ -677,7 +686,7 @@ def _block_sparse_attn_with_compensation(q: torch.Tensor, k: torch.Tensor, v: to
     _ensure_block_sparse_available()
     plan = ops.PLAN_CACHE.get(block_mask if block_mask.is_cuda else block_mask.to(q.device))
     out, _ = ops.block_sparse_attention_comp(q, k, v, plan, k_dynamic, v_dynamic, int(sample_gap),
-                                             comp_rows=compensated_rows, return_lse=False)
+                                             comp_rows=compensated_rows, return_lse=False, out=out)
     return out
 
 

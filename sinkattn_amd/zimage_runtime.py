@@ -16,7 +16,7 @@ from __future__ import annotations
 from contextlib import nullcontext
 from dataclasses import asdict
 from pathlib import Path
-from typing import Any, Dict, Optional
+from typing import Any, Callable, Dict, Optional
 
 import torch
 
@@ -25,6 +25,7 @@ from .sparse_attention import (
     SinkRuntimeState,
     SinkSparseConfig,
     _block_sparse_attn,
+    _block_sparse_attn_into,
     _block_sparse_attn_with_compensation,
     _build_direct_mean_coverage_mask,
     _build_direct_mean_coverage_masks,
@@ -379,15 +380,32 @@ class ZImageSinkMaskCalibrator:
         return package
 
 
-def _valid_lengths(attention_mask: Optional[torch.Tensor], batch_size: int, seq_len: int) -> list[int]:
+def _valid_lengths(attention_mask: Optional[torch.Tensor], batch_size: int, seq_len: int) -> Callable[[], list[int]]:
+    """Starts reading each sample's valid length and returns the call that waits for them: the
+    counts of a device mask are on their way to the host before the caller enqueues its
+    projections, so the wait is for the mask alone and the host runs ahead of the GPU."""
     if attention_mask is None:
-        return [seq_len] * batch_size
-    return [int(m.sum().item()) for m in attention_mask]
+        return lambda: [seq_len] * batch_size
+    if not (isinstance(attention_mask, torch.Tensor) and attention_mask.is_cuda and attention_mask.dim() >= 2):
+        return lambda: [int(m.sum().item()) for m in attention_mask]
+    with torch.cuda.device(attention_mask.device):
+        host = attention_mask.flatten(1).sum(dim=1).to("cpu", non_blocking=True)
+        done = torch.cuda.Event()
+        done.record()
+
+    def wait() -> list[int]:
+        done.synchronize()
+        return [int(x) for x in host.tolist()]
+
+    return wait
 
 
 def _sample_bhsd(t: torch.Tensor, b: int, n: int) -> torch.Tensor:
-    """Sample b's first n tokens of `[B, N, H, d]` as contiguous `[1, H, n, d]`."""
-    return t[b:b + 1, :n].permute(0, 2, 1, 3).contiguous()
+    """Sample b's first n tokens of `[B, N, H, d]` as `[1, H, n, d]`: a view when a token's heads are
+    contiguous (the kernels take row strides; pooled K/V then share them), else a copy."""
+    x = t[b:b + 1, :n].permute(0, 2, 1, 3)
+    h, d = int(t.size(2)), int(t.size(3))
+    return x if t.is_cuda and t.stride()[1:] == (h * d, d, 1) else x.contiguous()
 
 
 class ZImageSinkCalibrationProcessor:
@@ -405,9 +423,10 @@ class ZImageSinkCalibrationProcessor:
             raise AssertionError("Z-Image uses single-stream attention only.")
         if self.origin_processor is None:
             raise RuntimeError("Z-Image calibration requires access to the original dense attention processor.")
+        lengths = _valid_lengths(attention_mask, int(hidden_states.size(0)), int(hidden_states.size(1)))
         q, k, v = prepare_zimage_attention_tensors(attn, hidden_states, freqs_cis=freqs_cis)
         image_tokens = self.calibrator.image_token_count
-        for b, n in enumerate(_valid_lengths(attention_mask, int(hidden_states.size(0)), int(hidden_states.size(1)))):
+        for b, n in enumerate(lengths()):
             if n < image_tokens:
                 raise ValueError("Observed valid sequence shorter than the padded image token prefix. "
                                  f"valid_len={n}, image_token_count={image_tokens}")
@@ -436,6 +455,7 @@ class ZImageStaticSinkProcessor:
         self.image_token_count, self.image_blocks, self.total_blocks = _fixed_block_shape(self.config)
         self.max_text_tokens = _max_text_token_count(self.config)
         self._runtime_mask_cache: Dict[tuple, torch.Tensor] = {}
+        self._dense_mask_cache: Dict[tuple, torch.Tensor] = {}
 
     def _resolve_dynamic_plan(self) -> tuple[str, int]:
         mode = str(self.config.dynamic_mode).strip().lower()
@@ -464,6 +484,14 @@ class ZImageStaticSinkProcessor:
             self._runtime_mask_cache[key] = m
         return m
 
+    def _dense_mask(self, mask: torch.Tensor) -> torch.Tensor:
+        """The all-true mask a forced-dense call reports, one per runtime mask."""
+        key = (mask.device, tuple(mask.shape))
+        m = self._dense_mask_cache.get(key)
+        if m is None:
+            m = self._dense_mask_cache[key] = torch.ones_like(mask, dtype=torch.bool)
+        return m
+
     def __call__(self, attn: Any, hidden_states: torch.Tensor, encoder_hidden_states: Optional[torch.Tensor] = None,
                  attention_mask: Optional[torch.Tensor] = None, freqs_cis: Optional[torch.Tensor] = None) -> torch.Tensor:
         if encoder_hidden_states is not None:
@@ -473,14 +501,18 @@ class ZImageStaticSinkProcessor:
             rs.enter_layer(self.layer_idx)
         sec = (lambda name: rs.time_section(name)) if rs is not None else (lambda name: nullcontext())
         with sec("inner_total"):
+            B, N = int(hidden_states.size(0)), int(hidden_states.size(1))
+            lengths = _valid_lengths(attention_mask, B, N)
             with sec("qkv"):
                 query, key, value = prepare_zimage_attention_tensors(attn, hidden_states, freqs_cis=freqs_cis)
-            B, N = int(hidden_states.size(0)), int(hidden_states.size(1))
-            out_padded = hidden_states.new_zeros((B, N, attn.heads, int(query.size(-1))))
+            out_padded = hidden_states.new_empty((B, N, attn.heads, int(query.size(-1))))
             mode, gap = self._resolve_dynamic_plan()
             dense_step = self._should_force_dense_current_step()
             force_dense = dense_step or self._should_force_dense_current_layer()
-            for b, n in enumerate(_valid_lengths(attention_mask, B, N)):
+            valid = lengths()
+            for b in range(len(valid), B):
+                out_padded[b] = 0
+            for b, n in enumerate(valid):
                 if n < self.image_token_count:
                     raise ValueError("Observed valid sequence shorter than the padded image token prefix. "
                                      f"valid_len={n}, image_token_count={self.image_token_count}")
@@ -491,11 +523,14 @@ class ZImageStaticSinkProcessor:
                 text_blocks = _ceil_div(int(text_tokens), int(self.config.block_size))
                 mask = self._runtime_mask(text_blocks, query.device)
                 q_i, k_i, v_i = _sample_bhsd(query, b, n), _sample_bhsd(key, b, n), _sample_bhsd(value, b, n)
+                # this sample's rows of the output, which the kernels write when the types agree
+                rows = out_padded[b:b + 1, :n].permute(0, 2, 1, 3)
+                into = rows if out_padded.dtype == q_i.dtype and out_padded.device == q_i.device else None
                 dyn_len = None
                 if force_dense:
                     with sec("dense_override"):
                         out_i = _dense_attention(q_i, k_i, v_i)
-                    mask = torch.ones_like(mask, dtype=torch.bool)
+                    mask = self._dense_mask(mask)
                     run_mode = "forced_dense_step" if dense_step else "forced_dense_layer"
                 elif (mode == "pooled_kv" and FUSE_COMPENSATION and self.image_token_count % 128 == 0
                       and _fused_compensation_supported(q_i, k_i, v_i)):
@@ -506,7 +541,11 @@ class ZImageStaticSinkProcessor:
                         dyn_len = int(dyn_k.size(2))
                     with sec("sparse_main"):  # sparse + compensation on the image rows + mix
                         out_i = _block_sparse_attn_with_compensation(q_i, k_i, v_i, mask, dyn_k, dyn_v, gap,
-                                                                     compensated_rows=il)
+                                                                     compensated_rows=il, out=into)
+                    run_mode = mode
+                elif mode == "none" and into is not None:
+                    with sec("sparse_main"):
+                        out_i = _block_sparse_attn_into(q_i, k_i, v_i, mask, into)
                     run_mode = mode
                 else:
                     with sec("sparse_main"):
@@ -537,7 +576,10 @@ class ZImageStaticSinkProcessor:
                                                            config=self.config, dynamic_sample_gap=gap)
                             out_i = out_i.clone()
                             out_i[:, :, :il] = mixed
-                out_padded[b, :n] = out_i.transpose(1, 2)[0]
+                if out_i is not into:
+                    rows.copy_(out_i)
+                if n < N:
+                    out_padded[b, n:] = 0
                 if rs is not None:
                     rs.record_mask_stats(layer_idx=self.layer_idx, sink_mask_tag="__base__", dynamic_mode=run_mode,
                                          dynamic_sample_gap=0 if force_dense else int(gap), base_runtime_mask=mask,
