@@ -687,6 +687,223 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_small_kernel(FwdArgs 
   fwd_qblock<CT, D, kSparse>(a, (SA_LDS char*)lds_k, (SA_LDS char*)lds_v);
 }
 
+// ------------------------------------------------------------------------------------
+// Calls of few q-blocks, 16-bit: a group takes a quarter of a q-block (32 query rows) and its four
+// waves the four 32-key quarters of every listed tile, each through its own 32-row slices of the K
+// and V buffers (copies, reads and waits are the wave's own: no barrier in the loop); the waves'
+// partial outputs meet at the end, rescaled to the common maximum.  Four times the groups, each with
+// a quarter of the matrix work per tile, for four times the K/V reads.  Bound by the latency of
+// a tile's copies.  bf16 D = 128: 16 q-blocks of 5 tiles 17.9 -> 11.5 us, 47 of 47 tiles 97 -> 54,
+// 125 of 39 tiles 109 -> 72; the line against the whole-q-block kernels is at split_rows.
+// A wave's tile: S^T (two 16-key tiles), K(t+1)'s copies once its reads are back, softmax, O^T.
+// V(t)'s copies fly under S and the softmax, K(t+1)'s under the softmax and O^T.
+// ------------------------------------------------------------------------------------
+template <int CT, int D>
+__global__ __launch_bounds__(256, 2) void block_sparse_fwd_split_kernel(FwdArgs a) {
+  using G = TileGeom<D>;
+  constexpr int KS = D / 32, DT = D / 16;
+  constexpr int NC = 32 / G::kCopyRows;  // copies of a wave's 32-row slice
+  constexpr int kSlice = 32 * G::kRow;   // bytes of a slice
+  __shared__ u32x4 lds_k[16 * D], lds_v[16 * D];  // four slices, then two waves' fp32 outputs, each
+  __shared__ float lds_m[4][32], lds_l[4][32];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, sl = lane & 15;
+  // the four parts of an order slot run on the slot's XCD, one after the other
+  const int slot = (int)(blockIdx.x / (4 * kXcds)) * kXcds + (int)(blockIdx.x % kXcds);
+  const int part = (int)(blockIdx.x / kXcds) & 3;
+  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+  if (item < 0 || item >= a.B * a.H * a.nqb) return;
+  const AttnItem it = attn_item<false>(a, item);
+  const int q0 = it.qb * 128 + part * 32;  // first query row of the group
+  if (q0 >= a.Nq) return;
+  const uint32_t kstride = (uint32_t)a.ks[2] * 2, vstride = (uint32_t)a.vs[2] * 2;
+  const TileLanes<D> L = tile_lanes<D>(0, lane, 0, 0);
+  SA_LDS char* lk = (SA_LDS char*)lds_k + wave * kSlice;
+  SA_LDS char* lv = (SA_LDS char*)lds_v + wave * kSlice;
+  uint32_t k_off[NC], v_off[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int row = G::kCopyRows * j + lane / G::kChunks, ch = lane % G::kChunks;
+    k_off[j] = (uint32_t)row * kstride + (uint32_t)((ch ^ G::kswz(row)) * 16);
+    v_off[j] = (uint32_t)row * vstride + (uint32_t)((ch ^ G::vswz(row)) * 16);
+  }
+  // this wave's 32 rows of the tile at key0 (none past klim: a 0-byte buffer reads as zeros)
+  auto copy = [&](SA_LDS char* dst, const char* base, uint32_t stride, const uint32_t (&off)[NC], int rows)
+                  __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, rows > 0 ? (uint32_t)rows * stride : 0u);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) dma16(rs, (SA_LDS void*)(dst + j * 1024), off[j]);
+  };
+
+  u32x4 qf[2][KS];
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    const int qrow = q0 + 16 * qt + sl;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[qt][ks] = qrow < a.Nq ? *(const u32x4*)(it.qbase + ((int64_t)qrow * a.qs[2] + 32 * ks + 8 * g) * 2)
+                               : u32x4{0, 0, 0, 0};
+  }
+  f32x4 o[DT][2];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt][0] = o[dt][1] = f32x4{};
+  float m_run[2] = {neg_inf(), neg_inf()};
+  f32x4 l_acc[2] = {f32x4{}, f32x4{}};
+  const float c = a.scale * kLog2e;
+  const int Nk = a.Nk, Nd = a.Nd;
+  const float comp_bias = a.comp_bias;
+
+  int key0 = attn_key0<false>(it, 0) + 32 * wave;  // this wave's first key
+  int klim = it.cnt > 0 ? Nk : Nd;
+  if (it.ntot > 0) copy(lk, (it.cnt == 0 ? it.kdbase : it.kbase) + (int64_t)key0 * kstride, kstride, k_off, klim - key0);
+  for (int t = 0; t < it.ntot; ++t) {
+    const bool next = t + 1 < it.ntot;
+    const bool comp = t >= it.cnt;
+    const bool comp_next = t + 1 >= it.cnt;
+    const int key0_next = attn_key0<false>(it, t + 1) + 32 * wave;
+    const int klim_next = comp_next ? Nd : Nk;
+    const bool some = key0 < klim;  // the last tile may have no keys for this wave
+    copy(lv, (comp ? it.vdbase : it.vbase) + (int64_t)key0 * vstride, vstride, v_off, klim - key0);
+    __builtin_amdgcn_s_waitcnt(NC | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(NC): K(t) has landed
+    f32x4 s[2][2];
+    s[0][0] = s[0][1] = s[1][0] = s[1][1] = f32x4{};
+    if (some) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+          const u32x4 kr = *(SA_LDS const u32x4*)(lk + L.ka[ks] + kt * (32 * D));
+          s[kt][0] = mfma16x16x32<CT>(kr, qf[0][ks], s[kt][0]);
+          s[kt][1] = mfma16x16x32<CT>(kr, qf[1][ks], s[kt][1]);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): K's reads are back
+    copy(lk, (comp_next ? it.kdbase : it.kbase) + (int64_t)key0_next * kstride, kstride, k_off,
+         next ? klim_next - key0_next : 0);
+    u32x4 p[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
+    if (some) {
+      if (key0 + 32 > klim) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (key0 + 16 * kt + 4 * g + i >= klim) s[kt][0][i] = s[kt][1][i] = neg_inf();
+      }
+      const float bias = comp ? comp_bias : 0.f;
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt) {
+        float mx = neg_inf();
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][qt][i]);
+        const float m_tile = __builtin_fmaf(max_col16(mx), c, bias);
+        if (m_tile > m_run[qt] + kLazyRescaleLog2) {
+          const float alpha = fast_exp2(m_run[qt] - m_tile);
+          l_acc[qt] *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o[dt][qt] *= alpha;
+          m_run[qt] = m_tile;
+        }
+        // a quarter whose scores are all -inf has no reference yet: its P are 0
+        const float nb = bias - (m_run[qt] == neg_inf() ? 0.f : m_run[qt]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const float v0 = fast_exp2(__builtin_fmaf(s[u][qt][2 * e], c, nb));
+            const float v1 = fast_exp2(__builtin_fmaf(s[u][qt][2 * e + 1], c, nb));
+            if constexpr (!kMfmaSums<D, kSparse>) l_acc[qt][0] += v0 + v1;
+            p[qt][2 * u + e] = pack2<CT>(v0, v1);
+          }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(NC | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(NC): V(t) has landed
+    if (some) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        SA_LDS char* at = lv + L.va[dt];
+        const u32x2 y0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)at));
+        const u32x2 y1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((SA_LDS v4i16*)(at + 32 * D)));
+        const u32x4 vr = u32x4{y0[0], y0[1], y1[0], y1[1]};
+        o[dt][0] = mfma16x16x32<CT>(vr, p[0], o[dt][0]);
+        o[dt][1] = mfma16x16x32<CT>(vr, p[1], o[dt][1]);
+      }
+      if constexpr (kMfmaSums<D, kSparse>) {
+        const uint32_t one = CT == kBF16 ? 0x3F803F80u : 0x3C003C00u;
+        const u32x4 ones = {one, one, one, one};
+        l_acc[0] = mfma16x16x32<CT>(ones, p[0], l_acc[0]);
+        l_acc[1] = mfma16x16x32<CT>(ones, p[1], l_acc[1]);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): V's reads are back
+    key0 = key0_next;
+    klim = klim_next;
+  }
+
+  // The waves' maxima and sums, then their outputs in units of the common maximum, through LDS.
+  float l[2];
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    l[qt] = kMfmaSums<D, kSparse> ? l_acc[qt][0] : sum_col16(l_acc[qt][0]);
+    if (g == 0) {
+      lds_m[wave][16 * qt + sl] = m_run[qt];
+      lds_l[wave][16 * qt + sl] = l[qt];
+    }
+  }
+  drain_then_barrier();  // every wave is done with its slices, no copy is in flight
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    const int row = 16 * qt + sl;
+    const float m = fmaxf(fmaxf(lds_m[0][row], lds_m[1][row]), fmaxf(lds_m[2][row], lds_m[3][row]));
+    const float f = m_run[qt] == neg_inf() ? 0.f : fast_exp2(m_run[qt] - m);
+    // fp32 [32 rows][D] per wave, 16-byte chunks swizzled by the row: waves 0 and 1 in the K
+    // buffer, 2 and 3 in the V buffer
+    SA_LDS char* ob = (SA_LDS char*)(wave < 2 ? lds_k : lds_v) + (wave & 1) * (32 * D * 4) + row * (D * 4);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      f32x4 x = o[dt][qt];
+      if (m_run[qt] == neg_inf()) x = l[qt] * x;  // no finite score: 0, or NaN
+      else x *= f;
+      *(SA_LDS f32x4*)(ob + ((4 * dt + g) ^ (row & (D / 4 - 1) & 15)) * 16) = x;
+    }
+  }
+  __syncthreads();
+  // eight lanes per row, D / 8 columns each
+  const int row = tid >> 3, col = (tid & 7) * (D / 8);
+  const int qrow = q0 + row;
+  float m = neg_inf(), lt = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) m = fmaxf(m, lds_m[w][row]);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float mw = lds_m[w][row];
+    lt += mw == neg_inf() ? lds_l[w][row] : lds_l[w][row] * fast_exp2(mw - m);
+  }
+  // no listed key: zeros; a sum of 0 over listed keys (every score -inf): NaN
+  const float inv = it.ntot == 0 ? 0.f : 1.f / lt;
+  u32x2 w2[D / 32];
+#pragma unroll
+  for (int j = 0; j < D / 32; ++j) {
+    const int at = row * (D * 4) + (((col >> 2) + j) ^ (row & (D / 4 - 1) & 15)) * 16;
+    f32x4 x = *(SA_LDS const f32x4*)((SA_LDS char*)lds_k + at);
+    x += *(SA_LDS const f32x4*)((SA_LDS char*)lds_k + 32 * D * 4 + at);
+    x += *(SA_LDS const f32x4*)((SA_LDS char*)lds_v + at);
+    x += *(SA_LDS const f32x4*)((SA_LDS char*)lds_v + 32 * D * 4 + at);
+    w2[j][0] = pack2<CT>(x[0] * inv, x[1] * inv);
+    w2[j][1] = pack2<CT>(x[2] * inv, x[3] * inv);
+  }
+  if (qrow >= a.Nq) return;
+  const int bh = item / a.nqb;
+  const int b = bh / a.H, h = bh - b * a.H;
+  char* op = (char*)a.out + ((int64_t)b * a.os[0] + (int64_t)h * a.os[1] + (int64_t)qrow * a.os[2] + col) * 2;
+#pragma unroll
+  for (int j = 0; j < D / 32; ++j) *reinterpret_cast<u32x2*>(op + 8 * j) = w2[j];
+  if (a.lse != nullptr && (tid & 7) == 0)
+    a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] = it.ntot > 0 ? (m + __log2f(lt)) * kLn2 : pos_inf();
+}
+
 // fp32 operands: every value is split as x = hi + lo with hi = bf16(x) and
 // lo = bf16(x - hi); each product is formed as hi*hi + hi*lo + lo*hi on the bf16 matrix
 // cores (about 16 mantissa bits), for QK^T and for PV (P split the same way).  Bound by those
@@ -1494,10 +1711,21 @@ static bool buffer_rows(const FwdArgs& a, int D) {
   return a.Nk > 0 && a.ks[2] >= D && a.vs[2] >= D && a.Nk * a.ks[2] * 2 < lim && a.Nk * a.vs[2] * 2 < lim;
 }
 
+// q-blocks up to which a 16-bit call runs the split kernel: as many as give one round of its
+// groups (two per CU at D = 128, four below).  Against the whole q-block per group, bf16: 1.15-1.8
+// times as fast up to 128 q-blocks at D = 128 (0.85-1.1 at 140-190, 0.75-0.9 past 230); f16 D = 64
+// 1.1-1.9 up to 200, 1.0-1.15 at 230-280, 0.93-1.0 past 310.
+constexpr int split_rows(int D) { return D == 128 ? 128 : 256; }
+
 template <int IT, int CT>
 static hipError_t launch_fwd_dt(const FwdArgs& a, int D, hipStream_t stream) {
   const int grid = fwd_grid(a);
-  if (D == 128)
+  if (a.B * a.H * a.nqb <= split_rows(D) && buffer_rows(a, D)) {
+    const int parts = 4 * ((grid + kXcds - 1) / kXcds * kXcds);
+    if (D == 128) block_sparse_fwd_split_kernel<CT, 128><<<parts, 256, 0, stream>>>(a);
+    else if (D == 64) block_sparse_fwd_split_kernel<CT, 64><<<parts, 256, 0, stream>>>(a);
+    else block_sparse_fwd_split_kernel<CT, 32><<<parts, 256, 0, stream>>>(a);
+  } else if (D == 128)
     block_sparse_fwd_d128_kernel<CT><<<grid, 256, 0, stream>>>(a);
   else if (buffer_rows(a, D))
     if (D == 64) block_sparse_fwd_small_kernel<CT, 64><<<grid, 256, 0, stream>>>(a);

@@ -308,6 +308,30 @@ def test_dense_mass_in_several_launches():
                                                                            v[:, h:h + 1])[0])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,Nq,Nk", [(128, 300, 417), (128, 33, 1000), (64, 300, 417), (32, 161, 97)])
+def test_few_and_many_q_blocks(dtype, D, Nq, Nk):
+    """The split kernel (few q-blocks) and the whole-q-block kernels (the same heads repeated over a
+    batch past the line) on ragged lengths, an empty row and a quarter of a tile whose scores are
+    all -inf: both at the attention bars, keys of -inf score without weight."""
+    q, k, v = _inputs(1, 2, Nq, Nk, D, dtype, seed=D + Nq)
+    q = q.abs()
+    mask = _random_mask(1, 2, -(-Nq // 128), -(-Nk // 128), 0.6, seed=9, empty_rows=1 if Nq > 128 else 0)
+    many = 300 // (2 * mask.shape[2]) + 1
+    for inf_keys in (0, 32):
+        kk = k.clone()
+        kk[:, :, 32:32 + inf_keys] = -math.inf
+        ref_o, ref_l = torch_ref.dense_masked_attention(q, kk, v, mask)
+        fin = torch.isfinite(ref_l)
+        for rep in (1, many):
+            qr, kr, vr, mr = (t.expand(rep, -1, -1, -1) for t in (q, kk, v, mask.contiguous()))
+            out, lse = ops.block_sparse_attention(qr, kr, vr, ops.block_sparse_plan(mr.contiguous()))
+            err = (out[-1:].float().cpu() - ref_o).abs()
+            assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS, (rep, inf_keys, err.max())
+            assert torch.equal(torch.isfinite(lse[-1:].cpu()), fin)
+            assert ((lse[-1:].cpu() - ref_l)[fin].abs() <= LSE_ABS + 1e-5 * ref_l[fin].abs()).all()
+
+
 def _chunk_layout(nbh, nqb):
     """Chunking of the launch order: heads [0, nbh_w) in Cw chunks (qb mod Cw), the heads
     of the partial last round of 8 in Cs = Cw * F finer chunks."""
