@@ -117,6 +117,16 @@ int sinkattn_block_sparse_fwd(const void* q, const void* k, const void* v, int d
                               const int32_t* counts, const int32_t* idx,
                               const int32_t* order, int64_t nqb, int64_t nkb,
                               float softmax_scale, void* stream);
+/* The same for bf16/f16 operands with lse [B,H,Nq] written in their type (rounded to nearest
+ * even), the form the reference's call returns (sinkattention/sparse_attention.py:776). */
+int sinkattn_block_sparse_fwd_lse16(const void* q, const void* k, const void* v, int dtype,
+                                    int64_t B, int64_t H, int64_t Nq, int64_t Nk, int64_t D,
+                                    const int64_t q_strides[4], const int64_t k_strides[4],
+                                    const int64_t v_strides[4],
+                                    void* out, const int64_t out_strides[4], void* lse,
+                                    const int32_t* counts, const int32_t* idx,
+                                    const int32_t* order, int64_t nqb, int64_t nkb,
+                                    float softmax_scale, void* stream);
 
 /* ------------------------------------------------------------------------------------
  * Block-sparse forward fused with the compensation branch ("pooled_kv" dynamic mode with

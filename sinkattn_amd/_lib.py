@@ -43,6 +43,12 @@ SIGNATURES = {
          _c_i64_4, _c_i64_4, _c_i64_4, _c_p, _c_i64_4, _c_p, _c_p, _c_p, _c_p,
          _c_i64, _c_i64, ctypes.c_float, _c_p],
     ),
+    "sinkattn_block_sparse_fwd_lse16": (
+        ctypes.c_int,
+        [_c_p, _c_p, _c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+         _c_i64_4, _c_i64_4, _c_i64_4, _c_p, _c_i64_4, _c_p, _c_p, _c_p, _c_p,
+         _c_i64, _c_i64, ctypes.c_float, _c_p],
+    ),
     "sinkattn_block_sparse_fwd_comp": (
         ctypes.c_int,
         [_c_p, _c_p, _c_p, ctypes.c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,

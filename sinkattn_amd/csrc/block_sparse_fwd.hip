@@ -27,6 +27,13 @@
 
 namespace sa {
 
+// A row's lse, fp32 or rounded to the call's 16-bit type.
+template <int CT>
+__device__ __forceinline__ void store_lse(const FwdArgs& a, int64_t row, float x) {
+  if (a.lse16) reinterpret_cast<uint16_t*>(a.lse)[row] = (uint16_t)(pack2<CT>(x, 0.f) & 0xffffu);
+  else reinterpret_cast<float*>(a.lse)[row] = x;
+}
+
 template <int IT, int CT, int D>
 __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
   constexpr int ES = ElemSize<IT>::value;
@@ -158,8 +165,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
                    o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv);
       }
     if (a.lse != nullptr && hl == 0)
-      a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] =
-          cnt > 0 ? (m_run + __log2f(l)) * kLn2 : pos_inf();
+      store_lse<CT>(a, ((int64_t)b * a.H + h) * a.Nq + qrow, cnt > 0 ? (m_run + __log2f(l)) * kLn2 : pos_inf());
   }
 }
 
@@ -535,7 +541,8 @@ __device__ __forceinline__ void store_o_staged(const FwdArgs& a, const AttnItem&
     for (int qt = 0; qt < 2; ++qt) {
       const int qrow = q0 + 16 * qt + sl;
       if (qrow < a.Nq)
-        a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] = it.ntot > 0 ? (m_run[qt] + __log2f(l[qt])) * kLn2 : pos_inf();
+        store_lse<CT>(a, ((int64_t)b * a.H + h) * a.Nq + qrow,
+                      it.ntot > 0 ? (m_run[qt] + __log2f(l[qt])) * kLn2 : pos_inf());
     }
   }
 }
@@ -901,7 +908,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_split_kernel(FwdArgs 
 #pragma unroll
   for (int j = 0; j < D / 32; ++j) *reinterpret_cast<u32x2*>(op + 8 * j) = w2[j];
   if (a.lse != nullptr && (tid & 7) == 0)
-    a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] = it.ntot > 0 ? (m + __log2f(lt)) * kLn2 : pos_inf();
+    store_lse<CT>(a, ((int64_t)b * a.H + h) * a.Nq + qrow, it.ntot > 0 ? (m + __log2f(lt)) * kLn2 : pos_inf());
 }
 
 // fp32 operands: every value is split as x = hi + lo with hi = bf16(x) and
@@ -1150,7 +1157,8 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_f32_kernel(FwdArgs a)
       store4<kF32>(obase + 16 * dt + 4 * g, o[dt][qt][0] * inv, o[dt][qt][1] * inv, o[dt][qt][2] * inv,
                    o[dt][qt][3] * inv);
     if (a.lse != nullptr && g == 0)
-      a.lse[((int64_t)b * a.H + h) * a.Nq + qrow] = cnt > 0 ? (m_run[qt] + __log2f(l)) * kLn2 : pos_inf();
+      reinterpret_cast<float*>(a.lse)[((int64_t)b * a.H + h) * a.Nq + qrow] =
+          cnt > 0 ? (m_run[qt] + __log2f(l)) * kLn2 : pos_inf();
   }
 }
 

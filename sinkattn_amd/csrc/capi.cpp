@@ -140,9 +140,9 @@ struct CompTiles {
 int block_sparse_fwd_impl(const void* q, const void* k, const void* v, int dtype, int64_t B,
                           int64_t H, int64_t Nq, int64_t Nk, int64_t D, const int64_t q_strides[4],
                           const int64_t k_strides[4], const int64_t v_strides[4], void* out,
-                          const int64_t out_strides[4], float* lse, const int32_t* counts,
+                          const int64_t out_strides[4], void* lse, const int32_t* counts,
                           const int32_t* idx, const int32_t* order, int64_t nqb, int64_t nkb,
-                          float softmax_scale, const CompTiles& comp, void* stream) {
+                          float softmax_scale, const CompTiles& comp, void* stream, bool lse16 = false) {
   if (!valid_dtype(dtype)) return fail("fwd: unsupported dtype %d", dtype);
   if (D != 32 && D != 64 && D != 128) return fail("fwd: head dim %lld not supported (32, 64 or 128)", (long long)D);
   if (B < 0 || H < 0 || Nq < 0 || Nk < 0) return fail("fwd: negative size");
@@ -168,6 +168,7 @@ int block_sparse_fwd_impl(const void* q, const void* k, const void* v, int dtype
   a.v = v;
   a.out = out;
   a.lse = lse;
+  a.lse16 = lse16 ? 1 : 0;
   for (int i = 0; i < 4; ++i) {
     a.qs[i] = q_strides[i];
     a.ks[i] = k_strides[i];
@@ -222,6 +223,19 @@ int sinkattn_block_sparse_fwd(const void* q, const void* k, const void* v, int d
   return block_sparse_fwd_impl(q, k, v, dtype, B, H, Nq, Nk, D, q_strides, k_strides, v_strides, out,
                                out_strides, lse, counts, idx, order, nqb, nkb, softmax_scale, CompTiles{},
                                stream);
+}
+
+int sinkattn_block_sparse_fwd_lse16(const void* q, const void* k, const void* v, int dtype, int64_t B,
+                                    int64_t H, int64_t Nq, int64_t Nk, int64_t D,
+                                    const int64_t q_strides[4], const int64_t k_strides[4],
+                                    const int64_t v_strides[4], void* out, const int64_t out_strides[4],
+                                    void* lse, const int32_t* counts, const int32_t* idx,
+                                    const int32_t* order, int64_t nqb, int64_t nkb, float softmax_scale,
+                                    void* stream) {
+  if (dtype == SINKATTN_F32) return fail("fwd_lse16: bf16 or f16 operands");
+  return block_sparse_fwd_impl(q, k, v, dtype, B, H, Nq, Nk, D, q_strides, k_strides, v_strides, out,
+                               out_strides, lse, counts, idx, order, nqb, nkb, softmax_scale, CompTiles{},
+                               stream, true);
 }
 
 int sinkattn_block_sparse_fwd_comp(const void* q, const void* k, const void* v, int dtype, int64_t B,

@@ -24,7 +24,8 @@ struct FwdArgs {
   const void* k;
   const void* v;
   void* out;
-  float* lse;
+  void* lse;  // fp32 [B,H,Nq], or the operands' 16-bit type when lse16, or null
+  int lse16;
   int64_t qs[4], ks[4], vs[4], os[4];
   const int32_t* counts;
   const int32_t* idx;

@@ -183,11 +183,13 @@ def block_sparse_attention(
     softmax_scale: Optional[float] = None,
     return_lse: bool = True,
     out: Optional[torch.Tensor] = None,
+    lse_in_dtype: bool = False,
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """Block-sparse attention forward on [B, H, N, D] views.
 
     Returns out as a [B, H, Nq, D] view of [B, Nq, H, D] memory (the layout the
-    reference's varlen call returns), or writes `out`, and lse as fp32 [B, H, Nq] (or None).
+    reference's varlen call returns), or writes `out`, and lse [B, H, Nq] as fp32, or rounded
+    to q.dtype with `lse_in_dtype` (or None).
     """
     _require_cuda("block_sparse_attention", q, k, v)
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
@@ -206,11 +208,15 @@ def block_sparse_attention(
         softmax_scale = 1.0 / math.sqrt(D)
     qk, kk, vk = _kernel_operand(q), _kernel_operand(k), _kernel_operand(v)
     out = _output(out, q)
-    lse = torch.empty((B, H, Nq), dtype=torch.float32, device=q.device) if return_lse else None
+    lse16 = lse_in_dtype and q.dtype != torch.float32
+    lse = None
+    if return_lse:
+        lse = torch.empty((B, H, Nq), dtype=q.dtype if lse16 else torch.float32, device=q.device)
     L = _lib.lib()
+    fwd = L.sinkattn_block_sparse_fwd_lse16 if lse16 else L.sinkattn_block_sparse_fwd
     with torch.cuda.device(q.device):
         _lib.check(
-            L.sinkattn_block_sparse_fwd(
+            fwd(
                 qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), dt, B, H, Nq, Nk, D,
                 _lib.strides4(qk), _lib.strides4(kk), _lib.strides4(vk),
                 out.data_ptr(), _lib.strides4(out), _lib.ptr(lse),

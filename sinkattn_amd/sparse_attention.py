@@ -647,10 +647,8 @@ def _block_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block_
     """
     _ensure_block_sparse_available()
     plan = ops.PLAN_CACHE.get(block_mask if block_mask.is_cuda else block_mask.to(q.device))
-    out, lse = ops.block_sparse_attention(q, k, v, plan, softmax_scale=None, return_lse=return_lse)
-    if lse is None:
-        return out, None
-    return out, lse.unsqueeze(-1).to(device=q.device, dtype=q.dtype)
+    out, lse = ops.block_sparse_attention(q, k, v, plan, softmax_scale=None, return_lse=return_lse, lse_in_dtype=True)
+    return out, None if lse is None else lse.unsqueeze(-1)
 
 
 def _block_sparse_attn_into(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block_mask: torch.Tensor,

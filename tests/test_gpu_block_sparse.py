@@ -332,6 +332,23 @@ def test_few_and_many_q_blocks(dtype, D, Nq, Nk):
             assert ((lse[-1:].cpu() - ref_l)[fin].abs() <= LSE_ABS + 1e-5 * ref_l[fin].abs()).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("D,B,N", [(128, 1, 300), (128, 60, 300), (64, 1, 300), (64, 100, 300), (32, 2, 129)])
+def test_lse_in_the_operands_type(dtype, D, B, N):
+    """The kernels' rounded lse is the fp32 lse cast to the type, bit for bit, rows without a
+    listed key (+inf) included, in every 16-bit kernel (few and many q-blocks, overlapping rows)."""
+    q, k, v = _inputs(1, 2, N, N, D, dtype, seed=D + B)
+    nb = -(-N // 128)
+    mask = _random_mask(B, 2, nb, nb, 0.6, seed=9, empty_rows=1)
+    plan = ops.block_sparse_plan(mask)
+    q, k, v = (t.expand(B, -1, -1, -1) for t in (q, k, v))
+    forms = [(k, v)] + ([(k[:, :, :1].expand(-1, -1, N, -1),) * 2] if D < 128 else [])
+    for kk, vv in forms:
+        full = ops.block_sparse_attention(q, kk, vv, plan)[1]
+        own = ops.block_sparse_attention(q, kk, vv, plan, lse_in_dtype=True)[1]
+        assert own.dtype == dtype and torch.equal(own, full.to(dtype)) and bool(torch.isinf(own).any())
+
+
 def _chunk_layout(nbh, nqb):
     """Chunking of the launch order: heads [0, nbh_w) in Cw chunks (qb mod Cw), the heads
     of the partial last round of 8 in Cs = Cw * F finer chunks."""
