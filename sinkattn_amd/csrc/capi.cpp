@@ -541,8 +541,7 @@ size_t sinkattn_block_mass_pool_workspace_bytes(int64_t B, int64_t H, int64_t Nq
                                                 int64_t block_size, int dtype) {
   if (dtype == SINKATTN_F32 || !mass_mfma_block(block_size)) return 0;
   const int64_t items = B * H * cdiv(Nq, 128);  // items of 128 query rows
-  const int64_t groups = items < sa::block_mass_groups() ? items : sa::block_mass_groups();
-  return (size_t)(groups * cdiv(Nk, block_size) * 128 * (int64_t)sizeof(float));
+  return sa::block_mass_workspace_floats(items, cdiv(Nk, block_size), Nk) * sizeof(float);
 }
 
 int sinkattn_block_mass_pool(const void* q, const void* k, int dtype, int64_t B, int64_t H,

@@ -124,6 +124,7 @@ hipError_t launch_dense_mass(const FwdArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
 bool pool_f32_mfma(const PoolArgs& a);
 int block_mass_groups();
+size_t block_mass_workspace_floats(int64_t items, int64_t nkb, int64_t Nk);
 int device_cu_count();
 // Resident work-groups of the persistent max-pool kernel: its workspace holds one slot per
 // group, so the launch and the workspace query both use this count.

@@ -50,19 +50,20 @@ __device__ __forceinline__ constexpr int sub_block(int t, int j) {
   return KB == 16 ? 2 * t + (j >> 3) : (t * 32) / KB;
 }
 
-template <int CT, int KB>
-__global__ __launch_bounds__(256, 3) void block_mass_persistent_kernel(PoolArgs a, int items) {
+// The tiles [t0, t1) of one item: each row's block sums into ws[kb][row], its reference maximum
+// and the sum of all of them in m_ref and l_tot (the same in both lanes of a row).  RANGED (t0 may
+// be past the first tile): a row whose scores are all -inf so far has no reference and takes it
+// from the first tile that has one.
+template <int CT, int KB, bool RANGED>
+__device__ __forceinline__ void mass_tiles(const PoolArgs& a, SA_LDS char* lk, int item, int t0, int t1, float* ws,
+                                           float& m_ref, float& l_tot) {
   constexpr int DS = 8;
   constexpr int NS = 128 / KB;  // key blocks per 128-key tile, q-blocks per 128-row item
-  __shared__ u32x4 lds_k[2048];
-  __shared__ float row_inv[128];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hl = lane >> 5, l32 = lane & 31;
-  const int nkb = a.nkb;                 // key blocks of the map (KB keys each)
-  const int ntiles = (a.Nk + 127) >> 7;  // 128-key tiles
-  const int nqi = (a.Nq + 127) >> 7;     // 128-row items per head
-  float* ws = a.ws + (size_t)blockIdx.x * (size_t)nkb * 128;
+  const int nkb = a.nkb;               // key blocks of the map (KB keys each)
+  const int nqi = (a.Nq + 127) >> 7;   // 128-row items per head
   const uint32_t kstride = (uint32_t)a.ks[2] * 2;
   const int drow = 4 * wave + (lane >> 4);
   const uint32_t k_off = (uint32_t)drow * kstride + (uint32_t)(((lane & 15) ^ (drow & 15)) * 16);
@@ -70,97 +71,118 @@ __global__ __launch_bounds__(256, 3) void block_mass_persistent_kernel(PoolArgs 
   uint32_t ka[DS];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) ka[ds] = (uint32_t)(prow * 256 + (((2 * ds + hl) ^ (prow & 15)) * 16));
-  SA_LDS char* lk = (SA_LDS char*)lds_k;
   const float c = a.scale * kLog2e;
+  const int r = wave * 32 + l32;
+  const int bh = item / nqi;
+  const int qi = item - bh * nqi;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const char* qbase = (const char*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1]) * 2;
+  const char* kbase = (const char*)a.k + ((int64_t)b * a.ks[0] + (int64_t)h * a.ks[1]) * 2;
+  const int qrow = qi * 128 + r;
+  u32x4 qf[DS];
+  load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
+  m_ref = neg_inf();
+  l_tot = 0.f;
+
+  for (int kt = t0; kt < t1; ++kt) {
+    const int key0 = kt * 128;
+    __syncthreads();  // the previous tile (or item epilogue) is done with lds_k
+    {
+      const __amdgpu_buffer_rsrc_t rs =
+          make_rsrc(kbase + (int64_t)key0 * kstride, (uint32_t)(a.Nk - key0) * kstride);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        dma16(rs, (SA_LDS void*)(lk + (256 * j + 64 * wave) * 16), k_off + (uint32_t)j * 16u * kstride);
+    }
+    __syncthreads();  // waits for this group's DMA
+    f32x16 s[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s[t] = f32x16{};
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const u32x4 av = *(SA_LDS const u32x4*)(lk + ka[ds] + t * 8192);
+        s[t] = mfma32x32x16<CT>(av, qf[ds], s[t]);
+      }
+    if (key0 + 128 > a.Nk) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          if (key0 + t * 32 + tile_key(hl, j) >= a.Nk) s[t][j] = neg_inf();
+    }
+    if (RANGED ? __any(m_ref == neg_inf()) : kt == 0) {  // reference maximum from the first tile
+      float mx = neg_inf();
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[t][j]);
+      mx = max_xor32(mx) * c;
+      m_ref = RANGED && m_ref != neg_inf() ? m_ref : mx;
+    }
+    float ps[NS];
+    auto sums = [&]() {
+      const float ref = RANGED && m_ref == neg_inf() ? 0.f : m_ref;
+#pragma unroll
+      for (int i = 0; i < NS; ++i) ps[i] = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) ps[sub_block<KB>(t, j)] += fast_exp2(__builtin_fmaf(s[t][j], c, -ref));
+#pragma unroll
+      for (int i = 0; i < NS; ++i) ps[i] = sum_xor32(ps[i]);
+    };
+    sums();
+    float tot = 0.f;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) tot += ps[i];
+    if (!(tot <= kSumLimit)) {
+      // Rare: scores far above m_ref.  Move m_ref to this tile's maximum and rescale
+      // the row's earlier sums (the two lanes of the row split them by parity).
+      float mx = neg_inf();
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[t][j]);
+      mx = max_xor32(mx) * c;
+      const float f = fast_exp2(m_ref - mx);
+      for (int j = t0 * NS + hl; j < kt * NS; j += 2) ws[j * 128 + r] *= f;
+      l_tot *= f;
+      m_ref = mx;
+      sums();
+      tot = 0.f;
+#pragma unroll
+      for (int i = 0; i < NS; ++i) tot += ps[i];
+    }
+    l_tot += tot;
+    // the lanes of a row split the stores: lane half hl stores key blocks i = hl (mod 2)
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+      if ((NS == 1 ? hl == 0 : (i & 1) == hl) && kt * NS + i < nkb) ws[(kt * NS + i) * 128 + r] = ps[i];
+  }
+}
+
+template <int CT, int KB>
+__global__ __launch_bounds__(256, 3) void block_mass_persistent_kernel(PoolArgs a, int items) {
+  constexpr int NS = 128 / KB;
+  __shared__ u32x4 lds_k[2048];
+  __shared__ float row_inv[128];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, l32 = lane & 31;
+  const int nkb = a.nkb;
+  const int ntiles = (a.Nk + 127) >> 7;  // 128-key tiles
+  const int nqi = (a.Nq + 127) >> 7;
+  float* ws = a.ws + (size_t)blockIdx.x * (size_t)nkb * 128;
   const int r = wave * 32 + l32;
 
   for (int item = blockIdx.x; item < items; item += gridDim.x) {
     const int bh = item / nqi;
     const int qi = item - bh * nqi;
-    const int b = bh / a.H, h = bh - b * a.H;
-    const char* qbase = (const char*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1]) * 2;
-    const char* kbase = (const char*)a.k + ((int64_t)b * a.ks[0] + (int64_t)h * a.ks[1]) * 2;
     const int qrow = qi * 128 + r;
-    u32x4 qf[DS];
-    load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
-    float m_ref = neg_inf();
-    float l_tot = 0.f;
-
-    for (int kt = 0; kt < ntiles; ++kt) {
-      const int key0 = kt * 128;
-      __syncthreads();  // the previous tile (or item epilogue) is done with lds_k
-      {
-        const __amdgpu_buffer_rsrc_t rs =
-            make_rsrc(kbase + (int64_t)key0 * kstride, (uint32_t)(a.Nk - key0) * kstride);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          dma16(rs, (SA_LDS void*)(lk + (256 * j + 64 * wave) * 16), k_off + (uint32_t)j * 16u * kstride);
-      }
-      __syncthreads();  // waits for this group's DMA
-      f32x16 s[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) s[t] = f32x16{};
-#pragma unroll
-      for (int ds = 0; ds < DS; ++ds)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const u32x4 av = *(SA_LDS const u32x4*)(lk + ka[ds] + t * 8192);
-          s[t] = mfma32x32x16<CT>(av, qf[ds], s[t]);
-        }
-      if (key0 + 128 > a.Nk) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            if (key0 + t * 32 + tile_key(hl, j) >= a.Nk) s[t][j] = neg_inf();
-      }
-      if (kt == 0) {  // reference maximum from the first tile (key 0 always exists)
-        float mx = neg_inf();
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[t][j]);
-        m_ref = max_xor32(mx) * c;
-      }
-      float ps[NS];
-      auto sums = [&]() {
-#pragma unroll
-        for (int i = 0; i < NS; ++i) ps[i] = 0.f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) ps[sub_block<KB>(t, j)] += fast_exp2(__builtin_fmaf(s[t][j], c, -m_ref));
-#pragma unroll
-        for (int i = 0; i < NS; ++i) ps[i] = sum_xor32(ps[i]);
-      };
-      sums();
-      float tot = 0.f;
-#pragma unroll
-      for (int i = 0; i < NS; ++i) tot += ps[i];
-      if (!(tot <= kSumLimit)) {
-        // Rare: scores far above m_ref.  Move m_ref to this tile's maximum and rescale
-        // the row's earlier sums (the two lanes of the row split them by parity).
-        float mx = neg_inf();
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[t][j]);
-        mx = max_xor32(mx) * c;
-        const float f = fast_exp2(m_ref - mx);
-        for (int j = hl; j < kt * NS; j += 2) ws[j * 128 + r] *= f;
-        l_tot *= f;
-        m_ref = mx;
-        sums();
-        tot = 0.f;
-#pragma unroll
-        for (int i = 0; i < NS; ++i) tot += ps[i];
-      }
-      l_tot += tot;
-      // the lanes of a row split the stores: lane half hl stores key blocks i = hl (mod 2)
-#pragma unroll
-      for (int i = 0; i < NS; ++i)
-        if ((NS == 1 ? hl == 0 : (i & 1) == hl) && kt * NS + i < nkb) ws[(kt * NS + i) * 128 + r] = ps[i];
-    }
+    float m_ref, l_tot;
+    mass_tiles<CT, KB, false>(a, (SA_LDS char*)lds_k, item, 0, ntiles, ws, m_ref, l_tot);
 
     // Epilogue: out[qb][kb] = mean over the q-block's rows of ws[kb][row] / total(row); lane l
     // holds rows l and l + 64, so a q-block of KB rows is one group of KB lanes (KB < 64) or
@@ -196,6 +218,82 @@ __global__ __launch_bounds__(256, 3) void block_mass_persistent_kernel(PoolArgs 
           if (qb < a.nqb && rows > 0)
             out[((int64_t)bh * a.nqb + qb) * nkb + kb] = (half == 0 ? v0 : v1) / (float)rows;
         }
+      }
+    }
+  }
+}
+
+// The items of a partial round (all of them when they are fewer than the resident groups), whose
+// groups would leave the others idle: S groups per item, each a range of its key tiles.  Group
+// (item i, range s) writes its block sums to item i's slot and every row's reference and sum to
+// ml[i][s][2][128]; block_mass_combine_kernel puts the ranges together.
+// bf16, blocks of 128: [1,12,2048,128] 36 -> 26 us, [1,12,4096,128] 80 -> 64, [1,1,16000,128]
+// 239 -> 84, [1,7,16000,128] (875 items) 593 -> 514.
+template <int CT, int KB>
+__global__ __launch_bounds__(256, 3) void block_mass_ranged_kernel(PoolArgs a, int first, int n, int S, float* ml) {
+  __shared__ u32x4 lds_k[2048];
+  const int i = (int)blockIdx.x % n, s = (int)blockIdx.x / n;
+  const int ntiles = (a.Nk + 127) >> 7;
+  float m_ref, l_tot;
+  mass_tiles<CT, KB, true>(a, (SA_LDS char*)lds_k, first + i, s * ntiles / S, (s + 1) * ntiles / S,
+                           a.ws + (size_t)i * (size_t)a.nkb * 128, m_ref, l_tot);
+  const int lane = threadIdx.x & 63, r = (threadIdx.x >> 6) * 32 + (lane & 31);
+  if (lane < 32) {
+    float* p = ml + ((size_t)i * S + s) * 256;
+    p[r] = m_ref;
+    p[128 + r] = l_tot;
+  }
+}
+
+constexpr int kMassMaxRanges = 8;
+
+// Group (item, slice of the key blocks): the map entries of the item from its ranges' sums.
+template <int KB>
+__global__ __launch_bounds__(256) void block_mass_combine_kernel(PoolArgs a, int first, int S, const float* ml) {
+  constexpr int NS = 128 / KB, G = KB >= 64 ? 64 : KB;
+  __shared__ float f[kMassMaxRanges][128];  // range s, row: 2^(m_s - m) / total
+  const int i = blockIdx.x, item = first + i;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nkb = a.nkb, ntiles = (a.Nk + 127) >> 7, nqi = (a.Nq + 127) >> 7;
+  const int bh = item / nqi, qi = item - bh * nqi;
+  const float* p = ml + (size_t)i * S * 256;
+  if (tid < 128) {
+    float m = neg_inf(), l = 0.f;
+    for (int s = 0; s < S; ++s) m = fmaxf(m, p[s * 256 + tid]);
+    for (int s = 0; s < S; ++s) {
+      const float ms = p[s * 256 + tid];
+      const float e = ms == neg_inf() ? 0.f : fast_exp2(ms - m);
+      f[s][tid] = e;
+      l += p[s * 256 + 128 + tid] * e;
+    }
+    // a row without a finite score: 0 / 0, as in one range
+    const float inv = qi * 128 + tid >= a.Nq ? 0.f : (m == neg_inf() ? __builtin_nanf("") : 1.f / fmaxf(l, 1e-6f));
+    for (int s = 0; s < S; ++s) f[s][tid] = inv == 0.f ? 0.f : f[s][tid] * inv;
+  }
+  __syncthreads();
+  const float* ws = a.ws + (size_t)i * (size_t)nkb * 128;
+  float* out = reinterpret_cast<float*>(a.out);
+  for (int kb = blockIdx.y * 4 + wave; kb < nkb; kb += 4 * gridDim.y) {
+    const int s = ((kb / NS + 1) * S - 1) / ntiles;  // the range that holds this block's tile
+    float v0 = ws[(size_t)kb * 128 + lane] * f[s][lane], v1 = ws[(size_t)kb * 128 + 64 + lane] * f[s][lane + 64];
+    if constexpr (KB == 128) {
+      v0 += v1;
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) v0 += __shfl_xor(v0, off, 64);
+    } else {
+#pragma unroll
+      for (int off = G / 2; off >= 1; off >>= 1) {
+        v0 += __shfl_xor(v0, off, 64);
+        v1 += __shfl_xor(v1, off, 64);
+      }
+    }
+    if (lane % G == 0) {
+#pragma unroll
+      for (int half = 0; half < (KB == 128 ? 1 : 2); ++half) {
+        const int qb = qi * NS + half * (NS / 2 > 0 ? NS / 2 : 1) + lane / G;
+        const int rows = min(KB, a.Nq - qb * KB);
+        if (qb < a.nqb && rows > 0)
+          out[((int64_t)bh * a.nqb + qb) * nkb + kb] = (half == 0 ? v0 : v1) / (float)rows;
       }
     }
   }
@@ -958,6 +1056,51 @@ int device_cu_count() {
 int block_mass_groups() { return 3 * device_cu_count(); }
 int max_pool_groups() { return 4 * device_cu_count(); }
 
+// Split of a 16-bit call's last, partial round of items: `n` items in S ranges of at least
+// kMassMinTiles key tiles each (n = 0: none).  Only a first or second round: after two whole
+// rounds the persistent groups have drifted apart and cover a short last round themselves (items
+// in rounds of 768: 990 items 175 -> 172 us, 2698 898 -> 895, 3960 2198 -> 2242).  Four tiles: at
+// [1,12,1024,128] 17.8 -> 14.8 us in two ranges (a range of eight tiles would leave it whole).
+constexpr int kMassMinTiles = 4;
+
+struct MassSplit {
+  int n, S;
+};
+
+static MassSplit mass_split(int64_t items, int Nk) {
+  const int G = block_mass_groups();
+  const int n = (int)(items % G), tiles = (Nk + 127) / 128;
+  if (n == 0 || items >= 2 * (int64_t)G) return {0, 1};
+  int S = G / n;
+  S = min(min(S, kMassMaxRanges), tiles / kMassMinTiles);
+  return S >= 2 ? MassSplit{n, S} : MassSplit{0, 1};
+}
+
+size_t block_mass_workspace_floats(int64_t items, int64_t nkb, int64_t Nk) {
+  const int64_t groups = items < block_mass_groups() ? items : block_mass_groups();
+  const MassSplit sp = mass_split(items, (int)Nk);
+  return (size_t)(groups * nkb * 128 + (int64_t)sp.n * (sp.n > 0 ? sp.S : 0) * 256);
+}
+
+template <int CT, int KB>
+static hipError_t launch_mass(const PoolArgs& a, hipStream_t stream) {
+  const int items = a.B * a.H * ((a.Nq + 127) / 128);
+  const MassSplit sp = mass_split(items, a.Nk);
+  const int whole = items - sp.n;
+  if (whole > 0) {
+    block_mass_persistent_kernel<CT, KB><<<min(whole, block_mass_groups()), 256, 0, stream>>>(a, whole);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || sp.n == 0) return e;
+  }
+  float* ml = a.ws + (size_t)min(items, block_mass_groups()) * (size_t)a.nkb * 128;
+  block_mass_ranged_kernel<CT, KB><<<sp.n * sp.S, 256, 0, stream>>>(a, whole, sp.n, sp.S, ml);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int slices = min((a.nkb + 15) / 16, max(1, 1024 / sp.n));
+  block_mass_combine_kernel<KB><<<dim3(sp.n, slices), 256, 0, stream>>>(a, whole, sp.S, ml);
+  return hipGetLastError();
+}
+
 hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream) {
   (void)D;
   if (a.B * a.H * a.nqb == 0) return hipSuccess;
@@ -969,23 +1112,12 @@ hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream
       default: return launch_mass_f32<128>(a, stream);
     }
   }
-  const int items = a.B * a.H * ((a.Nq + 127) / 128);
-  const int groups = min(items, block_mass_groups());
-#define SA_MASS(KB)                                                                     \
-  do {                                                                                  \
-    if (dtype == kBF16)                                                                 \
-      block_mass_persistent_kernel<kBF16, KB><<<groups, 256, 0, stream>>>(a, items);    \
-    else                                                                                \
-      block_mass_persistent_kernel<kF16, KB><<<groups, 256, 0, stream>>>(a, items);     \
-  } while (0)
   switch (a.bs) {
-    case 16: SA_MASS(16); break;
-    case 32: SA_MASS(32); break;
-    case 64: SA_MASS(64); break;
-    default: SA_MASS(128); break;
+    case 16: return dtype == kBF16 ? launch_mass<kBF16, 16>(a, stream) : launch_mass<kF16, 16>(a, stream);
+    case 32: return dtype == kBF16 ? launch_mass<kBF16, 32>(a, stream) : launch_mass<kF16, 32>(a, stream);
+    case 64: return dtype == kBF16 ? launch_mass<kBF16, 64>(a, stream) : launch_mass<kF16, 64>(a, stream);
+    default: return dtype == kBF16 ? launch_mass<kBF16, 128>(a, stream) : launch_mass<kF16, 128>(a, stream);
   }
-#undef SA_MASS
-  return hipGetLastError();
 }
 
 hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream) {

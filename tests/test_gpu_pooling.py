@@ -290,6 +290,28 @@ def test_pooling_mode_dispatch():
     assert t.dtype == torch.float32 and t.shape == (1, 2, 2, 2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bs,H,Nq,Nk", [(128, 2, 1, 1024), (128, 3, 300, 1025), (64, 2, 1100, 4200), (32, 1, 130, 1500),
+                                        (16, 1, 257, 1281), (128, 85, 1200, 1100)])
+def test_exact_mass_key_ranges(dtype, bs, H, Nq, Nk):
+    """Items of a partial round split over key ranges: one to eight ranges, ragged ends, a round of
+    items plus a few (85 heads of 10), scores that rise past 2^64 in a later range, and a first
+    range whose scores are all -inf (no reference there).  The pooling bar of 1e-5."""
+    g = torch.Generator().manual_seed(bs + Nk)
+    q = 0.5 + 0.1 * torch.randn(1, H, Nq, 128, generator=g)
+    k = torch.randn(1, H, Nk, 128, generator=g)
+    for low in (None, -10.0, -math.inf):
+        if low == -math.inf and H > 8:
+            continue  # a whole round takes its reference from the first tile
+        kk = k.clone()
+        if low is not None:
+            kk[:, :, : Nk // 2] = low
+        qd, kd = q.to(dtype), kk.to(dtype)
+        ours = ops.block_mass_scores(qd.cuda(), kd.cuda(), block_size=bs)
+        heads = [0, H - 1]
+        _close(ours[:, heads], torch_ref.exact_block_mass(qd[:, heads], kd[:, heads], block_size=bs))
+
+
 # The fp32 matrix-core kernels (head dim 128, blocks 16-128): items of 64 rows (two to a
 # 128-row block), tiles of 32 keys (two blocks of 16 each), the last key counts before the row
 # values no longer fit LDS, keys whose rows overlap, and the 2^64 rescale.  Bar: the pooling
