@@ -573,10 +573,7 @@ int sinkattn_block_mass_pool(const void* q, const void* k, int dtype, int64_t B,
 size_t sinkattn_max_pool_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t block_size, int dtype) {
   if (dtype == SINKATTN_F32 || !mass_mfma_block(block_size)) return 0;
   const int64_t items = B * H * cdiv(N, 128);  // items of 128 query rows
-  const int64_t groups = items < sa::max_pool_groups() ? items : sa::max_pool_groups();
-  // per group: the rows' block maxima, and below block 128 the item's column maxima
-  const int64_t per_kb = 128 + (block_size == 128 ? 0 : 128 / block_size);
-  return (size_t)(groups * cdiv(N, block_size) * per_kb * (int64_t)sizeof(float));
+  return sa::max_pool_workspace_floats(items, cdiv(N, block_size), N, (int)block_size) * sizeof(float);
 }
 
 int sinkattn_max_pool(const void* q, const void* k, int dtype, int64_t B, int64_t H, int64_t Hk,

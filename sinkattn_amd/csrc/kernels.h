@@ -129,6 +129,7 @@ int device_cu_count();
 // Resident work-groups of the persistent max-pool kernel: its workspace holds one slot per
 // group, so the launch and the workspace query both use this count.
 int max_pool_groups();
+size_t max_pool_workspace_floats(int64_t items, int64_t nkb, int64_t N, int block_size);
 hipError_t launch_max_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
 int mean_pool_row_len(int D);
 hipError_t launch_mean_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);

@@ -312,6 +312,23 @@ def test_exact_mass_key_ranges(dtype, bs, H, Nq, Nk):
         _close(ours[:, heads], torch_ref.exact_block_mass(qd[:, heads], kd[:, heads], block_size=bs))
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bs,N", [(128, 1025), (128, 2300), (64, 1100), (32, 1281), (16, 1030)])
+def test_max_pool_key_ranges(dtype, bs, N, causal):
+    """Few items split over key ranges: the map of the whole-item kernel bit for bit (the same
+    heads repeated over a batch past the line), on ragged lengths, causal too."""
+    q, k = _qkd(1, 4, 2, N, N, 128, dtype, seed=bs + N, sinks=2)
+    qc, kc = q.cuda(), k.cuda()
+    few = ops.max_pool_scores(qc, kc, 0.0883, block_size=bs, causal=causal)
+    rep = 600 // (4 * (-(-N // 128))) + 1
+    many = ops.max_pool_scores(qc.expand(rep, -1, -1, -1), kc.expand(rep, -1, -1, -1), 0.0883, block_size=bs,
+                               causal=causal)
+    assert torch.equal(few, many[:1]) and torch.equal(few, many[-1:])
+    _max_pool_close(few.cpu(), torch_ref.max_pool_map(q, k, 0.0883, block_size=bs, causal=causal), q, k, 0.0883, bs,
+                    causal, what=f"{bs} {N}")
+
+
 # The fp32 matrix-core kernels (head dim 128, blocks 16-128): items of 64 rows (two to a
 # 128-row block), tiles of 32 keys (two blocks of 16 each), the last key counts before the row
 # values no longer fit LDS, keys whose rows overlap, and the 2^64 rescale.  Bar: the pooling
