@@ -504,8 +504,11 @@ bool pool_f32_mfma(const PoolArgs& a) {
 
 // The kernel's dynamic LDS and, where two items share a map entry, the zeroed map.
 static hipError_t f32_pool_setup(const void* kern, const PoolArgs& a, bool zero, size_t lds, hipStream_t stream) {
-  const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess || !zero) return e;
+  if (kF32StaticLds + lds > 64 * 1024) {  // past what a launch gets without asking
+    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  if (!zero) return hipSuccess;
   const int64_t n = (int64_t)a.B * a.H * a.nqb * a.nkb;
   fill_zero_kernel<<<(int)min((int64_t)1024, (n + 255) / 256), 256, 0, stream>>>((float*)a.out, n);
   return hipGetLastError();
@@ -683,6 +686,191 @@ __device__ __forceinline__ float round_to<kF16>(float x) {
 // the item's column maxima in LDS (nkb <= 1024); smaller blocks keep them after the
 // group's slot, in (128 / KB) * nkb floats of the workspace.
 // ------------------------------------------------------------------------------------
+template <int CT, int KB>
+__global__ __launch_bounds__(256, 4) void max_pool_persistent_kernel(PoolArgs a, int items) {
+  constexpr int DS = 8;
+  constexpr int NS = 128 / KB;  // key blocks per tile, q-blocks per item
+  __shared__ u32x4 lds_k[2048];
+  __shared__ float row_m[128];
+  __shared__ float colmax[KB == 128 ? 1024 : 1];
+  __shared__ float total_sh[KB == 128 ? 1 : 4];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hl = lane >> 5, l32 = lane & 31;
+  const int nkb = a.nkb;
+  const int ntiles = (a.Nk + 127) >> 7;
+  const int nqi = (a.Nq + 127) >> 7;
+  float* ws = a.ws + (size_t)blockIdx.x * (size_t)nkb * (128 + (KB == 128 ? 0 : NS));
+  float* cm = ws + (size_t)nkb * 128;  // [NS][nkb] column maxima (KB < 128)
+  const uint32_t kstride = (uint32_t)a.ks[2] * 2;
+  const int drow = 4 * wave + (lane >> 4);
+  const uint32_t k_off = (uint32_t)drow * kstride + (uint32_t)(((lane & 15) ^ (drow & 15)) * 16);
+  const int prow = k_row_perm(l32);
+  // chunk (2ds + hl) ^ (prow & 15) of row prow: the k-step only flips bits 5-7
+  const uint32_t ka0 = (uint32_t)(prow * 256 + ((hl ^ (prow & 15)) * 16));
+  SA_LDS char* lk = (SA_LDS char*)lds_k;
+  // The reference forms qk_scale = fp32(sm_scale) * fp32(1.44269504).
+  const float qk_scale = a.scale * 1.44269504f;
+  const int r = wave * 32 + l32;
+
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int bh = item / nqi;
+    const int qi = item - bh * nqi;
+    const int b = bh / a.H, h = bh - b * a.H;
+    const int hk = h / (a.H / a.Hk);
+    const int kt_end = a.causal ? min(ntiles, qi + 1) : ntiles;
+    const int kb_item = a.causal ? min(nkb, (qi + 1) * NS) : nkb;  // key blocks any row of the item sees
+    const char* qbase = (const char*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1]) * 2;
+    const char* kbase = (const char*)a.k + ((int64_t)b * a.ks[0] + (int64_t)hk * a.ks[1]) * 2;
+    const int qrow = qi * 128 + r;
+    const int qbr = qrow / KB;  // this row's q-block
+    u32x4 qf[DS];
+    load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
+    float m = neg_inf();
+
+    for (int kt = 0; kt < kt_end; ++kt) {
+      const int key0 = kt * 128;
+      __syncthreads();  // the previous tile (or item epilogue) is done with lds_k
+      {
+        const __amdgpu_buffer_rsrc_t rs =
+            make_rsrc(kbase + (int64_t)key0 * kstride, (uint32_t)(a.Nk - key0) * kstride);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          dma16(rs, (SA_LDS void*)(lk + (256 * j + 64 * wave) * 16), k_off + (uint32_t)j * 16u * kstride);
+      }
+      __syncthreads();  // waits for this group's DMA
+      f32x16 s[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s[t] = f32x16{};
+      {
+        // Flat step i = 4 ds + t.  The read for step i + 2 is issued right after the MFMA
+        // of step i (the scheduling groups pin that order), so each read has two MFMAs to
+        // land; a deeper ring does not fit the 128 VGPRs of four groups per CU.
+        u32x4 kr[4];
+        auto kread = [&](int i) __attribute__((always_inline)) {
+          return *(SA_LDS const u32x4*)(lk + (ka0 ^ (32u * (i >> 2))) + (i & 3) * 8192);
+        };
+        kr[0] = kread(0);
+        kr[1] = kread(1);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+        for (int i = 0; i < 4 * DS; ++i) {
+          s[i & 3] = mfma32x32x16<CT>(kr[i & 3], qf[i >> 2], s[i & 3]);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (i + 2 < 4 * DS) {
+            kr[(i + 2) & 3] = kread(i + 2);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+        }
+      }
+      const bool diag = a.causal && kt == qi;
+      if (key0 + 128 > a.Nk || diag) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int key = key0 + t * 32 + tile_key(hl, j);
+            if (diag) {
+              const int kbk = key / KB;
+              if (kbk == qbr && qrow < key) s[t][j] += -1.0e6f;
+              if (kbk > qbr) s[t][j] = neg_inf();  // a key block past the row's own: not seen
+            }
+            if (key >= a.Nk) s[t][j] = neg_inf();
+          }
+      }
+      float mx[NS];
+#pragma unroll
+      for (int i = 0; i < NS; ++i) mx[i] = neg_inf();
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx[sub_block<KB>(t, j)] = fmaxf(mx[sub_block<KB>(t, j)], s[t][j]);
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        mx[i] = max_xor32(mx[i]) * qk_scale;
+        m = fmaxf(m, mx[i]);
+        if ((NS == 1 ? hl == 0 : (i & 1) == hl) && kt * NS + i < nkb) ws[(kt * NS + i) * 128 + r] = round_to<CT>(mx[i]);
+      }
+    }
+
+    // Epilogue.  Rows past the end of the sequence take no part (m = +inf gives 0).
+    if (hl == 0) row_m[r] = (qrow < a.Nq) ? m : pos_inf();
+    __syncthreads();
+    const float m0 = row_m[lane], m1 = row_m[lane + 64];
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(ws, (uint32_t)nkb * 512u);
+    if constexpr (KB == 128) {
+      for (int kb = wave; kb < kb_item; kb += 4) {
+        // coherent (L1-bypassing) loads of values other waves of the group wrote
+        const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
+        const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
+        float v = fmaxf(fast_exp2(x0 - m0), fast_exp2(x1 - m1));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+        if (lane == 0) colmax[kb] = round_to<CT>(v);
+      }
+      __syncthreads();
+      // Row normalisation in q.dtype: sum (fp32 accumulate, rounded), then divide.
+      if (wave == 0) {
+        float part = 0.f;
+        for (int kb = lane; kb < kb_item; kb += 64) part += colmax[kb];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+        if (lane == 0) total_sh[0] = round_to<CT>(part);
+      }
+      __syncthreads();
+      const float total = total_sh[0];
+      uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qi) * nkb;
+      for (int kb = tid; kb < nkb; kb += 256) {
+        const float v = kb < kb_item ? colmax[kb] / total : 0.f;
+        out[kb] = (uint16_t)(pack2<CT>(v, 0.f) & 0xffffu);
+      }
+    } else {
+      // Pass 1: column maxima of every (q-block, key block) of the item into cm[qs][kb]:
+      // lane l holds rows l and l + 64, so a q-block is a group of KB lanes (KB < 64) or a
+      // whole half (KB = 64).
+      constexpr int G = KB >= 64 ? 64 : KB;
+      for (int kb = wave; kb < kb_item; kb += 4) {
+        const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
+        const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
+        float v0 = fast_exp2(x0 - m0), v1 = fast_exp2(x1 - m1);
+#pragma unroll
+        for (int off = G / 2; off >= 1; off >>= 1) {
+          v0 = fmaxf(v0, __shfl_xor(v0, off, 64));
+          v1 = fmaxf(v1, __shfl_xor(v1, off, 64));
+        }
+        if (lane % G == 0) {
+          const int g = lane / G;
+          cm[(size_t)g * nkb + kb] = round_to<CT>(v0);
+          cm[(size_t)(NS / 2 + g) * nkb + kb] = round_to<CT>(v1);
+        }
+      }
+      __syncthreads();  // the column maxima are in memory (the barrier drains this group's stores)
+      // Pass 2: per q-block (one wave each), the row total in q.dtype, then the division.
+      const __amdgpu_buffer_rsrc_t crs = make_rsrc(cm, (uint32_t)(NS * nkb) * 4u);
+      for (int qs = wave; qs < NS; qs += 4) {
+        const int qb = qi * NS + qs;
+        if (qb >= a.nqb) continue;
+        const int kb_end = a.causal ? min(nkb, qb + 1) : nkb;
+        float part = 0.f;
+        for (int kb = lane; kb < kb_end; kb += 64)
+          part += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+        const float total = round_to<CT>(part);
+        uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qb) * nkb;
+        for (int kb = lane; kb < nkb; kb += 64) {
+          const float cv = kb < kb_end ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                              crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1))
+                                       : 0.f;
+          out[kb] = (uint16_t)(pack2<CT>(kb < kb_end ? cv / total : 0.f, 0.f) & 0xffffu);
+        }
+      }
+    }
+  }
+}
+
+// The parts of that kernel for items split over key ranges (called from the persistent loop, they
+// made it 1% slower at the Wan layer).
 // 128-key tiles that any row of item `qi` of a head sees.
 template <int KB>
 __device__ __forceinline__ int max_pool_tiles(const PoolArgs& a, int qi) {
@@ -871,28 +1059,6 @@ __device__ __forceinline__ void max_pool_rows(const PoolArgs& a, int item, float
         out[kb] = (uint16_t)(pack2<CT>(kb < kb_end ? cv / total : 0.f, 0.f) & 0xffffu);
       }
     }
-  }
-}
-
-template <int CT, int KB>
-__global__ __launch_bounds__(256, 4) void max_pool_persistent_kernel(PoolArgs a, int items) {
-  constexpr int NS = 128 / KB;
-  __shared__ u32x4 lds_k[2048];
-  __shared__ float row_m[128];
-  __shared__ float colmax[KB == 128 ? 1024 : 1];
-  __shared__ float total_sh[KB == 128 ? 1 : 4];
-  const int lane = threadIdx.x & 63, r = (threadIdx.x >> 6) * 32 + (lane & 31);
-  const int nqi = (a.Nq + 127) >> 7;
-  float* ws = a.ws + (size_t)blockIdx.x * (size_t)a.nkb * (128 + (KB == 128 ? 0 : NS));
-  float* cm = ws + (size_t)a.nkb * 128;  // [NS][nkb] column maxima (KB < 128)
-  for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int qi = item % nqi;
-    float m;
-    max_pool_walk<CT, KB>(a, (SA_LDS char*)lds_k, item, 0, max_pool_tiles<KB>(a, qi), ws, m);
-    // Rows past the end of the sequence take no part (m = +inf gives 0).
-    if (lane < 32) row_m[r] = qi * 128 + r < a.Nq ? m : pos_inf();
-    __syncthreads();
-    max_pool_rows<CT, KB>(a, item, ws, cm, row_m, colmax, total_sh);
   }
 }
 
@@ -1125,8 +1291,12 @@ int max_pool_groups() { return 4 * device_cu_count(); }
 // kMassMinTiles key tiles each (n = 0: none).  Only a first or second round: after two whole
 // rounds the persistent groups have drifted apart and cover a short last round themselves (items
 // in rounds of 768: 990 items 175 -> 172 us, 2698 898 -> 895, 3960 2198 -> 2242).  Four tiles: at
-// [1,12,1024,128] 17.8 -> 14.8 us in two ranges (a range of eight tiles would leave it whole).
+// [1,4,2048,128] 30 -> 17 us in four ranges, 22 in the two that eight tiles would allow.
 constexpr int kMassMinTiles = 4;
+// Key tiles from which a call is split.  Below, the second launch costs a program that records
+// call after call as much as the ranges save: max-pool at [1,9,1847,128] 28 -> 22 us on the GPU,
+// but 37.5 -> 41 us per recorded call.
+constexpr int kMassSplitTiles = 16, kMaxSplitTiles = 24;
 
 struct MassSplit {
   int n, S;
@@ -1135,7 +1305,7 @@ struct MassSplit {
 static MassSplit mass_split(int64_t items, int Nk) {
   const int G = block_mass_groups();
   const int n = (int)(items % G), tiles = (Nk + 127) / 128;
-  if (n == 0 || items >= 2 * (int64_t)G) return {0, 1};
+  if (n == 0 || items >= 2 * (int64_t)G || tiles < kMassSplitTiles) return {0, 1};
   int S = G / n;
   S = min(min(S, kMassMaxRanges), tiles / kMassMinTiles);
   return S >= 2 ? MassSplit{n, S} : MassSplit{0, 1};
@@ -1190,7 +1360,7 @@ hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream
 // 129.2), half a round below, whose longer map rows the join spreads (504 at 64: 160 -> 143).
 static int max_split(int64_t items, int Nk, int block_size) {
   const int G = max_pool_groups();
-  if (items <= 0 || items > (block_size == 128 ? 2 * G / 5 : G / 2)) return 1;
+  if (items <= 0 || items > (block_size == 128 ? 2 * G / 5 : G / 2) || (Nk + 127) / 128 < kMaxSplitTiles) return 1;
   return max(1, min(min((int)(max_pool_groups() / items), kMassMaxRanges), (Nk + 127) / 128 / kMassMinTiles));
 }
 
