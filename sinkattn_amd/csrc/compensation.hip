@@ -30,8 +30,9 @@ namespace sa {
 // (row r, chunk c) sums chunk c of the input rows of r in order, eight loads in flight.  Rows
 // before `prefix` and from `pool_end` on are copied.  Bound by the read of the input: K and V of
 // [2,12,32760,128] bf16 in groups of 30 take 73 us, 5.7 TB/s (77 us as two launches with the
-// loads of a group left to the compiler); the 4096 image rows and 224 text rows of 30 heads 13 us
-// (2 x 14.7 us, and 2 x 8 us to concatenate the text rows).
+// loads of a group left to the compiler); the 4096 image rows and 224 text rows of 30 heads
+// 13 us contiguous, 15 in the layer's [N,H,D] layout (2 x 14.7 us, and 2 x 8 us to concatenate
+// the text rows).
 // ---------------------------------------------------------------------------------------
 template <int IT>
 __device__ __forceinline__ void add_chunk(float* acc, u32x4 w) {

@@ -1065,8 +1065,8 @@ __device__ __forceinline__ void max_pool_rows(const PoolArgs& a, int item, float
 // Items of a first, partial round, whose groups would leave the others idle: S groups per item,
 // each a range of its key tiles; group (item i, range s) writes its block maxima to item i's slot
 // and its rows' maxima to ml[i][s][128].  max_pool_join_kernel makes the map rows: maxima do not
-// depend on the split, so the map is the same bit for bit.  bf16, blocks of 128: [1,12,2048,128]
-// 28.5 -> 22.9 us, [1,4,2048,128] 21.3 -> 13.0, [1,1,16000,128] 166 -> 81.
+// depend on the split, so the map is the same bit for bit.  bf16: [1,12,4096,128] 60 -> 56 us at
+// blocks of 128 and 78 -> 64 at 64, [1,1,16000,128] 166 -> 81.
 template <int CT, int KB>
 __global__ __launch_bounds__(256, 4) void max_pool_ranged_kernel(PoolArgs a, int n, int S, float* ml) {
   constexpr int NS = 128 / KB;
