@@ -286,6 +286,11 @@ constexpr float kMassLimitLog2 = 64.f;
 
 template <int D, int MODE>
 constexpr bool kMfmaSums = D == 128 && MODE == kSparse;
+// How far (log2 units) a tile's maximum may pass the reference point before it moves.  Head dims 64
+// and 32 and the dense forms follow the maximum at once: the largest P is then exactly 1 (a lagging
+// reference put their outputs 2-5% further from the 64-bit ones).
+template <int D, int MODE>
+constexpr float kRescaleMargin = D == 128 && MODE == kSparse ? kLazyRescaleLog2 : 0.f;
 
 template <int MODE>
 struct MassState {};
@@ -358,7 +363,7 @@ __device__ __forceinline__ void attn_tile(SA_LDS char* lk, SA_LDS char* lv, cons
       for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][qt][i]);
     mx = max_col16(mx);
     const float m_tile = __builtin_fmaf(mx, c, bias);
-    if (m_tile > m_run[qt] + (MODE == kSparse ? kLazyRescaleLog2 : 0.f)) {
+    if (m_tile > m_run[qt] + kRescaleMargin<D, MODE>) {
       const float alpha = fast_exp2(m_run[qt] - m_tile);
       l_acc[qt] *= alpha;
 #pragma unroll
@@ -806,7 +811,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_split_kernel(FwdArgs 
 #pragma unroll
           for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][qt][i]);
         const float m_tile = __builtin_fmaf(max_col16(mx), c, bias);
-        if (m_tile > m_run[qt] + kLazyRescaleLog2) {
+        if (m_tile > m_run[qt] + kRescaleMargin<D, kSparse>) {
           const float alpha = fast_exp2(m_run[qt] - m_tile);
           l_acc[qt] *= alpha;
 #pragma unroll
