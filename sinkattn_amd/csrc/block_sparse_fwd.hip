@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
   f32x16 o[DT];
 #pragma unroll
   for (int i = 0; i < DT; ++i) o[i] = f32x16{};
-  float m_run = neg_inf();
+  float m_run = lowest();
   float l_run = 0.f;
   const float c = a.scale * kLog2e;
 
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
   }
 
   const float l = sum_xor32(l_run);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = cnt > 0 ? 1.f / l : 0.f;  // a sum of 0 over listed keys: NaN
   if (qrow < a.Nq) {
     char* obase = (char*)a.out +
                   ((int64_t)b * a.os[0] + (int64_t)h * a.os[1] + (int64_t)qrow * a.os[2]) * ES;
@@ -516,7 +516,10 @@ __device__ __forceinline__ void store_o_staged(const FwdArgs& a, const AttnItem&
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     l[qt] = kMfmaSums<D, MODE> ? l_acc[qt][0] : sum_col16(l_acc[qt][0]);
-    inv[qt] = l[qt] > 0.f ? 1.f / l[qt] : 0.f;
+    // A sum of 0 over listed keys (every score -inf): NaN, as a softmax gives; the dense forms give
+    // 0 there, as the flash attention they take the place of.
+    const bool some = MODE == kSparse ? it.ntot > 0 : l[qt] > 0.f;
+    inv[qt] = some ? 1.f / l[qt] : 0.f;
   }
   SA_LDS char* ob = buf + wave * (64 * D);
 #pragma unroll
@@ -592,7 +595,7 @@ __device__ __forceinline__ void fwd_qblock(const FwdArgs& a, SA_LDS char* lk, SA
     o[dt][0] = f32x4{};
     o[dt][1] = f32x4{};
   }
-  float m_run[2] = {neg_inf(), neg_inf()};
+  float m_run[2] = {lowest(), lowest()};
   f32x4 l_acc[2] = {f32x4{}, f32x4{}};
   MassState<MODE> mass;
   if constexpr (MODE == kDenseMass) {

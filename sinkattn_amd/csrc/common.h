@@ -23,6 +23,9 @@ constexpr float kLn2 = 0.6931471805599453f;
 
 __device__ __forceinline__ float neg_inf() { return -__builtin_inff(); }
 __device__ __forceinline__ float pos_inf() { return __builtin_inff(); }
+// The lowest finite float: a softmax's reference point before its row has seen a finite score.
+// Scores of -inf then get the weight exp2(-inf) = 0 (against a reference of -inf it is NaN).
+__device__ __forceinline__ float lowest() { return -__FLT_MAX__; }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 

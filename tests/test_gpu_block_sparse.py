@@ -332,6 +332,47 @@ def test_few_and_many_q_blocks(dtype, D, Nq, Nk):
             assert ((lse[-1:].cpu() - ref_l)[fin].abs() <= LSE_ABS + 1e-5 * ref_l[fin].abs()).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_first_tile_of_minus_infinity(dtype, D):
+    """A first listed tile whose scores are all -inf weighs nothing, in the split kernel, the
+    whole-q-block kernels, the overlapping-row kernel (broadcast keys) and the dense forms; rows
+    whose every score is -inf are NaN (a softmax of them) with an lse of -inf, and 0 in the dense
+    forms, as scaled_dot_product_attention gives."""
+    q, k, v = _inputs(1, 2, 256, 417, D, dtype, seed=D)
+    q = q.abs()
+    k[:, 0, :128] = -math.inf
+    k[:, 1] = -math.inf
+    mask = _random_mask(1, 2, 2, 4, 0.6, seed=9)
+    ref_o, ref_l = torch_ref.dense_masked_attention(q, k, v, mask)
+
+    def close(out, lse):
+        assert torch.isnan(out[:, 1]).all() and (lse[:, 1] == -math.inf).all()
+        err = (out[:, 0].float().cpu() - ref_o[:, 0]).abs()
+        assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS
+        assert ((lse[:, 0].cpu() - ref_l[:, 0]).abs() <= LSE_ABS + 1e-5 * ref_l[:, 0].abs()).all()
+
+    for rep in (1, 80):  # 4 and 320 q-blocks
+        qr, kr, vr, mr = (t.expand(rep, -1, -1, -1) for t in (q, k, v, mask))
+        out, lse = ops.block_sparse_attention(qr, kr, vr, ops.block_sparse_plan(mr.contiguous()))
+        close(out[-1:], lse[-1:])
+    if D < 128:
+        inf = k[:, 1:, :1].expand(-1, 2, 417, -1)
+        out, lse = ops.block_sparse_attention(q, inf, v[:, :, :1].expand(-1, -1, 417, -1), ops.block_sparse_plan(mask))
+        assert torch.isnan(out).all() and (lse == -math.inf).all()
+        return
+    want = torch.nn.functional.scaled_dot_product_attention(q, k, v)
+    full = torch_ref.dense_masked_attention(q[:, :1], k[:, :1], v[:, :1], torch.ones(1, 1, 2, 4, dtype=torch.bool))[0]
+    for out in (ops.dense_attention(q, k, v)[0], ops.dense_attention_mass(q, k, v)[0]):
+        assert torch.equal(out[:, 1], want[:, 1]) and not torch.isnan(want).any()
+        err = (out[:, :1].float().cpu() - full).abs()
+        assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS
+    mass = ops.dense_attention_mass(q, k, v)[1]
+    ref = torch_ref.exact_block_mass(q, k)
+    assert torch.equal(torch.isnan(mass.cpu()), torch.isnan(ref)) and torch.isnan(ref[:, 1]).all()
+    assert ((mass.cpu() - ref)[:, 0].abs() <= 1e-8 + 1e-5 * ref[:, 0].abs()).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("D,B,N", [(128, 1, 300), (128, 60, 300), (64, 1, 300), (64, 100, 300), (32, 2, 129)])
 def test_lse_in_the_operands_type(dtype, D, B, N):
