@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_f32_kernel(FwdArgs a)
   f32x4 o[DT][2];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt][0] = o[dt][1] = f32x4{};
-  float m_run[2] = {neg_inf(), neg_inf()}, l_run[2] = {0.f, 0.f};
+  float m_run[2] = {lowest(), lowest()}, l_run[2] = {0.f, 0.f};
 
   // two steps per listed block; a last block of at most 64 keys is one
   int steps = 2 * cnt;
@@ -1156,7 +1156,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_f32_kernel(FwdArgs a)
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     const float l = sum_col16(l_run[qt]);
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const float inv = cnt > 0 ? 1.f / l : 0.f;  // a sum of 0 over listed keys: NaN
     const int qrow = qb * 128 + wave * 32 + 16 * qt + sl;
     if (qrow >= a.Nq) continue;
     float* obase = (float*)a.out + ((int64_t)b * a.os[0] + (int64_t)h * a.os[1] + (int64_t)qrow * a.os[2]);

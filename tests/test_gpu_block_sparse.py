@@ -259,6 +259,26 @@ def test_f32_steps_edges(D, Nq, Nk, layout):
         assert (lse.cpu() - ref_l)[fin].abs().max() <= 1e-4
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("inf_keys", [64, 128])
+def test_f32_first_step_of_minus_infinity(D, inf_keys):
+    """fp32: a first step of 64 keys (and a whole first block) whose scores overflow to -inf weighs
+    nothing; rows without a finite score are NaN with an lse of -inf.  The keys are -3e38 in one
+    channel, where the queries are 4 (an infinite key has no finite remainder to split).  Bars of
+    test_f32_steps_edges."""
+    q, k, v = _inputs(1, 2, 200, 300, D, torch.float32, seed=D)
+    q[..., 0] = 4.0
+    k[:, 0, :inf_keys, 0] = -3e38
+    k[:, 1, :, 0] = -3e38
+    mask = _random_mask(1, 2, 2, 3, 0.6, seed=9)
+    ref_o, ref_l = torch_ref.dense_masked_attention(q, k, v, mask)
+    assert torch.isfinite(ref_o[:, 0]).all() and torch.isnan(ref_o[:, 1]).all()
+    out, lse = ops.block_sparse_attention(q, k, v, ops.block_sparse_plan(mask))
+    assert torch.isnan(out[:, 1]).all() and (lse[:, 1] == -math.inf).all()
+    assert (out.cpu() - ref_o)[:, 0].abs().max() <= 2e-4
+    assert (lse.cpu() - ref_l)[:, 0].abs().max() <= 1e-4
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Nq,Nk,layout", [(1, 1, "bhsd"), (130, 129, "bshd"), (700, 1500, "bhsd"), (1029, 640, "bshd")])
 def test_dense_forms(dtype, Nq, Nk, layout):
