@@ -45,6 +45,11 @@ namespace sa {
 // ------------------------------------------------------------------------------------
 constexpr float kSumLimit = 1.8446744073709552e19f;  // 2^64
 
+// A row's normalisation: 1 / total, NaN without a finite score (a total of 0).
+__device__ __forceinline__ float row_factor(float total) {
+  return total == 0.f ? __builtin_nanf("") : 1.f / fmaxf(total, 1e-6f);
+}
+
 template <int KB>
 __device__ __forceinline__ constexpr int sub_block(int t, int j) {
   return KB == 16 ? 2 * t + (j >> 3) : (t * 32) / KB;
@@ -113,13 +118,14 @@ __device__ __forceinline__ void mass_tiles(const PoolArgs& a, SA_LDS char* lk, i
           if (key0 + t * 32 + tile_key(hl, j) >= a.Nk) s[t][j] = neg_inf();
     }
     if (RANGED ? __any(m_ref == neg_inf()) : kt == 0) {  // reference maximum from the first tile
+      // (the lowest float when its scores are all -inf: a later tile's sum then passes the limit)
       float mx = neg_inf();
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[t][j]);
       mx = max_xor32(mx) * c;
-      m_ref = RANGED && m_ref != neg_inf() ? m_ref : mx;
+      m_ref = RANGED ? (m_ref != neg_inf() ? m_ref : mx) : fmaxf(mx, lowest());
     }
     float ps[NS];
     auto sums = [&]() {
@@ -187,7 +193,7 @@ __global__ __launch_bounds__(256, 3) void block_mass_persistent_kernel(PoolArgs 
     // Epilogue: out[qb][kb] = mean over the q-block's rows of ws[kb][row] / total(row); lane l
     // holds rows l and l + 64, so a q-block of KB rows is one group of KB lanes (KB < 64) or
     // a whole half (KB = 64) or both halves (KB = 128).
-    if (hl == 0) row_inv[r] = (qrow < a.Nq) ? 1.f / fmaxf(l_tot, 1e-6f) : 0.f;
+    if (hl == 0) row_inv[r] = (qrow < a.Nq) ? row_factor(l_tot) : 0.f;
     __syncthreads();
     const float inv0 = row_inv[lane], inv1 = row_inv[lane + 64];
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(ws, (uint32_t)nkb * 512u);
@@ -425,7 +431,9 @@ __global__ __launch_bounds__(256, 3) void block_mass_f32_kernel(PoolArgs a, int 
           if (!cut || 16 * kt + i < left) mx = fmaxf(mx, s[kt][i] * c);
       return max_col16(mx);
     };
-    if (t == 0) m_ref = row_max();  // key 0 always exists
+    // key 0 always exists; a first tile whose scores are all -inf leaves the lowest float, and the
+    // first finite score's tile then passes the limit below
+    if (t == 0) m_ref = fmaxf(row_max(), lowest());
     float ps[2];
     auto tile_sums = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -467,7 +475,7 @@ __global__ __launch_bounds__(256, 3) void block_mass_f32_kernel(PoolArgs a, int 
     if (t + 1 < ntiles) tile(t + 1, (SA_LDS char*)lds_k1, (SA_LDS char*)lds_k0);
   }
 
-  if (g == 0) row_inv[r] = qrow < a.Nq ? 1.f / fmaxf(l_tot, 1e-6f) : 0.f;
+  if (g == 0) row_inv[r] = qrow < a.Nq ? row_factor(l_tot) : 0.f;
   __syncthreads();
   // Map entries: the mean over a q-block's rows of sum / total.
   constexpr int RB = KB < kF32Rows ? KB : kF32Rows;  // rows of this item in one q-block

@@ -312,6 +312,28 @@ def test_exact_mass_key_ranges(dtype, bs, H, Nq, Nk):
         _close(ours[:, heads], torch_ref.exact_block_mass(qd[:, heads], kd[:, heads], block_size=bs))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("bs", [16, 32, 64, 128])
+@pytest.mark.parametrize("H,B", [(2, 1), (4, 200)])
+def test_exact_mass_first_tile_of_minus_infinity(dtype, bs, H, B):
+    """A first tile (32 keys in fp32, 128 in 16 bits) whose scores are all -inf weighs nothing, in calls
+    of few items and of more than a round of them (the last batch entry is compared); rows without
+    a finite score are NaN, as the oracle's.  The pooling bar of 1e-5."""
+    g = torch.Generator().manual_seed(bs)
+    q = torch.randn(1, H, 128, 128, generator=g)
+    k = torch.randn(1, H, 400, 128, generator=g)
+    q[..., 0] = 4.0
+    low = -3e38 if dtype == torch.float32 else -math.inf
+    k[:, 0, :32 if dtype == torch.float32 else 128, 0] = low
+    k[:, 1, :, 0] = low
+    q, k = q.to(dtype), k.to(dtype)
+    ref = torch_ref.exact_block_mass(q, k, block_size=bs)
+    ours = ops.block_mass_scores(q.cuda().expand(B, -1, -1, -1), k.cuda().expand(B, -1, -1, -1), block_size=bs).cpu()[-1:]
+    assert torch.isnan(ref[:, 1]).all() and torch.isnan(ours[:, 1]).all()
+    rest = [h for h in range(H) if h != 1]
+    assert ((ours - ref)[:, rest].abs() <= ATOL + RTOL * ref[:, rest].abs()).all()
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bs,N", [(128, 3073), (128, 3300), (64, 3100), (32, 3201), (16, 3075)])
