@@ -579,15 +579,16 @@ __device__ __forceinline__ void fwd_qblock(const FwdArgs& a, SA_LDS char* lk, SA
   const uint32_t kstride = (uint32_t)a.ks[2] * 2, vstride = (uint32_t)a.vs[2] * 2;
   const TileLanes<D> L = tile_lanes<D>(wave, lane, kstride, vstride);
 
-  // Q^T B operands: query 16 qt + l % 16 of the wave's rows, d slice 32 ks + 8 (l / 16)
+  // Q^T B operands: query 16 qt + l % 16 of the wave's rows, d slice 32 ks + 8 (l / 16).  Rows past
+  // the end repeat the last one: their outputs are not stored, and their map rows have the factor 0
+  // (0 times what zeros would make of an infinite key is NaN).
   u32x4 qf[2][D / 32];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
-    const int qrow = it.qb * 128 + wave * 32 + 16 * qt + sl;
+    const int qrow = min(it.qb * 128 + wave * 32 + 16 * qt + sl, a.Nq - 1);
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks)
-      qf[qt][ks] = qrow < a.Nq ? *(const u32x4*)(it.qbase + ((int64_t)qrow * a.qs[2] + 32 * ks + 8 * g) * 2)
-                               : u32x4{0, 0, 0, 0};
+      qf[qt][ks] = *(const u32x4*)(it.qbase + ((int64_t)qrow * a.qs[2] + 32 * ks + 8 * g) * 2);
   }
   f32x4 o[D / 16][2];
 #pragma unroll

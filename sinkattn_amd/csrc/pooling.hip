@@ -85,7 +85,9 @@ __device__ __forceinline__ void mass_tiles(const PoolArgs& a, SA_LDS char* lk, i
   const char* kbase = (const char*)a.k + ((int64_t)b * a.ks[0] + (int64_t)h * a.ks[1]) * 2;
   const int qrow = qi * 128 + r;
   u32x4 qf[DS];
-  load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
+  // rows past the end repeat the last one: their factor is 0, and 0 times what zeros would make of
+  // an infinite key is NaN
+  load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], min(qrow, a.Nq - 1), a.Nq, hl);
   m_ref = neg_inf();
   l_tot = 0.f;
 
@@ -350,10 +352,11 @@ struct F32Tiles {
     doff[0] = (uint32_t)drow * kstride + (uint32_t)(((lane & 31) ^ drow) * 16);
     doff[1] = (uint32_t)drow * kstride + (uint32_t)(((lane & 31) ^ (drow + 8)) * 16);
     ka = (uint32_t)(sl * 512 + ((g ^ sl) * 16));  // chunk 4 j + g: XOR 64 j
-    const float* q = (const float*)a.q + ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1] + (int64_t)qrow * a.qs[2]);
+    // rows past the end repeat the last one (as in the 16-bit kernel)
+    const float* q = (const float*)a.q +
+                     ((int64_t)b * a.qs[0] + (int64_t)h * a.qs[1] + (int64_t)min(qrow, a.Nq - 1) * a.qs[2]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      qv[j] = qrow < a.Nq ? *reinterpret_cast<const f32x4*>(q + 16 * j + 4 * g) : f32x4{};
+    for (int j = 0; j < 8; ++j) qv[j] = *reinterpret_cast<const f32x4*>(q + 16 * j + 4 * g);
   }
 
   __device__ __forceinline__ void copy(SA_LDS char* dst, int t) const {

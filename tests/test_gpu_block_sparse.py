@@ -312,6 +312,17 @@ def test_dense_mass_reference_moves():
            torch.ones(1, 2, 4, 12, dtype=torch.bool).cuda())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Nq", [1, 130, 383])
+def test_dense_mass_infinite_keys_and_ragged_rows(dtype, Nq):
+    """Keys of -inf and a last q-block that is not full: the rows past the end add nothing to its map."""
+    q, k, v = _inputs(1, 2, Nq, 500, 128, dtype, seed=Nq)
+    q = q.abs() + 0.5
+    k[:, :, 64:300] = -math.inf
+    mass, ref = ops.dense_attention_mass(q, k, v)[1].cpu(), torch_ref.exact_block_mass(q, k)
+    assert ((mass - ref).abs() <= 1e-8 + 1e-5 * ref.abs()).all()
+
+
 def test_dense_mass_in_several_launches():
     # more heads than one launch's workspace holds (2 GiB of row sums): the heads at the seam
     # against the pooling kernel's own map
