@@ -400,12 +400,20 @@ def _valid_lengths(attention_mask: Optional[torch.Tensor], batch_size: int, seq_
     return wait
 
 
-def _sample_bhsd(t: torch.Tensor, b: int, n: int) -> torch.Tensor:
-    """Sample b's first n tokens of `[B, N, H, d]` as `[1, H, n, d]`: a view when a token's heads are
-    contiguous (the kernels take row strides; pooled K/V then share them), else a copy."""
-    x = t[b:b + 1, :n].permute(0, 2, 1, 3)
+def _kernels_take_rows(t: torch.Tensor, n: int) -> bool:
+    """Whether the kernels can address the first n tokens of `[B, N, H, d]` where they are: a token's
+    heads contiguous (pooled K/V then have the same row stride), 16-byte rows, and one head's rows
+    within the 2 GiB that the 16-bit kernels' buffer offsets reach (279,620 tokens of 30 heads of
+    128; contiguous heads reach thirty times as far)."""
     h, d = int(t.size(2)), int(t.size(3))
-    return x if t.is_cuda and t.stride()[1:] == (h * d, d, 1) else x.contiguous()
+    return t.stride()[1:] == (h * d, d, 1) and t.data_ptr() % 16 == 0 and n * h * d * 2 < 1 << 31
+
+
+def _sample_bhsd(t: torch.Tensor, b: int, n: int) -> torch.Tensor:
+    """Sample b's first n tokens of `[B, N, H, d]` as `[1, H, n, d]`: a view where the kernels can take
+    it in place, else a copy."""
+    x = t[b:b + 1, :n].permute(0, 2, 1, 3)
+    return x if t.is_cuda and _kernels_take_rows(t, n) else x.contiguous()
 
 
 class ZImageSinkCalibrationProcessor:

@@ -15,6 +15,7 @@ import torch
 import torch.nn as nn
 
 from oracle import torch_ref
+from sinkattn_amd import sparse_attention as sa
 from sinkattn_amd import wan_runtime as wr
 from sinkattn_amd import zimage_runtime as zr
 from sinkattn_amd.sparse_attention import SinkRuntimeState, SinkSparseConfig
@@ -315,3 +316,18 @@ def test_wan_calibration_processor_dense_attention(N, mode):
     xg = x.clone().requires_grad_()
     wr.WanSinkCalibrationProcessor2_0(cal, 0)(attn, xg).float().sum().backward()
     assert xg.grad is not None and bool(xg.grad.abs().sum() > 0)
+
+
+def test_zimage_sample_past_the_kernels_row_reach():
+    """One head's rows past 2 GiB as a view of token rows: the sample is copied and the sparse call
+    takes it.  A diagonal mask: the last block against torch's attention of that block."""
+    H, D, N = 120, 128, 69906  # 120 * 128 * 2 * 69906 bytes > 2^31
+    g = torch.Generator(device=DEV).manual_seed(0)
+    q, k, v = (zr._sample_bhsd(torch.randn(1, N, H, D, device=DEV, dtype=torch.bfloat16, generator=g), 0, N)
+               for _ in range(3))
+    nb = -(-N // 128)
+    mask = torch.eye(nb, dtype=torch.bool, device=DEV).expand(1, H, nb, nb)
+    out = sa._block_sparse_attn(q, k, v, mask, return_lse=False)[0]
+    r = slice((nb - 1) * 128, N)
+    want = torch.softmax((q[:, :, r].float() @ k[:, :, r].float().transpose(2, 3).contiguous()) / D ** 0.5, -1) @ v[:, :, r].float()
+    _check(out[:, :, r], want.cpu(), 2e-2, 1e-3, "last block of a long sample")

@@ -354,3 +354,16 @@ def test_qk_prep_dispatch_helpers():
     re2, im2 = wr.rotary_tables_2d((cos, sin), N, D)
     assert torch.allclose(re2, c.real) and torch.allclose(im2, c.imag)
     assert wr.rotary_tables_2d(torch.randn(N, D), N, D) is None
+
+
+@pytest.mark.parametrize("h,d", [(30, 128), (1, 128), (24, 64)])
+def test_zimage_samples_in_place_within_the_kernels_reach(h, d):
+    """A sample is passed as a view only up to the 2 GiB of one head's rows that the 16-bit kernels
+    address (a copy with contiguous heads reaches h times as far), and only with whole token rows."""
+    edge = -(-(1 << 31) // (2 * h * d))  # first length that spans 2 GiB
+    t = torch.empty(2, edge + 1, h, d, device="meta", dtype=torch.bfloat16)
+    assert zr._kernels_take_rows(t, edge - 1) and not zr._kernels_take_rows(t, edge)
+    assert h == 1 or not zr._kernels_take_rows(t.transpose(1, 2).contiguous().transpose(1, 2), 64)
+    assert not zr._kernels_take_rows(t[..., : d // 2], 64)
+    x = torch.randn(2, 40, h, d)
+    assert zr._sample_bhsd(x, 1, 33).is_contiguous() and torch.equal(zr._sample_bhsd(x, 1, 33)[0, 0], x[1, :33, 0])
