@@ -7,7 +7,9 @@
  *    <0            invalid argument (nothing was enqueued); see sinkattn_last_error()
  *    >0            a hipError_t from a launch
  * No C++ exception crosses this boundary and no entry point allocates device memory:
- * outputs and workspaces are supplied by the caller (sizes from the *_bytes queries).
+ * outputs and workspaces are supplied by the caller (sizes from the *_bytes queries; at one
+ * block size, head dim and dtype a workspace sized for a call also serves every call that is no
+ * larger in any dimension).
  * All work is stream-ordered.  Every function is stateless and reentrant except
  * sinkattn_block_sparse_attn_noalloc (end of this file): it keeps its plan in one static
  * device array per GPU (SINKATTN_NOALLOC_SCRATCH_BYTES = 32 MiB, reserved on every GPU
@@ -260,7 +262,7 @@ int sinkattn_lse_mix(const void* sink_out, const int64_t sink_strides[4],
  * block_size 16, 32, 64 or 128 with D 128: bf16/f16 inputs use the bf16/f16 matrix cores
  * (products are exact, sums fp32) and a device workspace of
  * sinkattn_block_mass_pool_workspace_bytes() bytes (per-row block sums of the resident
- * work-groups, queried for the current device); f32 inputs at these block sizes, D 128 use
+ * work-groups and records of split key ranges, queried for the current device); f32 inputs at these block sizes, D 128 use
  * the fp32 matrix cores (up to about 490 key blocks) and need no workspace.  Every other shape
  * (block_size 1..1024, D 1..256, f32 otherwise) runs a generic kernel (fp32 dot products,
  * two passes over the keys, no workspace; the query may still return a size for a

@@ -1769,10 +1769,17 @@ hipError_t launch_dense_fwd(const FwdArgs& args, int dtype, hipStream_t stream) 
 // at most 2 GiB.
 constexpr int64_t kMassWsBytes = (int64_t)2 << 30;
 
-int64_t dense_mass_heads(int64_t nbh, int64_t nqb, int64_t nkb) {
+static int64_t dense_mass_heads(int64_t nbh, int64_t nqb, int64_t nkb) {
   const int64_t head = nqb * nkb * 512;
   const int64_t fit = head > 0 ? kMassWsBytes / head : nbh;
   return fit < 1 ? 1 : (fit < nbh ? fit : nbh);
+}
+
+// Bytes of the whole call's sums up to that limit (a launch of fewer heads needs no more), so that
+// a workspace sized for a call also serves every smaller one.
+size_t dense_mass_workspace_bytes(int64_t nbh, int64_t nqb, int64_t nkb) {
+  const int64_t head = nqb * nkb * 512, all = nbh * head, most = head > kMassWsBytes ? head : kMassWsBytes;
+  return (size_t)(all < most ? all : most);
 }
 
 hipError_t launch_dense_mass(const FwdArgs& args, int dtype, hipStream_t stream) {

@@ -312,8 +312,7 @@ int sinkattn_dense_fwd(const void* q, const void* k, const void* v, int dtype, i
 
 size_t sinkattn_dense_mass_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk) {
   if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0) return 0;
-  const int64_t nqb = cdiv(Nq, 128), nkb = cdiv(Nk, 128);
-  return (size_t)(sa::dense_mass_heads(B * H, nqb, nkb) * nqb * nkb * 512);
+  return sa::dense_mass_workspace_bytes(B * H, cdiv(Nq, 128), cdiv(Nk, 128));
 }
 
 int sinkattn_dense_mass(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t H,

@@ -119,7 +119,7 @@ int64_t plan_order_cache_ints(int rows, int nqb, int entries);
 hipError_t launch_block_sparse_plan(const PlanArgs& a, hipStream_t stream);
 hipError_t launch_block_sparse_fwd(const FwdArgs& a, int dtype, int D, hipStream_t stream);
 hipError_t launch_dense_fwd(const FwdArgs& a, int dtype, hipStream_t stream);
-int64_t dense_mass_heads(int64_t nbh, int64_t nqb, int64_t nkb);
+size_t dense_mass_workspace_bytes(int64_t nbh, int64_t nqb, int64_t nkb);
 hipError_t launch_dense_mass(const FwdArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_block_mass_pool(const PoolArgs& a, int dtype, int D, hipStream_t stream);
 bool pool_f32_mfma(const PoolArgs& a);

@@ -1322,10 +1322,13 @@ static MassSplit mass_split(int64_t items, int Nk) {
   return S >= 2 ? MassSplit{n, S} : MassSplit{0, 1};
 }
 
+// The resident groups' slots, then the range records of a split round: n * S <= G of 256 floats.  From
+// the length that may be split on the room for a full round of them is always there, so that a
+// workspace sized for a call also serves every smaller one (0.8 MB).
 size_t block_mass_workspace_floats(int64_t items, int64_t nkb, int64_t Nk) {
-  const int64_t groups = items < block_mass_groups() ? items : block_mass_groups();
-  const MassSplit sp = mass_split(items, (int)Nk);
-  return (size_t)(groups * nkb * 128 + (int64_t)sp.n * (sp.n > 0 ? sp.S : 0) * 256);
+  const int64_t G = block_mass_groups(), groups = items < G ? items : G;
+  const bool may_split = items > 0 && (Nk + 127) / 128 >= kMassSplitTiles;
+  return (size_t)(groups * nkb * 128 + (may_split ? G * 256 : 0));
 }
 
 template <int CT, int KB>
@@ -1375,12 +1378,13 @@ static int max_split(int64_t items, int Nk, int block_size) {
   return max(1, min(min((int)(max_pool_groups() / items), kMassMaxRanges), (Nk + 127) / 128 / kMassMinTiles));
 }
 
+// Per group the rows' block maxima and, below block 128, the item's column maxima; then the ranges'
+// row maxima (items * S <= G of 128 floats), with room for a full round as in the block-mass call.
 size_t max_pool_workspace_floats(int64_t items, int64_t nkb, int64_t N, int block_size) {
-  const int64_t groups = items < max_pool_groups() ? items : max_pool_groups();
-  // per group: the rows' block maxima, and below block 128 the item's column maxima
+  const int64_t G = max_pool_groups(), groups = items < G ? items : G;
   const int64_t per_kb = 128 + (block_size == 128 ? 0 : 128 / block_size);
-  const int S = max_split(items, (int)N, block_size);
-  return (size_t)(groups * nkb * per_kb + (S > 1 ? items * S * 128 : 0));
+  const bool may_split = items > 0 && (N + 127) / 128 >= kMaxSplitTiles;
+  return (size_t)(groups * nkb * per_kb + (may_split ? G * 128 : 0));
 }
 
 template <int CT, int KB>

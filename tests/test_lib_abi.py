@@ -121,6 +121,36 @@ def test_workspace_queries(lib):
     assert lib.sinkattn_abi_version() >= 1
 
 
+@pytest.mark.parametrize("name", ["sinkattn_block_mass_pool_workspace_bytes", "sinkattn_max_pool_workspace_bytes",
+                                  "sinkattn_dense_mass_workspace_bytes", "sinkattn_mean_pool_workspace_bytes"])
+def test_a_workspace_serves_every_smaller_call(lib, name):
+    """The entry points take no workspace size, so a buffer sized for a caller's largest call has to
+    hold for its smaller ones: every query is non-decreasing in the batch, heads and lengths."""
+    query = getattr(lib, name)
+
+    def size(bh, n, block, nk):
+        if "max_pool" in name:
+            return query(1, bh, n, block, 0)
+        if "dense_mass" in name:
+            return query(1, bh, n, nk)
+        return query(1, bh, n, nk, 128, block) if "mean" in name else query(1, bh, n, nk, block, 0)
+
+    heads = list(range(1, 19)) + [24, 30, 40, 64, 100, 128, 400]
+    lengths = [1, 128, 129, 1000, 1920, 2048, 2049, 3072, 4096, 8192, 12288, 16384, 32760, 75600, 140800]
+    for block in (16, 64, 128):
+        for n in lengths:
+            for nk in (lengths if "max" not in name else [n]):
+                got = [size(bh, n, block, nk) for bh in heads]
+                assert got == sorted(got), (block, n, nk)
+        for bh in heads:
+            got = [size(bh, n, block, n) for n in lengths]
+            assert got == sorted(got), (block, bh)
+            if "max" not in name:
+                for n in lengths:
+                    assert [size(bh, n, block, x) for x in lengths] == sorted(size(bh, n, block, x) for x in lengths)
+                    assert [size(bh, x, block, n) for x in lengths] == sorted(size(bh, x, block, n) for x in lengths)
+
+
 def test_fwd_rejects_heads_past_the_32bit_copy_range(lib):
     # K/V tiles are copied through buffer descriptors with a 32-bit byte range: one head of
     # k/v (and of the compensation kd/vd) must stay under 2 GiB.
