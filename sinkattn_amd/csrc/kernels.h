@@ -137,6 +137,10 @@ hipError_t launch_mean_pool(const PoolArgs& a, int dtype, int D, hipStream_t str
 // kGenericPoolMaxLds (the LDS of a CU).
 constexpr size_t kGenericPoolMaxLds = 160 * 1024;
 size_t generic_pool_lds_need(int D, int nkb, int dtype);
+// Lets a pooling kernel launch with all of a CU's LDS beside its `static_lds` bytes.  The limit belongs
+// to the process, so every call sets the same one: set to each call's need, a host thread could
+// lower it between another's set and launch.
+hipError_t allow_all_lds(const void* kern, size_t static_lds);
 hipError_t launch_block_mass_generic(const PoolArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_max_pool_generic(const PoolArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_coverage_mask(const MaskArgs& a, hipStream_t stream);

@@ -516,7 +516,7 @@ bool pool_f32_mfma(const PoolArgs& a) {
 // The kernel's dynamic LDS and, where two items share a map entry, the zeroed map.
 static hipError_t f32_pool_setup(const void* kern, const PoolArgs& a, bool zero, size_t lds, hipStream_t stream) {
   if (kF32StaticLds + lds > 64 * 1024) {  // past what a launch gets without asking
-    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e = allow_all_lds(kern, kF32StaticLds);
     if (e != hipSuccess) return e;
   }
   if (!zero) return hipSuccess;

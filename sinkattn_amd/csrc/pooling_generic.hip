@@ -266,6 +266,8 @@ __global__ __launch_bounds__(256) void block_mass_generic_kernel(PoolArgs a) {
 // of the whole block).  Causal: key blocks after the query block are skipped and the
 // diagonal block adds -1e6 to raw scores above the diagonal.
 // ------------------------------------------------------------------------------------
+constexpr size_t kMaxGenericStaticLds = 16;  // bytes
+
 template <int IT, bool MF>
 __global__ __launch_bounds__(256) void max_pool_generic_kernel(PoolArgs a) {
   extern __shared__ float gsm[];
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(256) void max_pool_generic_kernel(PoolArgs a) {
   // Po in q.dtype, its row sum (fp32 accumulation, rounded to q.dtype), then the division.
   for (int kb = threadIdx.x; kb < nkb; kb += blockDim.x) acc[kb] = kb < kb_end ? round_elem<IT>(acc[kb]) : 0.f;
   __syncthreads();
-  __shared__ float part[4];
+  __shared__ float part[kMaxGenericStaticLds / 4];  // one per wave
   float sum = 0.f;
   for (int kb = threadIdx.x; kb < nkb; kb += blockDim.x) sum += acc[kb];
 #pragma unroll
@@ -363,12 +365,15 @@ size_t generic_pool_lds_need(int D, int nkb, int dtype) {
   return generic_pool_lds_bytes(D, nkb, generic_mf(D, dtype));
 }
 
+hipError_t allow_all_lds(const void* kern, size_t static_lds) {
+  return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kGenericPoolMaxLds - static_lds));
+}
+
 template <typename Kern>
-static hipError_t launch_generic(Kern kern, const PoolArgs& a, bool mf, hipStream_t stream) {
+static hipError_t launch_generic(Kern kern, const PoolArgs& a, bool mf, size_t static_lds, hipStream_t stream) {
   const dim3 grid(a.nqb, a.B * a.H);
   const size_t lds = generic_pool_lds_bytes(a.D, a.nkb, mf);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const hipError_t e = allow_all_lds(reinterpret_cast<const void*>(kern), static_lds);
   if (e != hipSuccess) return e;
   kern<<<grid, 256, lds, stream>>>(a);
   return hipGetLastError();
@@ -378,24 +383,24 @@ hipError_t launch_block_mass_generic(const PoolArgs& a, int dtype, hipStream_t s
   if (a.B * a.H * a.nqb == 0) return hipSuccess;
   const bool mf = generic_mf(a.D, dtype);
   if (dtype == kBF16)
-    return mf ? launch_generic(block_mass_generic_kernel<kBF16, true>, a, true, stream)
-              : launch_generic(block_mass_generic_kernel<kBF16, false>, a, false, stream);
+    return mf ? launch_generic(block_mass_generic_kernel<kBF16, true>, a, true, 0, stream)
+              : launch_generic(block_mass_generic_kernel<kBF16, false>, a, false, 0, stream);
   if (dtype == kF16)
-    return mf ? launch_generic(block_mass_generic_kernel<kF16, true>, a, true, stream)
-              : launch_generic(block_mass_generic_kernel<kF16, false>, a, false, stream);
-  return launch_generic(block_mass_generic_kernel<kF32, false>, a, false, stream);
+    return mf ? launch_generic(block_mass_generic_kernel<kF16, true>, a, true, 0, stream)
+              : launch_generic(block_mass_generic_kernel<kF16, false>, a, false, 0, stream);
+  return launch_generic(block_mass_generic_kernel<kF32, false>, a, false, 0, stream);
 }
 
 hipError_t launch_max_pool_generic(const PoolArgs& a, int dtype, hipStream_t stream) {
   if (a.B * a.H * a.nqb == 0) return hipSuccess;
   const bool mf = generic_mf(a.D, dtype);
   if (dtype == kBF16)
-    return mf ? launch_generic(max_pool_generic_kernel<kBF16, true>, a, true, stream)
-              : launch_generic(max_pool_generic_kernel<kBF16, false>, a, false, stream);
+    return mf ? launch_generic(max_pool_generic_kernel<kBF16, true>, a, true, kMaxGenericStaticLds, stream)
+              : launch_generic(max_pool_generic_kernel<kBF16, false>, a, false, kMaxGenericStaticLds, stream);
   if (dtype == kF16)
-    return mf ? launch_generic(max_pool_generic_kernel<kF16, true>, a, true, stream)
-              : launch_generic(max_pool_generic_kernel<kF16, false>, a, false, stream);
-  return launch_generic(max_pool_generic_kernel<kF32, false>, a, false, stream);
+    return mf ? launch_generic(max_pool_generic_kernel<kF16, true>, a, true, kMaxGenericStaticLds, stream)
+              : launch_generic(max_pool_generic_kernel<kF16, false>, a, false, kMaxGenericStaticLds, stream);
+  return launch_generic(max_pool_generic_kernel<kF32, false>, a, false, kMaxGenericStaticLds, stream);
 }
 
 }  // namespace sa

@@ -13,6 +13,7 @@ max mode    vs oracle/torch_ref.max_pool_map (the reference's four rounding poin
 mean mode   vs oracle/torch_ref.mean_pool_scores: rtol 1e-5.
 """
 import math
+import threading
 
 import pytest
 import torch
@@ -404,3 +405,43 @@ def test_mean_mode_tile_edges(B, H, Nq, Nk, bs, D, dtype):
     ref = torch_ref.mean_pool_scores(q, k, block_size=bs)
     assert ours.shape == ref.shape
     assert torch.allclose(ours, ref, rtol=2e-5, atol=1e-7)
+
+
+def test_pooling_lds_from_two_threads():
+    """Host threads whose calls need different amounts of LDS (the fp32 and the generic kernels past
+    64 KB): the limit a kernel may launch with is one per process, and both get theirs."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+
+    def call(fn, N, D):
+        q, k = (torch.randn(1, 1, N, D, device="cuda", generator=g) for _ in range(2))
+        return lambda: fn(q, k)
+
+    def mass(q, k):
+        return ops.block_mass_scores(q, k, block_size=16)
+
+    def most(q, k):
+        return ops.max_pool_scores(q, k, 0.09, block_size=16)
+
+    for fn, D, sizes in ((mass, 128, (2400, 7000)), (most, 128, (2400, 7000)), (mass, 64, (640, 9000)), (most, 64, (640, 9000))):
+        calls = [call(fn, N, D) for N in sizes]
+        want = [c() for c in calls]
+        bad = []
+
+        def work(i):
+            with torch.cuda.stream(torch.cuda.Stream()):
+                try:
+                    for _ in range(40):
+                        got = calls[i]()
+                    torch.cuda.current_stream().synchronize()
+                    if not torch.allclose(got, want[i], rtol=1e-5, atol=1e-8):
+                        bad.append(f"{sizes[i]}: other values")
+                except Exception as e:  # a launch past the limit another thread set
+                    bad.append(f"{sizes[i]}: {e}")
+
+        torch.cuda.synchronize()
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad, bad
