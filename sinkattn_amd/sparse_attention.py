@@ -783,15 +783,28 @@ def _dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch
     return F.scaled_dot_product_attention(q, k, v, attn_mask=None, dropout_p=0.0, is_causal=False)
 
 
+# What a recorded call runs, as defined here: the one-pass form stands in for these alone.
+_RECORD_PATH = (SinkMaskCalibrator.record, _compute_block_scores, _compute_exact_block_mass_scores)
+
+
+def _records_exact_map(calibrator: SinkMaskCalibrator) -> bool:
+    """Whether `calibrator.record` is this module's own, block size 128, exact mode: not a subclass,
+    and nothing on its path replaced on the instance, the class or this module."""
+    if type(calibrator) is not SinkMaskCalibrator or "record" in vars(calibrator):
+        return False
+    if (SinkMaskCalibrator.record, _compute_block_scores, _compute_exact_block_mass_scores) != _RECORD_PATH:
+        return False
+    cfg = calibrator.config
+    return int(cfg.block_size) == 128 and str(cfg.pooling_mode).strip().lower() == "exact"
+
+
 def _record_and_attend(calibrator: SinkMaskCalibrator, layer_idx: int, q: torch.Tensor, k: torch.Tensor,
                        v: torch.Tensor) -> torch.Tensor:
     """`calibrator.record(layer_idx, q, k, v)` and the dense attention of the same call.  The exact
     map at block size 128 comes out of the attention's own pass over the scores; a calibrator
     with a `record` of its own, another mode, or operands the dense kernel does not take get
     the two steps."""
-    cfg = calibrator.config if type(calibrator) is SinkMaskCalibrator else None
-    if (cfg is not None and "record" not in vars(calibrator) and int(cfg.block_size) == 128
-            and str(cfg.pooling_mode).strip().lower() == "exact" and _dense_kernel_takes(q, k, v)):
+    if _records_exact_map(calibrator) and _dense_kernel_takes(q, k, v):
         out, mass = ops.dense_attention_mass(q, k, v)
         with torch.no_grad():
             calibrator._record_scores(layer_idx, lambda: mass)

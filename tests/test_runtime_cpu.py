@@ -9,6 +9,7 @@ import torch
 import torch.nn as nn
 
 from oracle import torch_ref
+from sinkattn_amd import sparse_attention as sa
 from sinkattn_amd import wan_runtime as wr
 from sinkattn_amd import zimage_runtime as zr
 from sinkattn_amd.sparse_attention import SinkRuntimeState, SinkSparseConfig
@@ -367,3 +368,29 @@ def test_zimage_samples_in_place_within_the_kernels_reach(h, d):
     assert not zr._kernels_take_rows(t[..., : d // 2], 64)
     x = torch.randn(2, 40, h, d)
     assert zr._sample_bhsd(x, 1, 33).is_contiguous() and torch.equal(zr._sample_bhsd(x, 1, 33)[0, 0], x[1, :33, 0])
+
+
+# --- which calls the calibration pass hands to the one-pass kernel -----------------------------
+class _Subclass(sa.SinkMaskCalibrator):
+    pass
+
+
+@pytest.mark.parametrize("where", ["none", "subclass", "instance", "class", "scores", "exact_scores"])
+def test_a_replaced_record_is_called(where, monkeypatch):
+    """Attention and map come from one pass only for a calibrator whose `record` is the package's
+    own; one replaced on a subclass, the instance, the class or below it in the module is run."""
+    calls = []
+    fused = (torch.full((1, 2, 300, 4), 7.0), torch.ones(1, 2, 3, 3))
+    monkeypatch.setattr(sa, "_dense_kernel_takes", lambda q, k, v: True)
+    monkeypatch.setattr(sa.ops, "dense_attention_mass", lambda q, k, v: calls.append("fused") or fused)
+    monkeypatch.setattr(sa.ops, "dense_attention", lambda q, k, v: (q, None))
+    monkeypatch.setattr(sa.ops, "block_mass_scores", lambda q, k, **kw: fused[1])
+    cal = (_Subclass if where == "subclass" else sa.SinkMaskCalibrator)(SinkSparseConfig(pooling_mode="exact"))
+    own = {"instance": (cal, "record"), "class": (sa.SinkMaskCalibrator, "record"), "scores": (sa, "_compute_block_scores"),
+           "exact_scores": (sa, "_compute_exact_block_mass_scores")}.get(where)
+    if own is not None:
+        monkeypatch.setattr(*own, lambda *a: calls.append("own") or fused[1])
+    q = torch.randn(1, 2, 300, 4)
+    out = sa._record_and_attend(cal, 0, q, q, q)
+    assert calls == {"none": ["fused"], "subclass": []}.get(where, ["own"])
+    assert torch.equal(out, fused[0] if where == "none" else q)
