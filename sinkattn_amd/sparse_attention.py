@@ -755,7 +755,10 @@ def _plain_gpu_call(*tensors: torch.Tensor) -> bool:
 def _dense_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """Whether the dense kernel computes scaled_dot_product_attention(q, k, v): 16-bit GPU tensors
     [B, H, N, 128] of one dtype and head count that it can address in place, enough keys, no
-    autocast to another dtype and the flash backend not switched off."""
+    autocast to another dtype, the flash backend not switched off, and torch's own function not
+    replaced by a program's."""
+    if F.scaled_dot_product_attention is not getattr(torch._C._nn, "scaled_dot_product_attention", None):
+        return False
     if not _HAS_BLOCK_SPARSE or not _plain_gpu_call(q, k, v):
         return False
     if not (q.dim() == k.dim() == v.dim() == 4 and q.dtype == k.dtype == v.dtype

@@ -394,3 +394,17 @@ def test_a_replaced_record_is_called(where, monkeypatch):
     out = sa._record_and_attend(cal, 0, q, q, q)
     assert calls == {"none": ["fused"], "subclass": []}.get(where, ["own"])
     assert torch.equal(out, fused[0] if where == "none" else q)
+
+
+def test_a_replaced_sdpa_is_called(monkeypatch):
+    """A program's own scaled_dot_product_attention (an accelerated or an instrumented one) is called
+    for the dense attention of the runtimes, as before the dense kernel."""
+    monkeypatch.setattr(sa, "_plain_gpu_call", lambda *t: True)
+    monkeypatch.setattr(sa, "_HAS_BLOCK_SPARSE", True)
+    monkeypatch.setattr(sa.ops, "dense_attention", lambda q, k, v: (torch.zeros_like(q), None))
+    q, k, v = (torch.randn(1, 2, n, 128, dtype=torch.bfloat16) for n in (64, 1024, 1024))
+    assert not sa._dense_attention(q, k, v).any()
+    own = torch.nn.functional.scaled_dot_product_attention
+    monkeypatch.setattr(torch.nn.functional, "scaled_dot_product_attention", lambda *a, **kw: own(*a, **kw) + 1)
+    assert not sa._dense_kernel_takes(q, k, v)
+    assert torch.equal(sa._dense_attention(q, k, v), own(q, k, v) + 1)
