@@ -741,15 +741,24 @@ def _adapt_block_mask_for_kernel(block_mask: torch.Tensor, *, source_block_size:
 _DENSE_KERNEL_MIN_KEYS = 1024
 
 
+def _ops_are_watched() -> bool:
+    """Whether a mode that watches or rewrites torch ops is on (tracing, dispatch and function modes,
+    vmap and the other function transforms, forward-mode AD).  Torch has no public question for
+    all of them; one that a torch version does not answer counts as yes."""
+    try:
+        return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
+                    or torch._C._len_torch_function_stack()
+                    or torch._C._functorch.peek_interpreter_stack() is not None
+                    or torch.autograd.forward_ad._current_level >= 0)
+    except AttributeError:
+        return True
+
+
 def _plain_gpu_call(*tensors: torch.Tensor) -> bool:
-    """Plain GPU tensors outside every mode that watches or rewrites torch ops: the raw kernels
-    are invisible to autograd, forward-mode AD, vmap, tracing and dispatch modes."""
+    """Plain GPU tensors without gradients, outside every mode the raw kernels are invisible to."""
     return (all(type(t) is torch.Tensor and t.is_cuda for t in tensors)
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0)
+            and not _ops_are_watched())
 
 
 def _dense_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:

@@ -7,6 +7,7 @@ import math
 import pytest
 import torch
 import torch.nn as nn
+from torch.utils.flop_counter import FlopCounterMode
 
 from oracle import torch_ref
 from sinkattn_amd import sparse_attention as sa
@@ -408,3 +409,26 @@ def test_a_replaced_sdpa_is_called(monkeypatch):
     monkeypatch.setattr(torch.nn.functional, "scaled_dot_product_attention", lambda *a, **kw: own(*a, **kw) + 1)
     assert not sa._dense_kernel_takes(q, k, v)
     assert torch.equal(sa._dense_attention(q, k, v), own(q, k, v) + 1)
+
+
+def test_watching_modes_and_unknown_torch_versions(monkeypatch):
+    """Modes that watch torch ops are seen; a torch that lacks one of the questions is taken to watch,
+    and does not raise."""
+    seen = []
+    probe = lambda x: seen.append(sa._ops_are_watched()) or x * 2
+    assert not sa._ops_are_watched()
+    torch.func.vmap(probe)(torch.ones(3))
+    torch.func.jvp(probe, (torch.ones(3),), (torch.ones(3),))
+    with FlopCounterMode(display=False):
+        probe(torch.ones(3))
+    with torch.device("cpu"):  # a function mode
+        probe(torch.ones(3))
+    with torch.autograd.forward_ad.dual_level():
+        probe(torch.ones(3))
+    assert seen == [True] * 5 and not sa._ops_are_watched()
+    for owner, name in ((torch._C, "_len_torch_dispatch_stack"), (torch._C, "_len_torch_function_stack"),
+                        (torch._C._functorch, "peek_interpreter_stack"), (torch.autograd.forward_ad, "_current_level")):
+        with monkeypatch.context() as m:
+            m.delattr(owner, name)
+            assert sa._ops_are_watched(), name
+    assert not sa._ops_are_watched()
