@@ -817,10 +817,14 @@ def _record_and_attend(calibrator: SinkMaskCalibrator, layer_idx: int, q: torch.
     with a `record` of its own, another mode, or operands the dense kernel does not take get
     the two steps."""
     if _records_exact_map(calibrator) and _dense_kernel_takes(q, k, v):
-        out, mass = ops.dense_attention_mass(q, k, v)
-        with torch.no_grad():
-            calibrator._record_scores(layer_idx, lambda: mass)
-        return out
+        try:
+            out, mass = ops.dense_attention_mass(q, k, v)
+        except torch.OutOfMemoryError:  # up to 2 GiB of row sums; the two steps' (at most 768 q-blocks') are fewer
+            out = None
+        if out is not None:
+            with torch.no_grad():
+                calibrator._record_scores(layer_idx, lambda: mass)
+            return out
     calibrator.record(layer_idx, q, k, v)
     return _dense_attention(q, k, v)
 

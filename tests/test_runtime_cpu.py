@@ -397,6 +397,22 @@ def test_a_replaced_record_is_called(where, monkeypatch):
     assert torch.equal(out, fused[0] if where == "none" else q)
 
 
+def test_calibration_layer_without_room_for_the_row_sums(monkeypatch):
+    """Where the one-pass form's workspace does not fit, the layer records and attends in two steps,
+    which need less, and the call is counted once."""
+    def no_room(q, k, v):
+        raise torch.OutOfMemoryError("row sums")
+
+    monkeypatch.setattr(sa, "_dense_kernel_takes", lambda q, k, v: True)
+    monkeypatch.setattr(sa.ops, "dense_attention_mass", no_room)
+    monkeypatch.setattr(sa.ops, "dense_attention", lambda q, k, v: (q, None))
+    monkeypatch.setattr(sa.ops, "block_mass_scores", lambda q, k, **kw: torch.ones(1, 2, 3, 3))
+    cal = sa.SinkMaskCalibrator(SinkSparseConfig(pooling_mode="exact"))
+    q = torch.randn(1, 2, 300, 4)
+    assert torch.equal(sa._record_and_attend(cal, 0, q, q, q), q)
+    assert cal.current_step == 0 and cal.score_counts == {0: 1}
+
+
 def test_a_replaced_sdpa_is_called(monkeypatch):
     """A program's own scaled_dot_product_attention (an accelerated or an instrumented one) is called
     for the dense attention of the runtimes, as before the dense kernel."""
