@@ -353,7 +353,10 @@ static int mean_pool_impl(const char* who, sa::TokenPoolArgs& a, int dtype, int6
   int64_t p = prefix < 0 ? 0 : (prefix > end ? end : prefix);
   if (gap == 1) p = end;  // every row is kept
   const int64_t nout = p + cdiv(end - p, gap) + (N - end);
-  if (B * H > 65535 || N > kMaxInt || gap > kMaxInt) return fail("%s: sizes exceed the launch limits", who);
+  if (B * H > 65535 || N > kMaxInt) return fail("%s: sizes exceed the launch limits", who);
+  // a group's row numbers, up to N + gap + 7 before they are held to its last row, are 32-bit
+  if (p == end) gap = 1;  // nothing is pooled
+  else if (gap > kMaxInt - 8 - N) return fail("%s: gap %lld exceeds the row range", who, (long long)gap);
   if (B * H * nout == 0) return 0;
   for (int z = 0; z < a.tensors; ++z) {
     int rc;

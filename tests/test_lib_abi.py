@@ -151,6 +151,14 @@ def test_a_workspace_serves_every_smaller_call(lib, name):
                     assert [size(bh, x, block, n) for x in lengths] == sorted(size(bh, x, block, n) for x in lengths)
 
 
+def test_mean_pool_rejects_groups_past_32_bit_rows(lib):
+    s = _i64x4(0, 0, 64, 1)
+    for gap in ((1 << 31) - 100, 1 << 31, 1 << 40):
+        assert lib.sinkattn_mean_pool_tokens(16, 0, 1, 1, 100, 64, s, 0, gap, 16, s, None) == -1 and "gap" in _err(lib)
+        assert lib.sinkattn_mean_pool_kv(16, 16, 0, 1, 1, 100, 64, s, s, 0, 90, gap, 16, 16, s, s, None) == -1
+        assert lib.sinkattn_mean_pool_tokens(16, 0, 1, 1, 0, 64, s, 0, gap, 16, s, None) == 0  # nothing to pool
+
+
 def test_fwd_rejects_heads_past_the_32bit_copy_range(lib):
     # K/V tiles are copied through buffer descriptors with a 32-bit byte range: one head of
     # k/v (and of the compensation kd/vd) must stay under 2 GiB.
