@@ -540,13 +540,13 @@ static hipError_t launch_mass_f32(const PoolArgs& a, hipStream_t stream) {
 // ------------------------------------------------------------------------------------
 // Max-pool map, f32 inputs, head dim 128: the tiles and items of block_mass_f32_kernel with each
 // row's block maxima R[r,kb] = max_j s * (sm_scale * log2e) in LDS (fp32, so the reference's
-// rounding of R to q.dtype is the identity) and m_r the maximum over the row.  Po[qb,kb] =
+// rounding of R to q.dtype is the identity) and m_r the maximum of R over the row.  Po[qb,kb] =
 // max over the block's rows of exp2(R - m_r); rows past the end take m = +inf, which gives 0.
 // The maximum is taken over the bits (values >= 0, a NaN above them all), atomically into the
 // zeroed map where a block of 128 rows spans two items; max_pool_f32_norm_kernel then divides
 // each map row by its sum.  Causal: key blocks after the query block are not seen and raw scores
-// above the diagonal of the diagonal block get -1e6.  [1,10,6545,128]: 1.07 ms at
-// blocks of 128 and 1.1 at 64 (19.1 ms on the generic kernel).
+// above the diagonal of the diagonal block get -1e6.  [1,10,6545,128]: 1.00 ms at
+// blocks of 128 and 1.04 at 64 (19.1 ms on the generic kernel).
 // ------------------------------------------------------------------------------------
 template <int KB>
 __global__ __launch_bounds__(256, 3) void max_pool_f32_kernel(PoolArgs a, int items, int items_per_xcd) {
@@ -602,18 +602,22 @@ __global__ __launch_bounds__(256, 3) void max_pool_f32_kernel(PoolArgs a, int it
     for (int kt = 0; kt < 2; ++kt) {
       mx[kt] = neg_inf();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        mx[kt] = fmaxf(mx[kt], s[kt][i]);
-        if (s[kt][i] != neg_inf()) m = fmaxf(m, s[kt][i] * c);
-      }
+      for (int i = 0; i < 4; ++i) mx[kt] = fmaxf(mx[kt], s[kt][i]);
       mx[kt] = max_col16(mx[kt]);
     }
+    // a block's raw maximum first, then the scale; unseen blocks (raw maximum -inf) take no part in m
+    auto block = [&](int kb, float raw, bool mine) __attribute__((always_inline)) {
+      if (raw != neg_inf()) m = fmaxf(m, raw * c);
+      if (mine) my[kb] = raw * c;
+    };
     if constexpr (NS == 2) {
-      if (g < 2 && 2 * t + g < nkb) my[2 * t + g] = (g == 0 ? mx[0] : mx[1]) * c;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        if (2 * t + kt < nkb) block(2 * t + kt, mx[kt], g == kt);
     } else {
       run = fmaxf(run, fmaxf(mx[0], mx[1]));
       if ((t + 1) % TPB == 0 || t + 1 == ntiles) {
-        if (g == 0) my[t / TPB] = run * c;
+        block(t / TPB, run, g == 0);
         run = neg_inf();
       }
     }
@@ -623,7 +627,6 @@ __global__ __launch_bounds__(256, 3) void max_pool_f32_kernel(PoolArgs a, int it
     if (t + 1 < ntiles) tile(t + 1, (SA_LDS char*)lds_k1, (SA_LDS char*)lds_k0);
   }
 
-  m = max_col16(m);
   if (g == 0) row_m[r] = qrow < a.Nq ? m : pos_inf();
   __syncthreads();
   constexpr int RB = KB < kF32Rows ? KB : kF32Rows;  // rows of this item in one q-block

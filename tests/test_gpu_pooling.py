@@ -382,12 +382,13 @@ def test_exact_mass_f32_rescale(bs):
 @pytest.mark.parametrize("bs,H,Hk,N", [(128, 2, 2, 1), (128, 4, 2, 321), (64, 2, 1, 190), (32, 2, 2, 333),
                                        (16, 4, 4, 259), (16, 1, 1, 7800)])
 def test_max_pool_f32_tile_edges(bs, H, Hk, N, causal):
-    """exp2 of fp32 scores of 128 products each: the fp32 bar below, as on the generic kernel."""
+    """exp2 of fp32 scores of 128 products each: the fp32 bar below, as on the generic kernel.  A negative
+    scale too: a block's raw maximum is scaled, and the row's reference is the largest of those."""
     q, k = _qkd(1, H, Hk, N, N, 128, torch.float32, seed=bs + N)
-    sm = 1.0 / 128 ** 0.5
-    ours = ops.max_pool_scores(q.cuda(), k.cuda(), sm, block_size=bs, causal=causal).cpu()
-    ref = torch_ref.max_pool_map(q, k, sm, block_size=bs, causal=causal)
-    assert torch.allclose(ours, ref, rtol=2e-5, atol=1e-8)
+    for sm in (1.0 / 128 ** 0.5, -0.05):
+        ours = ops.max_pool_scores(q.cuda(), k.cuda(), sm, block_size=bs, causal=causal).cpu()
+        ref = torch_ref.max_pool_map(q, k, sm, block_size=bs, causal=causal)
+        assert torch.allclose(ours, ref, rtol=2e-5, atol=1e-8), sm
 
 
 @pytest.mark.parametrize("B,H,Nq,Nk,bs,D", [(1, 1, 1, 1, 128, 128), (1, 2, 17 * 16 + 1, 33, 16, 128),
