@@ -263,7 +263,7 @@ int sinkattn_lse_mix(const void* sink_out, const int64_t sink_strides[4],
  * (products are exact, sums fp32) and a device workspace of
  * sinkattn_block_mass_pool_workspace_bytes() bytes (per-row block sums of the resident
  * work-groups and records of split key ranges, queried for the current device); f32 inputs at these block sizes, D 128 use
- * the fp32 matrix cores (up to about 490 key blocks) and need no workspace.  Every other shape
+ * the fp32 matrix cores (up to 511 key blocks) and need no workspace.  Every other shape
  * (block_size 1..1024, D 1..256, f32 otherwise) runs a generic kernel (fp32 dot products,
  * two passes over the keys, no workspace; the query may still return a size for a
  * matrix-core block size, which the call then leaves unused), limited by LDS to about
@@ -295,7 +295,7 @@ int sinkattn_block_mass_pool(const void* q, const void* k, int dtype,
  * D 128 (nd <= 1024 at block_size 128) run the persistent MFMA kernel: `workspace` is a
  * device buffer of at least sinkattn_max_pool_workspace_bytes(...) bytes (per-(row,
  * key-block) maxima of the rows in flight); calls that share one workspace must be
- * ordered on one stream.  f32 with D 128 (up to about 490 key blocks) runs on the fp32 matrix
+ * ordered on one stream.  f32 with D 128 (up to 511 key blocks) runs on the fp32 matrix
  * cores, other shapes on the generic kernel (no workspace; same LDS bound as the generic
  * block-mass kernel).
  * ---------------------------------------------------------------------------------- */

@@ -503,7 +503,7 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(float* p, int64_t n) {
 }
 
 // Whether the fp32 matrix-core kernels take a call: head dim 128, a block size they have, the
-// values of an item's rows within the CU's LDS beside the K tiles (about 490 key blocks), a tile
+// values of an item's rows within the CU's LDS beside the K tiles (511 key blocks), a tile
 // of K rows within a buffer's 32-bit offsets, and an item count within the grid.  Any other
 // call runs the generic kernels (6-7 TFLOP/s against 100-125).
 bool pool_f32_mfma(const PoolArgs& a) {

@@ -351,11 +351,13 @@ def test_max_pool_key_ranges(dtype, bs, N, causal):
 
 
 # The fp32 matrix-core kernels (head dim 128, blocks 16-128): items of 64 rows (two to a
-# 128-row block), tiles of 32 keys (two blocks of 16 each), the last key counts before the row
-# values no longer fit LDS, keys whose rows overlap, and the 2^64 rescale.  Bar: the pooling
-# bar of 1e-5 relative (fp32 products and sums on both sides).
+# 128-row block), tiles of 32 keys (two blocks of 16 each), the last key counts whose row values
+# fit LDS (511 key blocks, all 160 KB of it) and the first that take the generic kernel, keys
+# whose rows overlap, and the 2^64 rescale.  Bar: the pooling bar of 1e-5 relative (fp32 products
+# and sums on both sides).
 @pytest.mark.parametrize("bs,Nq,Nk", [(128, 1, 1), (128, 193, 127), (128, 64, 500), (64, 65, 33), (64, 130, 2000),
-                                      (32, 63, 31), (32, 300, 257), (16, 79, 49), (16, 90, 7830)])
+                                      (32, 63, 31), (32, 300, 257), (16, 79, 49), (16, 90, 7830), (16, 90, 8161),
+                                      (16, 90, 8176), (16, 90, 8177)])
 def test_exact_mass_f32_tile_edges(bs, Nq, Nk):
     g = torch.Generator().manual_seed(bs + Nq)
     q = torch.randn(2, Nq, 3, 128, generator=g).transpose(1, 2)
@@ -380,12 +382,13 @@ def test_exact_mass_f32_rescale(bs):
 
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("bs,H,Hk,N", [(128, 2, 2, 1), (128, 4, 2, 321), (64, 2, 1, 190), (32, 2, 2, 333),
-                                       (16, 4, 4, 259), (16, 1, 1, 7800)])
+                                       (16, 4, 4, 259), (16, 1, 1, 7800), (16, 1, 1, 8165), (16, 1, 1, 8176),
+                                       (16, 1, 1, 8177)])
 def test_max_pool_f32_tile_edges(bs, H, Hk, N, causal):
     """exp2 of fp32 scores of 128 products each: the fp32 bar below, as on the generic kernel.  A negative
     scale too: a block's raw maximum is scaled, and the row's reference is the largest of those."""
     q, k = _qkd(1, H, Hk, N, N, 128, torch.float32, seed=bs + N)
-    for sm in (1.0 / 128 ** 0.5, -0.05):
+    for sm in (1.0 / 128 ** 0.5, -0.05)[: 2 if N <= 511 * bs else 1]:  # the generic kernel's scale is positive
         ours = ops.max_pool_scores(q.cuda(), k.cuda(), sm, block_size=bs, causal=causal).cpu()
         ref = torch_ref.max_pool_map(q, k, sm, block_size=bs, causal=causal)
         assert torch.allclose(ours, ref, rtol=2e-5, atol=1e-8), sm
