@@ -404,6 +404,53 @@ def test_first_tile_of_minus_infinity(dtype, D):
     assert ((mass.cpu() - ref)[:, 0].abs() <= 1e-8 + 1e-5 * ref[:, 0].abs()).all()
 
 
+def _whole_q_blocks(q, k, v, mask):
+    """The heads repeated over a batch of more than 256 q-blocks, past which every 16-bit call takes the
+    whole-q-block kernels: the outputs of its last entry."""
+    rep = 256 // (q.shape[0] * q.shape[1] * mask.shape[2]) + 1
+    B = q.shape[0]
+    qr, kr, vr = (t.repeat(rep, 1, 1, 1) if B > 1 else t.expand(rep, -1, -1, -1) for t in (q, k, v))
+    out, lse = ops.block_sparse_attention(qr, kr, vr, ops.block_sparse_plan(mask.repeat(rep, 1, 1, 1)))
+    assert torch.equal(out[:B], out[-B:]) and torch.equal(lse[:B], lse[-B:])
+    return out[-B:], lse[-B:]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Nq,Nk,layout,empty", [(1, 1, "bhsd", 0), (1, 300, "bshd", 0), (31, 129, "bshd", 0), (130, 1, "bhsd", 0),
+                                                (257, 1000, "bshd", 1), (690, 690, "bshd", 2), (900, 129, "bhsd", 1)])
+def test_whole_q_block_kernels_edges(dtype, D, Nq, Nk, layout, empty):
+    """The shapes and layouts of the tests above (single rows and keys, ragged last blocks on both sides,
+    rows without a listed block), whose few q-blocks run the split kernel, on the whole-q-block
+    kernels.  Head dims 64 and 32 sum fp32 exponentials: their lse is held to 1e-4 + 1e-5 |lse|."""
+    q, k, v = _inputs(1, 2, Nq, Nk, D, dtype, seed=Nq * 1000 + Nk, sink_keys=1, layout=layout)
+    mask = _random_mask(1, 2, -(-Nq // 128), -(-Nk // 128), 0.4, seed=Nk, empty_rows=empty)
+    out, lse = _whole_q_blocks(q, k, v, mask)
+    _check(out, lse, q, k, v, mask)
+    if D < 128:
+        ref_l = torch_ref.dense_masked_attention(q, k, v, mask)[1]
+        fin = torch.isfinite(ref_l)
+        assert ((lse.cpu() - ref_l)[fin].abs() <= 1e-4 + 1e-5 * ref_l[fin].abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("step", [7.5, 30.0, -12.0])
+def test_whole_q_block_running_maximum(dtype, D, step):
+    """test_running_maximum_moves_across_tiles on the whole-q-block kernels: maxima that rise slowly
+    (the reference at head dim 128 lags them by up to 8 log2 units), fast, or fall."""
+    N = 1024
+    g = torch.Generator().manual_seed(21)
+    q, k, v = (torch.randn(1, 2, N, D, generator=g) * f for f in (0.5, 0.5, 1.0))
+    q[..., 0] = 1.0
+    offs = torch.arange(N) // 128 * step
+    k[..., 0] = ((offs - offs.min()) / (D ** -0.5 * 1.4426950408889634)).round()
+    q, k, v = (x.to("cuda", dtype) for x in (q, k, v))
+    mask = _random_mask(1, 2, 8, 8, 0.7, seed=5)
+    out, lse = _whole_q_blocks(q, k, v, mask)
+    _check(out, lse, q, k, v, mask)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("D,B,N", [(128, 1, 300), (128, 60, 300), (64, 1, 300), (64, 100, 300), (32, 2, 129)])
 def test_lse_in_the_operands_type(dtype, D, B, N):

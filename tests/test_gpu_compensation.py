@@ -182,6 +182,41 @@ def test_fused_compensation_vs_oracle(N, gap, prefix, comp_rows, seed):
         assert torch.equal(out[:, :, cr:], so[:, :, cr:])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,gap,prefix,comp_rows,empty", [
+    (2000, 30, 0, None, False), (2000, 30, 300, None, True), (556, 8, 0, 256, False), (700, 30, 0, 512, True),
+    (300, 1000, 0, None, True), (130, 1, 0, 128, False)])
+def test_fused_compensation_whole_q_blocks(dtype, N, gap, prefix, comp_rows, empty):
+    """The compensation walk of the whole-q-block kernel, which every real layer runs (the heads
+    repeated over a batch of more than 128 q-blocks; the tests above stay below and run the split
+    kernel): listed tiles, then pooled ones with their bias, ragged ends of both, q-blocks past the
+    compensated rows, and q-blocks with pooled tiles only.  The last entry against the oracle, at
+    the bars above (f16 row sums are within 2^-11)."""
+    H = 2
+    q, k, v, m = _case(1, H, N, 128, 0.3, N + gap, dtype)
+    if empty:
+        m[0, 0, 0] = False  # an empty list below the compensated rows
+    kd, vd = ops.mean_pool_kv(k, v, gap, prefix)
+    cr = N if comp_rows is None else comp_rows
+    so, sl = torch_ref.dense_masked_attention(q, k, v, m)
+    full = torch.ones(1, H, -(-cr // 128), -(-kd.size(2) // 128), dtype=torch.bool)
+    do, dl = torch_ref.dense_masked_attention(q[:, :, :cr], kd, vd, full)
+    sl = torch.where(sl == math.inf, torch.full_like(sl, -math.inf), sl)  # an empty list weighs nothing
+    a = torch.sigmoid(sl[:, :, :cr] - dl - math.log(gap)).unsqueeze(-1)
+    want, want_lse = so.clone(), sl.clone()
+    want[:, :, :cr] = so[:, :, :cr] * a + do * (1 - a)
+    want_lse[:, :, :cr] = torch.logaddexp(sl[:, :, :cr], dl + math.log(gap))
+    for rep in (1, 128 // (H * m.shape[2]) + 1):
+        qr, kr, vr, kdr, vdr = (t.expand(rep, -1, -1, -1) for t in (q, k, v, kd, vd))
+        plan = ops.block_sparse_plan(m.repeat(rep, 1, 1, 1).to(DEV))
+        out, lse = ops.block_sparse_attention_comp(qr, kr, vr, plan, kdr, vdr, gap, comp_rows=comp_rows, return_lse=True)
+        assert torch.equal(out[:1], out[-1:]) and torch.equal(lse[:1], lse[-1:])
+        err = (out[-1:].float().cpu() - want).abs()
+        assert err.max() <= 2e-2 and err.mean() <= 1e-3, (rep, err.max())
+        fin = torch.isfinite(want_lse)
+        assert ((lse[-1:].cpu() - want_lse)[fin].abs() <= 4e-3 + 1e-5 * want_lse[fin].abs()).all(), rep
+
+
 def test_fused_compensation_argument_checks():
     q, k, v, m = _case(1, 2, 512, 128, 0.5, 9)
     plan = ops.block_sparse_plan(m.to(DEV))
