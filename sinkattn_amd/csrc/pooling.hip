@@ -685,6 +685,91 @@ __device__ __forceinline__ float round_to<kF16>(float x) {
   return (float)(_Float16)x;
 }
 
+// The map rows of one item from its rows' block maxima and row maxima (row_m, complete for the
+// group).
+template <int CT, int KB>
+__device__ __forceinline__ void max_pool_rows(const PoolArgs& a, int item, float* ws, float* cm, const float* row_m,
+                                              float* colmax, float* total_sh) {
+  constexpr int NS = 128 / KB;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nkb = a.nkb;
+  const int nqi = (a.Nq + 127) >> 7;
+  const int bh = item / nqi;
+  const int qi = item - bh * nqi;
+  const int kb_item = a.causal ? min(nkb, (qi + 1) * NS) : nkb;  // key blocks any row of the item sees
+  const float m0 = row_m[lane], m1 = row_m[lane + 64];
+  const __amdgpu_buffer_rsrc_t wrs = make_rsrc(ws, (uint32_t)nkb * 512u);
+  if constexpr (KB == 128) {
+    for (int kb = wave; kb < kb_item; kb += 4) {
+      // coherent (L1-bypassing) loads of values other waves of the group wrote
+      const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
+      const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
+      float v = fmaxf(fast_exp2(x0 - m0), fast_exp2(x1 - m1));
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+      if (lane == 0) colmax[kb] = round_to<CT>(v);
+    }
+    __syncthreads();
+    // Row normalisation in q.dtype: sum (fp32 accumulate, rounded), then divide.
+    if (wave == 0) {
+      float part = 0.f;
+      for (int kb = lane; kb < kb_item; kb += 64) part += colmax[kb];
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+      if (lane == 0) total_sh[0] = round_to<CT>(part);
+    }
+    __syncthreads();
+    const float total = total_sh[0];
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qi) * nkb;
+    for (int kb = tid; kb < nkb; kb += 256) {
+      const float v = kb < kb_item ? colmax[kb] / total : 0.f;
+      out[kb] = (uint16_t)(pack2<CT>(v, 0.f) & 0xffffu);
+    }
+  } else {
+    // Pass 1: column maxima of every (q-block, key block) of the item into cm[qs][kb]:
+    // lane l holds rows l and l + 64, so a q-block is a group of KB lanes (KB < 64) or a
+    // whole half (KB = 64).
+    constexpr int G = KB >= 64 ? 64 : KB;
+    for (int kb = wave; kb < kb_item; kb += 4) {
+      const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
+      const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
+      float v0 = fast_exp2(x0 - m0), v1 = fast_exp2(x1 - m1);
+#pragma unroll
+      for (int off = G / 2; off >= 1; off >>= 1) {
+        v0 = fmaxf(v0, __shfl_xor(v0, off, 64));
+        v1 = fmaxf(v1, __shfl_xor(v1, off, 64));
+      }
+      if (lane % G == 0) {
+        const int g = lane / G;
+        cm[(size_t)g * nkb + kb] = round_to<CT>(v0);
+        cm[(size_t)(NS / 2 + g) * nkb + kb] = round_to<CT>(v1);
+      }
+    }
+    __syncthreads();  // the column maxima are in memory (the barrier drains this group's stores)
+    // Pass 2: per q-block (one wave each), the row total in q.dtype, then the division.
+    const __amdgpu_buffer_rsrc_t crs = make_rsrc(cm, (uint32_t)(NS * nkb) * 4u);
+    for (int qs = wave; qs < NS; qs += 4) {
+      const int qb = qi * NS + qs;
+      if (qb >= a.nqb) continue;
+      const int kb_end = a.causal ? min(nkb, qb + 1) : nkb;
+      float part = 0.f;
+      for (int kb = lane; kb < kb_end; kb += 64)
+        part += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1));
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+      const float total = round_to<CT>(part);
+      uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qb) * nkb;
+      for (int kb = lane; kb < nkb; kb += 64) {
+        const float cv = kb < kb_end ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                            crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1))
+                                     : 0.f;
+        out[kb] = (uint16_t)(pack2<CT>(kb < kb_end ? cv / total : 0.f, 0.f) & 0xffffu);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------------
 // Max-pool map, persistent form (bf16/f16, head dim 128, block size KB in {16, 32, 64,
 // 128}): the structure of block_mass_persistent_kernel (items of 128 query rows, K tiles of
@@ -807,93 +892,24 @@ __global__ __launch_bounds__(256, 4) void max_pool_persistent_kernel(PoolArgs a,
       }
     }
 
-    // Epilogue.  Rows past the end of the sequence take no part (m = +inf gives 0).
+    // Rows past the end of the sequence take no part (m = +inf gives 0).
     if (hl == 0) row_m[r] = (qrow < a.Nq) ? m : pos_inf();
     __syncthreads();
-    const float m0 = row_m[lane], m1 = row_m[lane + 64];
-    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(ws, (uint32_t)nkb * 512u);
-    if constexpr (KB == 128) {
-      for (int kb = wave; kb < kb_item; kb += 4) {
-        // coherent (L1-bypassing) loads of values other waves of the group wrote
-        const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
-        const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
-        float v = fmaxf(fast_exp2(x0 - m0), fast_exp2(x1 - m1));
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-        if (lane == 0) colmax[kb] = round_to<CT>(v);
-      }
-      __syncthreads();
-      // Row normalisation in q.dtype: sum (fp32 accumulate, rounded), then divide.
-      if (wave == 0) {
-        float part = 0.f;
-        for (int kb = lane; kb < kb_item; kb += 64) part += colmax[kb];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
-        if (lane == 0) total_sh[0] = round_to<CT>(part);
-      }
-      __syncthreads();
-      const float total = total_sh[0];
-      uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qi) * nkb;
-      for (int kb = tid; kb < nkb; kb += 256) {
-        const float v = kb < kb_item ? colmax[kb] / total : 0.f;
-        out[kb] = (uint16_t)(pack2<CT>(v, 0.f) & 0xffffu);
-      }
-    } else {
-      // Pass 1: column maxima of every (q-block, key block) of the item into cm[qs][kb]:
-      // lane l holds rows l and l + 64, so a q-block is a group of KB lanes (KB < 64) or a
-      // whole half (KB = 64).
-      constexpr int G = KB >= 64 ? 64 : KB;
-      for (int kb = wave; kb < kb_item; kb += 4) {
-        const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
-        const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
-        float v0 = fast_exp2(x0 - m0), v1 = fast_exp2(x1 - m1);
-#pragma unroll
-        for (int off = G / 2; off >= 1; off >>= 1) {
-          v0 = fmaxf(v0, __shfl_xor(v0, off, 64));
-          v1 = fmaxf(v1, __shfl_xor(v1, off, 64));
-        }
-        if (lane % G == 0) {
-          const int g = lane / G;
-          cm[(size_t)g * nkb + kb] = round_to<CT>(v0);
-          cm[(size_t)(NS / 2 + g) * nkb + kb] = round_to<CT>(v1);
-        }
-      }
-      __syncthreads();  // the column maxima are in memory (the barrier drains this group's stores)
-      // Pass 2: per q-block (one wave each), the row total in q.dtype, then the division.
-      const __amdgpu_buffer_rsrc_t crs = make_rsrc(cm, (uint32_t)(NS * nkb) * 4u);
-      for (int qs = wave; qs < NS; qs += 4) {
-        const int qb = qi * NS + qs;
-        if (qb >= a.nqb) continue;
-        const int kb_end = a.causal ? min(nkb, qb + 1) : nkb;
-        float part = 0.f;
-        for (int kb = lane; kb < kb_end; kb += 64)
-          part += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1));
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
-        const float total = round_to<CT>(part);
-        uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qb) * nkb;
-        for (int kb = lane; kb < nkb; kb += 64) {
-          const float cv = kb < kb_end ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                              crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1))
-                                       : 0.f;
-          out[kb] = (uint16_t)(pack2<CT>(kb < kb_end ? cv / total : 0.f, 0.f) & 0xffffu);
-        }
-      }
-    }
+    max_pool_rows<CT, KB>(a, item, ws, cm, row_m, colmax, total_sh);
   }
 }
 
-// The parts of that kernel for items split over key ranges (called from the persistent loop, they
-// made it 1% slower at the Wan layer).
 // 128-key tiles that any row of item `qi` of a head sees.
-template <int KB>
 __device__ __forceinline__ int max_pool_tiles(const PoolArgs& a, int qi) {
   const int ntiles = (a.Nk + 127) >> 7;
   return a.causal ? min(ntiles, qi + 1) : ntiles;
 }
 
 // The tiles [t0, t1) of one item: each row's rounded block maxima into ws[kb][row], the maximum of
-// the unrounded ones in m.
+// the unrounded ones in m.  The persistent kernel keeps a tile loop of its own: at its 128 VGPRs
+// the spills fall otherwise when the tile is a shared function (2 x 12 heads of 32760 at blocks of
+// 64: 5.9 -> 6.8 ms).  A change to one of the two loops belongs in both; their maps are compared bit
+// for bit in the tests.
 template <int CT, int KB>
 __device__ __forceinline__ void max_pool_walk(const PoolArgs& a, SA_LDS char* lk, int item, int t0, int t1, float* ws,
                                               float& m) {
@@ -991,91 +1007,6 @@ __device__ __forceinline__ void max_pool_walk(const PoolArgs& a, SA_LDS char* lk
   }
 }
 
-// The map rows of one item from its rows' block maxima and row maxima (row_m, complete for the
-// group).
-template <int CT, int KB>
-__device__ __forceinline__ void max_pool_rows(const PoolArgs& a, int item, float* ws, float* cm, const float* row_m,
-                                              float* colmax, float* total_sh) {
-  constexpr int NS = 128 / KB;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nkb = a.nkb;
-  const int nqi = (a.Nq + 127) >> 7;
-  const int bh = item / nqi;
-  const int qi = item - bh * nqi;
-  const int kb_item = a.causal ? min(nkb, (qi + 1) * NS) : nkb;  // key blocks any row of the item sees
-  const float m0 = row_m[lane], m1 = row_m[lane + 64];
-  const __amdgpu_buffer_rsrc_t wrs = make_rsrc(ws, (uint32_t)nkb * 512u);
-  if constexpr (KB == 128) {
-    for (int kb = wave; kb < kb_item; kb += 4) {
-      // coherent (L1-bypassing) loads of values other waves of the group wrote
-      const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
-      const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
-      float v = fmaxf(fast_exp2(x0 - m0), fast_exp2(x1 - m1));
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-      if (lane == 0) colmax[kb] = round_to<CT>(v);
-    }
-    __syncthreads();
-    // Row normalisation in q.dtype: sum (fp32 accumulate, rounded), then divide.
-    if (wave == 0) {
-      float part = 0.f;
-      for (int kb = lane; kb < kb_item; kb += 64) part += colmax[kb];
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
-      if (lane == 0) total_sh[0] = round_to<CT>(part);
-    }
-    __syncthreads();
-    const float total = total_sh[0];
-    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qi) * nkb;
-    for (int kb = tid; kb < nkb; kb += 256) {
-      const float v = kb < kb_item ? colmax[kb] / total : 0.f;
-      out[kb] = (uint16_t)(pack2<CT>(v, 0.f) & 0xffffu);
-    }
-  } else {
-    // Pass 1: column maxima of every (q-block, key block) of the item into cm[qs][kb]:
-    // lane l holds rows l and l + 64, so a q-block is a group of KB lanes (KB < 64) or a
-    // whole half (KB = 64).
-    constexpr int G = KB >= 64 ? 64 : KB;
-    for (int kb = wave; kb < kb_item; kb += 4) {
-      const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
-      const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
-      float v0 = fast_exp2(x0 - m0), v1 = fast_exp2(x1 - m1);
-#pragma unroll
-      for (int off = G / 2; off >= 1; off >>= 1) {
-        v0 = fmaxf(v0, __shfl_xor(v0, off, 64));
-        v1 = fmaxf(v1, __shfl_xor(v1, off, 64));
-      }
-      if (lane % G == 0) {
-        const int g = lane / G;
-        cm[(size_t)g * nkb + kb] = round_to<CT>(v0);
-        cm[(size_t)(NS / 2 + g) * nkb + kb] = round_to<CT>(v1);
-      }
-    }
-    __syncthreads();  // the column maxima are in memory (the barrier drains this group's stores)
-    // Pass 2: per q-block (one wave each), the row total in q.dtype, then the division.
-    const __amdgpu_buffer_rsrc_t crs = make_rsrc(cm, (uint32_t)(NS * nkb) * 4u);
-    for (int qs = wave; qs < NS; qs += 4) {
-      const int qb = qi * NS + qs;
-      if (qb >= a.nqb) continue;
-      const int kb_end = a.causal ? min(nkb, qb + 1) : nkb;
-      float part = 0.f;
-      for (int kb = lane; kb < kb_end; kb += 64)
-        part += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1));
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
-      const float total = round_to<CT>(part);
-      uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qb) * nkb;
-      for (int kb = lane; kb < nkb; kb += 64) {
-        const float cv = kb < kb_end ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                            crs, (uint32_t)((qs * nkb + kb) * 4), 0, 1))
-                                     : 0.f;
-        out[kb] = (uint16_t)(pack2<CT>(kb < kb_end ? cv / total : 0.f, 0.f) & 0xffffu);
-      }
-    }
-  }
-}
-
 // Items of a first, partial round, whose groups would leave the others idle: S groups per item,
 // each a range of its key tiles; group (item i, range s) writes its block maxima to item i's slot
 // and its rows' maxima to ml[i][s][128].  max_pool_join_kernel makes the map rows: maxima do not
@@ -1086,7 +1017,7 @@ __global__ __launch_bounds__(256, 4) void max_pool_ranged_kernel(PoolArgs a, int
   constexpr int NS = 128 / KB;
   __shared__ u32x4 lds_k[2048];
   const int i = (int)blockIdx.x % n, s = (int)blockIdx.x / n;
-  const int tiles = max_pool_tiles<KB>(a, i % ((a.Nq + 127) >> 7));
+  const int tiles = max_pool_tiles(a, i % ((a.Nq + 127) >> 7));
   float m;
   max_pool_walk<CT, KB>(a, (SA_LDS char*)lds_k, i, s * tiles / S, (s + 1) * tiles / S,
                         a.ws + (size_t)i * (size_t)a.nkb * (128 + (KB == 128 ? 0 : NS)), m);
