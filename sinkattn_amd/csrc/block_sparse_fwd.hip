@@ -34,9 +34,9 @@ __device__ __forceinline__ void store_lse(const FwdArgs& a, int64_t row, float x
   else reinterpret_cast<float*>(a.lse)[row] = x;
 }
 
-template <int IT, int CT, int D>
+template <int CT, int D>
 __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
-  constexpr int ES = ElemSize<IT>::value;
+  constexpr int ES = 2;
   constexpr int KC = D / 8;   // 16-byte chunks per staged K row
   constexpr int DS = D / 16;  // k-steps of the QK^T contraction
   constexpr int DT = D / 32;  // 32-row tiles of O^T
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
 
   const int qrow = qb * 128 + wave * 32 + l32;
   u32x4 qf[DS];
-  load_q_operand<IT, CT, D>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
+  load_q_operand<D>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
 
   f32x16 o[DT];
 #pragma unroll
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
     const int kb = list[it];
     const int key0 = kb * 128;
     __syncthreads();
-    stage_k_tile<IT, CT, D, 256>(lds_k, kbase, a.ks[2], key0, a.Nk, tid);
+    stage_k_tile<D, 256>(lds_k, kbase, a.ks[2], key0, a.Nk, tid);
     // Stage V^T: each thread gathers a d-pair of 8 consecutive keys.
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) {
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int key = key0 + kg * 8 + e;
-        w[e] = key < a.Nk ? load2<IT, CT>(vbase + ((int64_t)key * a.vs[2] + 2 * dp) * ES) : 0u;
+        w[e] = key < a.Nk ? *reinterpret_cast<const uint32_t*>(vbase + ((int64_t)key * a.vs[2] + 2 * dp) * ES) : 0u;
       }
       u32x4 ev, od;
 #pragma unroll
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256) void block_sparse_fwd_kernel(FwdArgs a) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int d = dt * 32 + 8 * g + 4 * hl;
-        store4<IT>(obase + (int64_t)d * ES, o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv,
+        store4<CT>(obase + (int64_t)d * ES, o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv,
                    o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv);
       }
     if (a.lse != nullptr && hl == 0)
@@ -1734,7 +1734,7 @@ static bool buffer_rows(const FwdArgs& a, int D) {
 // 1.1-1.9 up to 200, 1.0-1.15 at 230-280, 0.93-1.0 past 310.
 constexpr int split_rows(int D) { return D == 128 ? 128 : 256; }
 
-template <int IT, int CT>
+template <int CT>
 static hipError_t launch_fwd_dt(const FwdArgs& a, int D, hipStream_t stream) {
   const int grid = fwd_grid(a);
   if (a.B * a.H * a.nqb <= split_rows(D) && buffer_rows(a, D)) {
@@ -1748,9 +1748,9 @@ static hipError_t launch_fwd_dt(const FwdArgs& a, int D, hipStream_t stream) {
     if (D == 64) block_sparse_fwd_small_kernel<CT, 64><<<grid, 256, 0, stream>>>(a);
     else block_sparse_fwd_small_kernel<CT, 32><<<grid, 256, 0, stream>>>(a);
   else if (D == 64)
-    block_sparse_fwd_kernel<IT, CT, 64><<<grid, 256, 0, stream>>>(a);
+    block_sparse_fwd_kernel<CT, 64><<<grid, 256, 0, stream>>>(a);
   else
-    block_sparse_fwd_kernel<IT, CT, 32><<<grid, 256, 0, stream>>>(a);
+    block_sparse_fwd_kernel<CT, 32><<<grid, 256, 0, stream>>>(a);
   return hipGetLastError();
 }
 
@@ -1801,8 +1801,8 @@ hipError_t launch_dense_mass(const FwdArgs& args, int dtype, hipStream_t stream)
 hipError_t launch_block_sparse_fwd(const FwdArgs& a, int dtype, int D, hipStream_t stream) {
   if (a.B * a.H * a.nqb == 0) return hipSuccess;
   switch (dtype) {
-    case kBF16: return launch_fwd_dt<kBF16, kBF16>(a, D, stream);
-    case kF16: return launch_fwd_dt<kF16, kF16>(a, D, stream);
+    case kBF16: return launch_fwd_dt<kBF16>(a, D, stream);
+    case kF16: return launch_fwd_dt<kF16>(a, D, stream);
     default: {
       const int grid = fwd_grid(a);
       if (D == 128)

@@ -115,47 +115,6 @@ __device__ __forceinline__ float sum_col16(float x) {
   return sum_xor32(p[0] + p[1]);
 }
 
-// Load 8 consecutive elements of type IT at p (16-byte aligned for 16-bit types,
-// 32-byte aligned for f32) and return them as 8 packed 16-bit values of type CT.
-template <int IT, int CT>
-__device__ __forceinline__ u32x4 load8(const void* p);
-template <>
-__device__ __forceinline__ u32x4 load8<kBF16, kBF16>(const void* p) {
-  return *reinterpret_cast<const u32x4*>(p);
-}
-template <>
-__device__ __forceinline__ u32x4 load8<kF16, kF16>(const void* p) {
-  return *reinterpret_cast<const u32x4*>(p);
-}
-template <>
-__device__ __forceinline__ u32x4 load8<kF32, kBF16>(const void* p) {
-  const f32x4* f = reinterpret_cast<const f32x4*>(p);
-  f32x4 a = f[0], b = f[1];
-  u32x4 r;
-  r[0] = pack2<kBF16>(a[0], a[1]);
-  r[1] = pack2<kBF16>(a[2], a[3]);
-  r[2] = pack2<kBF16>(b[0], b[1]);
-  r[3] = pack2<kBF16>(b[2], b[3]);
-  return r;
-}
-
-// Load 2 consecutive elements as one packed pair of CT values.
-template <int IT, int CT>
-__device__ __forceinline__ uint32_t load2(const void* p);
-template <>
-__device__ __forceinline__ uint32_t load2<kBF16, kBF16>(const void* p) {
-  return *reinterpret_cast<const uint32_t*>(p);
-}
-template <>
-__device__ __forceinline__ uint32_t load2<kF16, kF16>(const void* p) {
-  return *reinterpret_cast<const uint32_t*>(p);
-}
-template <>
-__device__ __forceinline__ uint32_t load2<kF32, kBF16>(const void* p) {
-  f32x2 a = *reinterpret_cast<const f32x2*>(p);
-  return pack2<kBF16>(a[0], a[1]);
-}
-
 template <int IT>
 struct ElemSize;
 template <>
@@ -189,18 +148,11 @@ __device__ __forceinline__ void store4<kF32>(void* p, float a, float b, float c,
   *reinterpret_cast<f32x4*>(p) = v;
 }
 
-// s_waitcnt with only a vector-memory count (gfx9 encoding: vmcnt[3:0], expcnt[6:4],
-// lgkmcnt[11:8], vmcnt[15:14]); expcnt/lgkmcnt left at "no wait".
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // Work-group barrier after this wave's buffer->LDS copies have landed and its own LDS
 // reads have returned, so a buffer may be refilled by any wave right after it.
 // (__syncthreads would do the same plus a full fence; this keeps it to the counters.)
 __device__ __forceinline__ void drain_then_barrier() {
+  // gfx9 encoding: vmcnt[3:0], expcnt[6:4], lgkmcnt[11:8], vmcnt[15:14]
   __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8));  // vmcnt(0) expcnt(7) lgkmcnt(0)
   __builtin_amdgcn_s_barrier();
 }

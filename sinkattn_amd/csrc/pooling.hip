@@ -87,7 +87,7 @@ __device__ __forceinline__ void mass_tiles(const PoolArgs& a, SA_LDS char* lk, i
   u32x4 qf[DS];
   // rows past the end repeat the last one: their factor is 0, and 0 times what zeros would make of
   // an infinite key is NaN
-  load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], min(qrow, a.Nq - 1), a.Nq, hl);
+  load_q_operand<128>(qf, qbase, a.qs[2], min(qrow, a.Nq - 1), a.Nq, hl);
   m_ref = neg_inf();
   l_tot = 0.f;
 
@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256, 4) void max_pool_persistent_kernel(PoolArgs a,
     const int qrow = qi * 128 + r;
     const int qbr = qrow / KB;  // this row's q-block
     u32x4 qf[DS];
-    load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
+    load_q_operand<128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
     float m = neg_inf();
 
     for (int kt = 0; kt < kt_end; ++kt) {
@@ -938,7 +938,7 @@ __device__ __forceinline__ void max_pool_walk(const PoolArgs& a, SA_LDS char* lk
   const int qrow = qi * 128 + r;
   const int qbr = qrow / KB;  // this row's q-block
   u32x4 qf[DS];
-  load_q_operand<CT, CT, 128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
+  load_q_operand<128>(qf, qbase, a.qs[2], qrow, a.Nq, hl);
   m = neg_inf();
 
   for (int kt = t0; kt < t1; ++kt) {

@@ -28,10 +28,9 @@ __device__ __forceinline__ int tile_key(int hl, int j) {
 
 // Stage K rows [key0, key0+128) into lds_k (NT threads cooperate, thread index tid).
 // Rows at or beyond Nk are zero-filled.
-template <int IT, int CT, int D, int NT>
+template <int D, int NT>
 __device__ __forceinline__ void stage_k_tile(u32x4* lds_k, const char* kbase, int64_t ks2,
                                              int key0, int Nk, int tid) {
-  constexpr int ES = ElemSize<IT>::value;
   constexpr int KC = D / 8;
   constexpr int ITER = 128 * KC / NT;
 #pragma unroll
@@ -40,7 +39,7 @@ __device__ __forceinline__ void stage_k_tile(u32x4* lds_k, const char* kbase, in
     const int row = id / KC, ch = id % KC;
     const int key = key0 + row;
     u32x4 val = u32x4{0, 0, 0, 0};
-    if (key < Nk) val = load8<IT, CT>(kbase + ((int64_t)key * ks2 + ch * 8) * ES);
+    if (key < Nk) val = *reinterpret_cast<const u32x4*>(kbase + ((int64_t)key * ks2 + ch * 8) * 2);
     lds_k[row * KC + (ch ^ k_swz_kc<KC>(row))] = val;
   }
 }
@@ -65,14 +64,13 @@ __device__ __forceinline__ void qk_tile(const u32x4* lds_k, const u32x4* qf, int
 }
 
 // Load the Q^T B-operands of query row qrow (zeros when qrow >= Nq).
-template <int IT, int CT, int D>
+template <int D>
 __device__ __forceinline__ void load_q_operand(u32x4* qf, const char* qbase, int64_t qs2, int qrow,
                                                int Nq, int hl) {
-  constexpr int ES = ElemSize<IT>::value;
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) {
     if (qrow < Nq)
-      qf[s] = load8<IT, CT>(qbase + ((int64_t)qrow * qs2 + s * 16 + hl * 8) * ES);
+      qf[s] = *reinterpret_cast<const u32x4*>(qbase + ((int64_t)qrow * qs2 + s * 16 + hl * 8) * 2);
     else
       qf[s] = u32x4{0, 0, 0, 0};
   }

@@ -377,7 +377,7 @@ def block_sparse_attention_comp(
     """Block-sparse attention fused with the compensation branch: query rows below
     `comp_rows` (default all; must be a multiple of 128 or Nq) also attend every key of
     kd/vd with weight `gap` each, which equals the reference's LSE mix of the two
-    branches.  kd/vd must share k's/v's row strides (see mean_pool_tokens(like=...))."""
+    branches.  kd/vd must share k's/v's row strides (as mean_pool_kv gives them)."""
     _require_cuda("block_sparse_attention_comp", q, k, v, kd, vd)
     B, H, Nq, D = (int(x) for x in q.shape)
     Nk, Nd = int(k.shape[2]), int(kd.shape[2])

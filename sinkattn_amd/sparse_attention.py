@@ -679,7 +679,7 @@ def _block_sparse_attn_with_compensation(q: torch.Tensor, k: torch.Tensor, v: to
     listed keys plus every pooled key counted `sample_gap` times, which this computes in
     one online softmax (fp32 LSEs; the reference rounds both LSEs to q.dtype first).
     Rows at or beyond `compensated_rows` (a multiple of 128) get the sparse part only.
-    k_dynamic/v_dynamic must share k's/v's row strides (ops.mean_pool_tokens(like=k)).
+    k_dynamic/v_dynamic must share k's/v's row strides (as ops.mean_pool_kv gives them).
     """
     _ensure_block_sparse_available()
     plan = ops.PLAN_CACHE.get(block_mask if block_mask.is_cuda else block_mask.to(q.device))
