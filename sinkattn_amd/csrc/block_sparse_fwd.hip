@@ -1102,6 +1102,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_f32_kernel(FwdArgs a)
         for (int dt = 0; dt < DT; ++dt) o[dt][qt] *= alpha;
         m_run[qt] = m_tile;
       }
+      float ps = 0.f;  // the step's own sum: short chains of additions, as many as steps in the row's
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
@@ -1110,12 +1111,13 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_f32_kernel(FwdArgs a)
           for (int e = 0; e < 2; ++e) {
             const float v0 = fast_exp2(__builtin_fmaf(s[2 * kc + u][qt][2 * e], c, -m_run[qt]));
             const float v1 = fast_exp2(__builtin_fmaf(s[2 * kc + u][qt][2 * e + 1], c, -m_run[qt]));
-            l_run[qt] += v0 + v1;
+            ps += v0 + v1;
             uint32_t hv, lv;
             split_pair(v0, v1, hv, lv);
             ph[kc][qt][2 * u + e] = hv;
             pl[kc][qt][2 * u + e] = lv;
           }
+      l_run[qt] += ps;
     }
     x.template write<1, true>(vh, vl, tid);
     __syncthreads();  // V has landed, every wave is done with K
