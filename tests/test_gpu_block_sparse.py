@@ -404,6 +404,27 @@ def test_first_tile_of_minus_infinity(dtype, D):
     assert ((mass.cpu() - ref)[:, 0].abs() <= 1e-8 + 1e-5 * ref[:, 0].abs()).all()
 
 
+@pytest.mark.parametrize("form,dtype,D,bar", [("sparse", torch.float16, 64, 5.2e-7), ("sparse", torch.bfloat16, 32, 5.2e-7),
+                                              ("dense", torch.float16, 128, 5.2e-7), ("sparse", torch.float32, 128, 6.4e-7)])
+def test_row_sums_of_long_rows(form, dtype, D, bar):
+    """fp32 row sums of 32760 keys are taken in short chains (a tile's, then the tiles'): the spread of
+    the fp32 lse around the 64-bit one.  Its own rounding is 2.8e-7 rms (values of 8 to 16 have an
+    ulp of 9.5e-7), 256 additions of tile sums in each of four lanes 1.6e-7, the scores' and
+    exponentials' roundings bring it to 4.4e-7 (fp32 operands, split in bf16 pairs, 5.9e-7); one chain
+    over the row gave 6.2e-7 (7.0e-7)."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    H, N = 12, 32760
+    q, k, v = (torch.randn(1, H, N, D, device="cuda", generator=g).to(dtype) for _ in range(3))
+    if form == "dense":
+        lse = ops.dense_attention(q, k, v, return_lse=True)[1]
+    else:
+        lse = ops.block_sparse_attention(q, k, v, ops.block_sparse_plan(torch.ones(1, H, 256, 256, dtype=torch.bool, device="cuda")))[1]
+    d = torch.cat([lse[0, h, :1024].double()
+                   - torch.logsumexp(q[0, h, :1024].double() @ k[0, h].double().t().contiguous() / D ** 0.5, -1) for h in range(4)])
+    print(f"{form} {dtype} {D}: mean {d.mean():.2e} spread {d.std():.2e}", flush=True)
+    assert abs(float(d.mean())) <= 1e-6 and float(d.std()) <= bar
+
+
 def _whole_q_blocks(q, k, v, mask):
     """The heads repeated over a batch of more than 256 q-blocks, past which every 16-bit call takes the
     whole-q-block kernels: the outputs of its last entry."""
