@@ -165,14 +165,9 @@ class _PlanCache:
 PLAN_CACHE = _PlanCache()
 
 
-def _output(out: Optional[torch.Tensor], q: torch.Tensor) -> torch.Tensor:
-    """The caller's output tensor, checked, or a new one as a [B, H, N, D] view of [B, N, H, D] memory."""
-    if out is None:
-        B, H, N, D = q.shape
-        return torch.empty((B, N, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+def _check_output(out: torch.Tensor, q: torch.Tensor) -> None:
     if out.shape != q.shape or out.dtype != q.dtype or out.device != q.device:
         raise ValueError(f"out must be {tuple(q.shape)} {q.dtype} on {q.device}, got {tuple(out.shape)} {out.dtype}")
-    return out
 
 
 def block_sparse_attention(
@@ -207,13 +202,17 @@ def block_sparse_attention(
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
     qk, kk, vk = _kernel_operand(q), _kernel_operand(k), _kernel_operand(v)
-    out = _output(out, q)
-    lse16 = lse_in_dtype and q.dtype != torch.float32
-    lse = None
-    if return_lse:
-        lse = torch.empty((B, H, Nq), dtype=q.dtype if lse16 else torch.float32, device=q.device)
+    if out is None:
+        out = torch.empty((B, Nq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    else:
+        _check_output(out, q)
     L = _lib.lib()
-    fwd = L.sinkattn_block_sparse_fwd_lse16 if lse16 else L.sinkattn_block_sparse_fwd
+    lse, fwd = None, L.sinkattn_block_sparse_fwd
+    if return_lse:
+        lse_dtype = q.dtype if lse_in_dtype else torch.float32
+        lse = torch.empty((B, H, Nq), dtype=lse_dtype, device=q.device)
+        if lse_dtype != torch.float32:
+            fwd = L.sinkattn_block_sparse_fwd_lse16
     with torch.cuda.device(q.device):
         _lib.check(
             fwd(
@@ -399,7 +398,10 @@ def block_sparse_attention_comp(
     kdk, vdk = _kernel_operand(kd), _kernel_operand(vd)
     if kdk.stride(2) != kk.stride(2) or vdk.stride(2) != vk.stride(2):
         raise ValueError("kd/vd row strides must equal k/v row strides")
-    out = _output(out, q)
+    if out is None:
+        out = torch.empty((B, Nq, H, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
+    else:
+        _check_output(out, q)
     lse = torch.empty((B, H, Nq), dtype=torch.float32, device=q.device) if return_lse else None
     L = _lib.lib()
     with torch.cuda.device(q.device):
