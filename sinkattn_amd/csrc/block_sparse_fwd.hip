@@ -1735,7 +1735,9 @@ static bool buffer_rows(const FwdArgs& a, int D) {
 // q-blocks up to which a 16-bit call runs the split kernel: as many as give one round of its
 // groups (two per CU at D = 128, four below).  Against the whole q-block per group, bf16: 1.15-1.8
 // times as fast up to 128 q-blocks at D = 128 (0.85-1.1 at 140-190, 0.75-0.9 past 230); f16 D = 64
-// 1.1-1.9 up to 200, 1.0-1.15 at 230-280, 0.93-1.0 past 310.
+// 1.1-1.9 up to 200, 1.0-1.15 at 230-280, 0.93-1.0 past 310.  The lists' length does not move the
+// line: 125 q-blocks of one head of 16000 with 14, 51 and all 125 tiles each 52 -> 35, 132 -> 79, 244 ->
+// 173 us (two heads of 8000, all 63 tiles: 126 -> 90).
 constexpr int split_rows(int D) { return D == 128 ? 128 : 256; }
 
 template <int CT>
