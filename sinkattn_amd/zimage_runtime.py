@@ -493,8 +493,10 @@ class ZImageStaticSinkProcessor:
         return m
 
     def _dense_mask(self, mask: torch.Tensor) -> torch.Tensor:
-        """The all-true mask a forced-dense call reports, one per runtime mask."""
-        key = (mask.device, tuple(mask.shape))
+        """The all-true mask a forced-dense call reports, one per runtime mask and stream (another stream's
+        may not be filled yet)."""
+        key = (mask.device, tuple(mask.shape),
+               torch.cuda.current_stream(mask.device).cuda_stream if mask.is_cuda else 0)
         m = self._dense_mask_cache.get(key)
         if m is None:
             m = self._dense_mask_cache[key] = torch.ones_like(mask, dtype=torch.bool)

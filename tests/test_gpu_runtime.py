@@ -331,3 +331,16 @@ def test_zimage_sample_past_the_kernels_row_reach():
     r = slice((nb - 1) * 128, N)
     want = torch.softmax((q[:, :, r].float() @ k[:, :, r].float().transpose(2, 3).contiguous()) / D ** 0.5, -1) @ v[:, :, r].float()
     _check(out[:, :, r], want.cpu(), 2e-2, 1e-3, "last block of a long sample")
+
+
+def test_zimage_dense_mask_belongs_to_its_stream():
+    """The all-true mask of forced-dense calls is kept per stream: a call on another stream does not read
+    one whose fill it does not wait for."""
+    proc = zr.ZImageStaticSinkProcessor(layer_idx=0, total_layers=1, sink_mask=torch.ones(1, 64, 64, dtype=torch.bool),
+                                        config=zr.build_zimg_sink_config())
+    mask = torch.zeros(1, 1, 4, 4, dtype=torch.bool, device=DEV)
+    first = proc._dense_mask(mask)
+    assert proc._dense_mask(mask) is first and bool(first.all())
+    with torch.cuda.stream(torch.cuda.Stream()):
+        other = proc._dense_mask(mask)
+        assert other is not first and proc._dense_mask(mask) is other and bool(other.all())
