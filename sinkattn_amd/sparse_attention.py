@@ -23,7 +23,7 @@ import os
 import weakref
 from dataclasses import asdict, dataclass
 from pathlib import Path
-from typing import Callable, Dict, Iterable, List, Optional, Sequence, Tuple
+from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -527,12 +527,10 @@ class SinkMaskCalibrator:
     def record(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
         """Block scores of one call on the GPU kernels; their batch mean is added to the
         layer's device-resident sums (no host copy, no sync)."""
-        self._record_scores(layer_idx, lambda: _compute_block_scores(q, k, v, self.config).detach().float())
-
-    def _record_scores(self, layer_idx: int, scores: Callable[[], torch.Tensor]) -> None:
         if layer_idx == 0:
             self.current_step += 1
-        self._accumulate_score(layer_idx, scores().mean(dim=0))
+        samples = _compute_block_scores(q, k, v, self.config).detach().float()
+        self._accumulate_score(layer_idx, samples.mean(dim=0))
 
     def build_package(self, include_scores: bool = True,
                       config_override: Optional[SinkSparseConfig] = None) -> dict:
@@ -825,7 +823,9 @@ def _record_and_attend(calibrator: SinkMaskCalibrator, layer_idx: int, q: torch.
             out = None
         if out is not None:
             with torch.no_grad():
-                calibrator._record_scores(layer_idx, lambda: mass)
+                if layer_idx == 0:
+                    calibrator.current_step += 1
+                calibrator._accumulate_score(layer_idx, mass.mean(dim=0))
             return out
     calibrator.record(layer_idx, q, k, v)
     return _dense_attention(q, k, v)
