@@ -1240,7 +1240,11 @@ int max_pool_groups() { return 4 * device_cu_count(); }
 constexpr int kMassMinTiles = 4;
 // Key tiles from which a call is split.  Below, the second launch costs a program that records
 // call after call as much as the ranges save: max-pool at [1,9,1847,128] 28 -> 22 us on the GPU,
-// but 37.5 -> 41 us per recorded call.
+// but 37.5 -> 41 us per recorded call.  At the line itself a call that the program waits for, or
+// that follows other GPU work, gains all of it (one recorded call, block mass [1,2,2048,128] 64 -> 53
+// us, max-pool [1,2,3072,128] 67 -> 58), while calls of one to four heads back to back, which are
+// bound by the host, pay 3-4 us for the launch (39.8 -> 44.2 and 45.9 -> 49.1) up to 2400 and 4300
+// keys; past these both gain ([1,2,3500,128] block mass 57 -> 44, [1,2,6000,128] max-pool 70 -> 49).
 constexpr int kMassSplitTiles = 16, kMaxSplitTiles = 24;
 
 struct MassSplit {
