@@ -1,7 +1,7 @@
 """GPU parity of the block-sparse attention forward (sinkattn_block_sparse_fwd) against
 the fp32 dense masked-softmax oracle (oracle/torch_ref.dense_masked_attention).
 
-Tolerance (north star): max |out - ref| <= 2e-2 and mean |out - ref| <= 1e-3.  The fp32 lse
+Tolerance: max |out - ref| <= 2e-2 and mean |out - ref| <= 1e-3.  The fp32 lse
 the kernels write is held to 4e-3 + 1e-5 |ref|: the head-dim-128 kernel sums the 16-bit P
 values it multiplies V with (on the matrix cores), each within 2^-8 relative of the fp32
 value for bf16, so its row sum is within 2^-8 relative and its lse within log(1 + 2^-8) =
@@ -140,7 +140,7 @@ def test_running_maximum_moves_across_tiles(dtype, step):
 
 
 def test_config1_shape_fp32_with_sinks():
-    # BASELINE config 1: B=1, H=12, N=4096, d=128, fp32, 4 sink keys scaled 8x.
+    # B=1, H=12, N=4096, d=128, fp32, 4 sink keys scaled 8x.
     q, k, v = _inputs(1, 12, 4096, 4096, 128, torch.float32, seed=0, sink_keys=4)
     mask = _random_mask(1, 12, 32, 32, 0.25, seed=3)
     out, lse = sa._block_sparse_attn(q, k, v, mask, return_lse=True)
@@ -151,7 +151,7 @@ def test_config1_shape_fp32_with_sinks():
 
 
 def test_config1_chain_mass_mask_attention():
-    """BASELINE config 1 as one chain: exact block mass -> coverage-0.85 mask -> sparse
+    """[1,12,4096,128] fp32 as one chain: exact block mass -> coverage-0.85 mask -> sparse
     attention on that mask (sparse_attention.py:145-227, 268-376, 710-776).
 
     fp32 [1,12,4096,128], keys 0..3 x8.  Mass within 1e-5 relative of the oracle; the mask

@@ -62,7 +62,7 @@ def test_exact_mass_small(dtype, N):
 
 
 def test_exact_mass_config1_fp32():
-    # BASELINE config 1: [1,12,4096,128] fp32 with 4 sink keys scaled 8x -> [1,12,32,32]
+    # [1,12,4096,128] fp32 with 4 sink keys scaled 8x -> [1,12,32,32]
     q, k = _qk(1, 12, 4096, 4096, torch.float32, seed=0, sinks=4)
     cfg = sa.SinkSparseConfig(pooling_mode="exact")
     ours = sa._compute_block_scores(q.cuda(), k.cuda(), k.cuda(), cfg)
