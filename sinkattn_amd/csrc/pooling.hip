@@ -895,7 +895,37 @@ __global__ __launch_bounds__(256, 4) void max_pool_persistent_kernel(PoolArgs a,
     // Rows past the end of the sequence take no part (m = +inf gives 0).
     if (hl == 0) row_m[r] = (qrow < a.Nq) ? m : pos_inf();
     __syncthreads();
-    max_pool_rows<CT, KB>(a, item, ws, cm, row_m, colmax, total_sh);
+    if constexpr (KB != 128) {
+      max_pool_rows<CT, KB>(a, item, ws, cm, row_m, colmax, total_sh);
+    } else {  // max_pool_rows' part for blocks of 128, here: as a call 0.3% slower at the Wan layer
+      const float m0 = row_m[lane], m1 = row_m[lane + 64];
+      const __amdgpu_buffer_rsrc_t wrs = make_rsrc(ws, (uint32_t)nkb * 512u);
+      for (int kb = wave; kb < kb_item; kb += 4) {
+        // coherent (L1-bypassing) loads of values other waves of the group wrote
+        const float x0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4), 0, 1));
+        const float x1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (uint32_t)(kb * 512 + lane * 4 + 256), 0, 1));
+        float v = fmaxf(fast_exp2(x0 - m0), fast_exp2(x1 - m1));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+        if (lane == 0) colmax[kb] = round_to<CT>(v);
+      }
+      __syncthreads();
+      // Row normalisation in q.dtype: sum (fp32 accumulate, rounded), then divide.
+      if (wave == 0) {
+        float part = 0.f;
+        for (int kb = lane; kb < kb_item; kb += 64) part += colmax[kb];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+        if (lane == 0) total_sh[0] = round_to<CT>(part);
+      }
+      __syncthreads();
+      const float total = total_sh[0];
+      uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * a.nqb + qi) * nkb;
+      for (int kb = tid; kb < nkb; kb += 256) {
+        const float v = kb < kb_item ? colmax[kb] / total : 0.f;
+        out[kb] = (uint16_t)(pack2<CT>(v, 0.f) & 0xffffu);
+      }
+    }
   }
 }
 
